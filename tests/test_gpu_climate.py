@@ -121,3 +121,55 @@ def test_surface_temp_matches_oracle(oracle, tilt):
         climate.assign_surface_temp(pts, np.full(pts.shape[0], 3.0), 1.0, tilt)
     dev = climate.assign_surface_temp_device(torch.from_numpy(pts).cuda(), 1.0, tilt)
     assert np.array_equal(dev.cpu().numpy(), got)
+
+
+def _sun_vertices(kind):
+    pts, _ = util.create_mesh(17)
+    rng = np.random.default_rng(5)
+    if kind == "sphere":
+        return pts, 1.0
+    if kind == "world":
+        return pts * 6378100.0, 6378100.0
+    if kind == "relief":                      # off the sphere, on both sides of it
+        return pts * (1 + 1e-3 * rng.uniform(-1, 1, (pts.shape[0], 1))), 1.0
+    if kind == "inside":                      # latitudes clamped for |z| > r
+        return pts * 0.5, 0.25
+    if kind == "rounding":                    # around the rule's edge, |v|^2 - r^2 = 2^-50 .. 2^-44
+        return pts * (1 + 2.0 ** rng.uniform(-51, -45, (pts.shape[0], 1))), 1.0
+    special = np.array([[0, 0, 1], [0, 0, -1], [0, 0, 0], [1, 0, 0], [-1, 0, 0], [0, -1, 0],
+                        [-0.0, -0.0, 1], [1e-200, 0, 1], [1e-170, 1e-170, 1], [1e170, 1, 1],
+                        [np.inf, 0, 0], [0, 0, np.inf], [np.nan, 0, 0], [0, 0, np.nan]])
+    return special, 1.0
+
+
+@pytest.mark.parametrize("nsteps", [1, 3, 360])
+@pytest.mark.parametrize("kind", ["sphere", "world", "relief", "inside", "rounding", "special"])
+def test_insolation_on_and_off_the_sphere(oracle, kind, nsteps):
+    """The vector forms of the rotation step against the oracle's angles: one
+    float32 ulp per summed step, NaN where the oracle has NaN."""
+    verts, r = _sun_vertices(kind)
+    for tilt in (0.0, 23.44, 90.0):
+        dev = torch.from_numpy(verts).cuda()
+        arr = torch.zeros(verts.shape[0], dtype=torch.float32, device="cuda")
+        climate.sample_insolation_device(arr, dev, r, -180.0, tilt, nsteps, 360.0 / nsteps)
+        got = arr.cpu().numpy()
+        ref = oracle.sample_insolation(np.zeros(verts.shape[0], np.float32), verts, r, -180.0,
+                                       tilt, nsteps, 360.0 / nsteps)
+        fine = np.isfinite(ref)
+        assert np.array_equal(np.isnan(got), np.isnan(ref))
+        top = max(float(np.abs(ref[fine]).max()), 1.0)
+        assert np.abs(got[fine] - ref[fine]).max() <= nsteps * float(np.spacing(np.float32(top)))
+
+
+@pytest.mark.parametrize("radius", [1.0, 6378100.0])
+def test_year_of_each_latitude_band(oracle, radius):
+    """A year at whole and fractional latitudes, the poles among them: each
+    day's table entry within 360 float32 ulp, then one rounding of the year
+    against 360 of the sequential sum."""
+    lats = np.concatenate([np.arange(-90, 91), np.linspace(-89.999, 89.999, 400)]) * np.pi / 180
+    verts = radius * np.stack([np.cos(lats), np.zeros_like(lats), np.sin(lats)], axis=1)
+    got = climate.calc_yearly_insolation(verts, None, radius, 23.44)
+    ref = oracle.yearly_insolation(verts, radius, 23.44)
+    day_ulp = float(np.spacing(np.float32(ref.max() / 360)))
+    tol = 360 * 361 * day_ulp + 360 * float(np.spacing(np.float32(ref.max())))
+    assert got.dtype == np.float32 and np.abs(got.astype(np.float64) - ref).max() <= tol
