@@ -3,18 +3,23 @@
 // vertices of each pixel (the reference's scipy KD-tree query) and the
 // inverse-distance sampling of make_gray_array.
 //
-// Nearest neighbours come from a uniform grid instead of a tree: points are
-// sorted by the key of their cell, every occupied cell goes into an
-// open-addressing hash table (key -> first point, count), and a query visits
-// shells of cells around its own until the k-th best distance is no larger
-// than the distance from the query to the faces of the block searched, so
-// the result is the exact k nearest (ties ordered by point index).
+// Nearest neighbours come from a bin structure instead of a tree: points are
+// counted into bins and stored bin by bin, and a query scans the bins around
+// it, in growing blocks, until the k-th best distance is no larger than the
+// least distance that a point outside the block can have, so the result is
+// the exact k nearest (ties ordered by point index, whatever the order inside
+// a bin).  Two kinds of bins, chosen on the device when the grid is built:
+//   shell  points that surround the origin at nearly one radius (a planet's
+//          vertices): bands of equal latitude height, each cut into cells of
+//          about the same width in longitude.  A band's cells are consecutive
+//          in memory, so a block of 3 x 3 cells is three runs of points with
+//          no search; the band table has about 0.74 sqrt(V) entries.
+//   cells  any other points: cubes of a uniform grid, hashed into at least
+//          2V bins.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
 #include <vector>
-
-#include <hipcub/hipcub.hpp>
 
 #include "nx_ctx.h"
 #include "nx_reduce_dev.h"
@@ -24,21 +29,35 @@ namespace nx {
 namespace {
 
 constexpr int kKnnMax = 8;                // largest k
-constexpr unsigned long long kEmpty = ~0ull;
 constexpr int kAxisBits = 21;             // cell coordinate bits per axis
+// Height of a band, in mean spacings sqrt(4 pi / V) of V points on the unit
+// sphere.  The third nearest vertex of an icosphere lies within 1.18 of
+// them, so a block reaching one band and cell beyond the query's own settles
+// the reference's k = 3 in one round, over about 13 points.
+constexpr double kBandSpacings = 1.2;
+// Slack of the FP32 latitudes and longitudes, in radians (their rounding is
+// below 1e-6), and of the FP64 comparison of squared distances.
+constexpr float kAngleSlack = 2e-6f;
+constexpr double kGuardSlack = 1e-6;
+constexpr int kBoxBlocks = 256;           // one per CU
+constexpr int kScanBlocks = 1024;
 
 struct GridHead {
     double origin[3];
     double cell;
     int32_t dims[3];
-    int32_t pad;
-    unsigned long long box[6];  // min/max keys per axis
+    int32_t shell;              // 1: latitude bands, 0: hashed cells
+    int64_t nbins;
+    double rmin, rmax;          // shell: least and largest |p|
+    double cosa[2], sin2a[2];   // shell: cos a and sin^2 (a / 2) of blocks of 1 and 2 bands
 };
 static_assert(sizeof(GridHead) <= 256, "grid head must fit its 256 bytes");
 
-struct CellEntry {
-    unsigned long long key;
-    int32_t start, count;
+// A point in bin order; `tag` is the upper half of its cell's hash (cells).
+struct alignas(16) GridPoint {
+    double x, y, z;
+    int32_t idx;
+    uint32_t tag;
 };
 
 inline size_t a256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -50,41 +69,38 @@ uint64_t table_size(int64_t V)
     return t;
 }
 
-size_t sort_temp_bytes(int64_t V)
+int32_t band_count(int64_t V)
 {
-    size_t bytes = 0;
-    (void)hipcub::DeviceRadixSort::SortPairs(nullptr, bytes, (const uint64_t *)nullptr,
-                                             (uint64_t *)nullptr, (const int32_t *)nullptr,
-                                             (int32_t *)nullptr, (int)V, 0, 3 * kAxisBits);
-    return bytes;
+    const double h = kBandSpacings * std::sqrt(4.0 * 3.141592653589793 / (double)V);
+    return (int32_t)std::max(1.0, std::floor(3.141592653589793 / h));
 }
 
 struct GridLayout {
-    size_t head, spts, sidx, kin, kout, iin, temp, table, total;
-    uint64_t tsize;
+    size_t head, band, start, pts, bin, rank, part, total;
+    uint64_t tsize;    // bins for hashed cells
+    int32_t bands;
 };
 
 GridLayout grid_layout(int64_t V)
 {
     GridLayout L;
+    L.bands = band_count(V);
+    L.tsize = table_size(V);
     size_t o = 0;
     L.head = o;
     o += 256;
-    L.spts = o;
-    o += a256(24 * (size_t)V);
-    L.sidx = o;
+    L.band = o;
+    o += a256(4 * ((size_t)L.bands + 1));
+    L.start = o;
+    o += a256(4 * ((size_t)L.tsize + 1));
+    L.pts = o;
+    o += a256(sizeof(GridPoint) * (size_t)V);
+    L.bin = o;
     o += a256(4 * (size_t)V);
-    L.kin = o;
-    o += a256(8 * (size_t)V);
-    L.kout = o;
-    o += a256(8 * (size_t)V);
-    L.iin = o;
+    L.rank = o;
     o += a256(4 * (size_t)V);
-    L.temp = o;
-    o += a256(sort_temp_bytes(V));
-    L.tsize = table_size(V);
-    L.table = o;
-    o += a256(sizeof(CellEntry) * (size_t)L.tsize);
+    L.part = o;
+    o += a256(8 * 8 * kBoxBlocks);
     L.total = o;
     return L;
 }
@@ -113,268 +129,495 @@ __device__ __forceinline__ int cell_of(double q, double o, double cell, int dim)
     return t >= (double)(dim - 1) ? dim - 1 : (int)t;
 }
 
-}  // namespace
-
-__global__ void k_grid_init(GridHead *g)
+// Latitude + pi / 2, longitude + pi and the cosine of the latitude of a
+// direction, in FP32 (within kAngleSlack); scale brings it near length 1.
+__device__ __forceinline__ void angles_of(double x, double y, double z, double scale, float &lat,
+                                          float &lon, float &clat)
 {
-    if (threadIdx.x < 3) {
-        g->box[2 * threadIdx.x] = ~0ull;
-        g->box[2 * threadIdx.x + 1] = 0ull;
-    }
+    const float fx = (float)(x * scale), fy = (float)(y * scale), fz = (float)(z * scale);
+    const float rho = sqrtf(fx * fx + fy * fy);
+    lat = atan2f(fz, rho) + 1.57079633f;
+    lon = atan2f(fy, fx) + 3.14159265f;
+    clat = rho / sqrtf(rho * rho + fz * fz);
 }
 
-__global__ __launch_bounds__(256) void k_grid_box(const double *__restrict__ pts, int64_t V,
-                                                  GridHead *__restrict__ g)
+__device__ __forceinline__ int clamp_cell(float t, int n) { return min(max((int)t, 0), n - 1); }
+
+__device__ __forceinline__ int band_of(float lat, int bands)
 {
-    for (int k = 0; k < 3; ++k) {
-        unsigned long long lo = ~0ull, hi = 0ull;
-        for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < V;
-             i += (int64_t)gridDim.x * blockDim.x) {
-            const unsigned long long q = dkey(pts[3 * i + k]);
-            lo = q < lo ? q : lo;
-            hi = q > hi ? q : hi;
+    return clamp_cell(lat * ((float)bands * 0.318309886f), bands);
+}
+
+}  // namespace
+
+// Box of the points and least / largest squared norm, one record of eight
+// order-preserving keys per block.
+__global__ __launch_bounds__(1024) void k_grid_box(const double *__restrict__ pts, int64_t V,
+                                                   unsigned long long *__restrict__ part)
+{
+    unsigned long long lo[4], hi[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        lo[k] = ~0ull;
+        hi[k] = 0ull;
+    }
+    const int64_t step = (int64_t)gridDim.x * blockDim.x;
+#pragma unroll 2
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < V; i += step) {
+        const double p[3] = {pts[3 * i], pts[3 * i + 1], pts[3 * i + 2]};
+        const unsigned long long q[4] = {dkey(p[0]), dkey(p[1]), dkey(p[2]),
+                                         dkey(p[0] * p[0] + p[1] * p[1] + p[2] * p[2])};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            lo[k] = q[k] < lo[k] ? q[k] : lo[k];
+            hi[k] = q[k] > hi[k] ? q[k] : hi[k];
         }
-        block_minmax(lo, hi);
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        block_minmax(lo[k], hi[k]);
         if (threadIdx.x == 0) {
-            __hip_atomic_fetch_min(&g->box[2 * k], lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_fetch_max(&g->box[2 * k + 1], hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            part[8 * blockIdx.x + 2 * k] = lo[k];
+            part[8 * blockIdx.x + 2 * k + 1] = hi[k];
         }
         __syncthreads();
     }
 }
 
-// Grid geometry: a cell edge of twice the mean spacing of V points spread
-// over the sphere that fits the box (about four to six points per occupied
-// cell for a sphere mesh), at most 2^21 - 1 cells per axis.  The geometry
-// only sets the speed; the search is exact for any cell size.
-__global__ void k_grid_setup(GridHead *g, int64_t V)
+// Grid geometry (one block).  Points with norms in [0.8, 1] of the largest
+// that reach 0.7 of it on both sides of every axis get latitude bands: those
+// are sized for points over the whole sphere, and a band's cells bound the
+// distance of their points by direction alone.  Others get cells with an edge
+// of twice the mean spacing of V points spread over the sphere that fits the
+// box, at most 2^21 - 1 per axis.  The geometry only sets the speed; the
+// search is exact for any.
+__global__ __launch_bounds__(1024) void k_grid_setup(GridHead *__restrict__ g, int64_t V,
+                                                     const unsigned long long *__restrict__ part,
+                                                     int parts, int32_t bands, uint64_t tsize,
+                                                     int32_t *__restrict__ band)
 {
-    if (threadIdx.x != 0) return;
-    double ext[3], lo[3];
-    double R = 0.0;
-    for (int k = 0; k < 3; ++k) {
-        lo[k] = dunkey(g->box[2 * k]);
-        ext[k] = dunkey(g->box[2 * k + 1]) - lo[k];
-        R = fmax(R, 0.5 * ext[k]);
+    __shared__ double box[8];
+    __shared__ int shell;
+    const int t = threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        unsigned long long lo = ~0ull, hi = 0ull;
+        for (int i = t; i < parts; i += 1024) {
+            const unsigned long long a = part[8 * i + 2 * k], b = part[8 * i + 2 * k + 1];
+            lo = a < lo ? a : lo;
+            hi = b > hi ? b : hi;
+        }
+        block_minmax(lo, hi);
+        if (t == 0) {
+            box[2 * k] = dunkey(lo);
+            box[2 * k + 1] = dunkey(hi);
+        }
+        __syncthreads();
     }
-    double cell = 2.0 * sqrt(4.0 * 3.141592653589793 * R * R / (double)V);
-    for (int k = 0; k < 3; ++k) {
-        const double need = ext[k] / 2097150.0;
-        if (cell < need) cell = need;
+    const double pi = 3.141592653589793, h = pi / bands;
+    if (t == 0) {
+        double ext[3], R = 0.0;
+        const double n0 = box[6], n1 = box[7];
+        bool s = n1 >= 0x1p-600 && n1 <= 0x1p600 && n0 >= 0.64 * n1;
+        for (int k = 0; k < 3; ++k) {
+            ext[k] = box[2 * k + 1] - box[2 * k];
+            R = fmax(R, 0.5 * ext[k]);
+            s = s && box[2 * k] <= -0.7 * sqrt(n1) && box[2 * k + 1] >= 0.7 * sqrt(n1);
+        }
+        double cell = 2.0 * sqrt(4.0 * pi * R * R / (double)V);
+        for (int k = 0; k < 3; ++k) {
+            const double need = ext[k] / 2097150.0;
+            if (cell < need) cell = need;
+        }
+        if (!(cell > 0.0)) cell = 1.0;  // all points equal
+        g->cell = cell;
+        for (int k = 0; k < 3; ++k) {
+            g->origin[k] = box[2 * k];
+            const double n = floor(ext[k] / cell) + 1.0;
+            g->dims[k] = (int32_t)fmin(n, 2097151.0);
+        }
+        g->shell = shell = s;
+        g->rmin = sqrt(n0) * (1.0 - kGuardSlack);
+        g->rmax = sqrt(n1) * (1.0 + kGuardSlack);
+        for (int r = 1; r <= 2; ++r) {
+            const double a = r * h - 2.0 * kAngleSlack;
+            g->cosa[r - 1] = cos(a);
+            g->sin2a[r - 1] = sin(0.5 * a) * sin(0.5 * a);
+        }
+        if (!s) g->nbins = (int64_t)tsize;
     }
-    if (!(cell > 0.0)) cell = 1.0;  // all points equal
-    g->cell = cell;
-    for (int k = 0; k < 3; ++k) {
-        g->origin[k] = lo[k];
-        const double n = floor(ext[k] / cell) + 1.0;
-        g->dims[k] = (int32_t)fmin(n, 2097151.0);
+    __syncthreads();
+    if (!shell) return;
+    // cells of each band and their running sum
+    __shared__ int32_t wsum[16];
+    int32_t carry = 0;
+    for (int32_t b0 = 0; b0 < bands; b0 += 1024) {
+        const int32_t b = b0 + t;
+        int32_t n = 0;
+        if (b < bands) n = max(1, (int32_t)(2.0 * bands * cos((b + 0.5) * h - 0.5 * pi)));
+        int32_t inc = n;
+        for (int off = 1; off < 64; off <<= 1) {
+            const int32_t o = __shfl_up(inc, off, 64);
+            if ((t & 63) >= off) inc += o;
+        }
+        if ((t & 63) == 63) wsum[t >> 6] = inc;
+        __syncthreads();
+        int32_t before = carry, all = carry;
+        for (int w = 0; w < 16; ++w) {
+            if (w < (t >> 6)) before += wsum[w];
+            all += wsum[w];
+        }
+        if (b < bands) band[b] = before + inc - n;
+        carry = all;
+        __syncthreads();
+    }
+    if (t == 0) {
+        band[bands] = carry;
+        g->nbins = carry;
     }
 }
 
-__global__ __launch_bounds__(256) void k_grid_keys(const double *__restrict__ pts, int64_t V,
-                                                   const GridHead *__restrict__ g,
-                                                   unsigned long long *__restrict__ key,
-                                                   int32_t *__restrict__ idx)
+__global__ __launch_bounds__(256) void k_grid_clear(const GridHead *__restrict__ g,
+                                                    int32_t *__restrict__ count)
+{
+    const int64_t n = g->nbins;
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+         i += (int64_t)gridDim.x * blockDim.x)
+        count[i] = 0;
+}
+
+// Each point's bin and its rank among the bin's points.
+__global__ __launch_bounds__(256) void k_grid_count(const double *__restrict__ pts, int64_t V,
+                                                    const GridHead *__restrict__ g,
+                                                    const int32_t *__restrict__ band, int32_t bands,
+                                                    int32_t *__restrict__ count,
+                                                    uint32_t *__restrict__ bin,
+                                                    int32_t *__restrict__ rank)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= V) return;
-    const double c = g->cell;
-    const int x = cell_of(pts[3 * i], g->origin[0], c, g->dims[0]);
-    const int y = cell_of(pts[3 * i + 1], g->origin[1], c, g->dims[1]);
-    const int z = cell_of(pts[3 * i + 2], g->origin[2], c, g->dims[2]);
-    key[i] = cell_key(x, y, z);
-    idx[i] = (int32_t)i;
-}
-
-__global__ __launch_bounds__(256) void k_fill_cells(CellEntry *t, uint64_t n)
-{
-    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) {
-        t[i].key = kEmpty;
-        t[i].start = 0;
-        t[i].count = 0;
+    const double x = pts[3 * i], y = pts[3 * i + 1], z = pts[3 * i + 2];
+    uint32_t b;
+    if (g->shell) {
+        float lat, lon, clat;
+        angles_of(x, y, z, 1.0 / g->rmax, lat, lon, clat);
+        const int r = band_of(lat, bands);
+        const int n = band[r + 1] - band[r];
+        b = (uint32_t)(band[r] + clamp_cell(lon * ((float)n * 0.159154943f), n));
+    } else {
+        const double c = g->cell;
+        const uint64_t m = mix64(cell_key(cell_of(x, g->origin[0], c, g->dims[0]),
+                                          cell_of(y, g->origin[1], c, g->dims[1]),
+                                          cell_of(z, g->origin[2], c, g->dims[2])));
+        b = (uint32_t)(m & (uint64_t)(g->nbins - 1));
     }
+    bin[i] = b;
+    rank[i] = __hip_atomic_fetch_add(&count[b], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Sorted coordinates, and one table entry per run of equal keys.  The table
-// holds at least 2V slots, so every insertion finds a free one.
-__global__ __launch_bounds__(256) void k_grid_fill(const double *__restrict__ pts, int64_t V,
-                                                   const unsigned long long *__restrict__ skey,
-                                                   const int32_t *__restrict__ sidx,
-                                                   double *__restrict__ spts,
-                                                   CellEntry *__restrict__ table, uint64_t mask)
+// Points of each of gridDim.x equal runs of bins.
+__global__ __launch_bounds__(256) void k_grid_sums(const GridHead *__restrict__ g,
+                                                   const int32_t *__restrict__ count,
+                                                   int32_t *__restrict__ sums)
 {
-    const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= V) return;
-    const int64_t src = sidx[j];
-    spts[3 * j] = pts[3 * src];
-    spts[3 * j + 1] = pts[3 * src + 1];
-    spts[3 * j + 2] = pts[3 * src + 2];
-    const unsigned long long k = skey[j];
-    if (j > 0 && skey[j - 1] == k) return;
-    int64_t e = j + 1;
-    while (e < V && skey[e] == k) ++e;
-    uint64_t slot = mix64(k) & mask;
-    for (;;) {
-        const unsigned long long prev = atomicCAS(&table[slot].key, kEmpty, k);
-        if (prev == kEmpty) {
-            table[slot].start = (int32_t)j;
-            table[slot].count = (int32_t)(e - j);
-            return;
+    const int64_t n = g->nbins, per = (n + gridDim.x - 1) / gridDim.x;
+    const int64_t a = per * blockIdx.x, e = min(n, a + per);
+    int32_t s = 0;
+    for (int64_t i = a + threadIdx.x; i < e; i += 256) s += count[i];
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    __shared__ int32_t w[4];
+    if ((threadIdx.x & 63) == 0) w[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) sums[blockIdx.x] = w[0] + w[1] + w[2] + w[3];
+}
+
+// Counts to the first point of each bin, in place, over the same runs;
+// start[nbins] = V.
+__global__ __launch_bounds__(256) void k_grid_starts(const GridHead *__restrict__ g, int64_t V,
+                                                     const int32_t *__restrict__ sums,
+                                                     int32_t *__restrict__ start)
+{
+    const int64_t n = g->nbins, per = (n + gridDim.x - 1) / gridDim.x;
+    const int64_t a = per * blockIdx.x, e = min(n, a + per);
+    const int t = threadIdx.x, wave = t >> 6;
+    __shared__ int32_t w[4];
+    int32_t s = 0;
+    for (int i = t; i < (int)blockIdx.x; i += 256) s += sums[i];
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    if ((t & 63) == 0) w[wave] = s;
+    __syncthreads();
+    int32_t carry = w[0] + w[1] + w[2] + w[3];
+    for (int64_t i0 = a; i0 < e; i0 += 256) {
+        const int64_t i = i0 + t;
+        const int32_t c = i < e ? start[i] : 0;
+        int32_t inc = c;
+        for (int off = 1; off < 64; off <<= 1) {
+            const int32_t o = __shfl_up(inc, off, 64);
+            if ((t & 63) >= off) inc += o;
         }
-        slot = (slot + 1) & mask;
+        __syncthreads();
+        if ((t & 63) == 63) w[wave] = inc;
+        __syncthreads();
+        int32_t before = carry;
+        for (int k = 0; k < 4; ++k)
+            if (k < wave) before += w[k];
+        if (i < e) start[i] = before + inc - c;
+        carry += w[0] + w[1] + w[2] + w[3];
     }
+    if (blockIdx.x == 0 && t == 0) start[n] = (int32_t)V;
+}
+
+__global__ __launch_bounds__(256) void k_grid_place(const double *__restrict__ pts, int64_t V,
+                                                    const GridHead *__restrict__ g,
+                                                    const int32_t *__restrict__ start,
+                                                    const uint32_t *__restrict__ bin,
+                                                    const int32_t *__restrict__ rank,
+                                                    GridPoint *__restrict__ out)
+{
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= V) return;
+    GridPoint p;
+    p.x = pts[3 * i];
+    p.y = pts[3 * i + 1];
+    p.z = pts[3 * i + 2];
+    p.idx = (int32_t)i;
+    p.tag = 0;
+    if (!g->shell) {
+        const double c = g->cell;
+        p.tag = (uint32_t)(mix64(cell_key(cell_of(p.x, g->origin[0], c, g->dims[0]),
+                                          cell_of(p.y, g->origin[1], c, g->dims[1]),
+                                          cell_of(p.z, g->origin[2], c, g->dims[2]))) >> 32);
+    }
+    out[(int64_t)start[bin[i]] + rank[i]] = p;
 }
 
 namespace {
 
 struct GridView {
-    double ox, oy, oz, cell;
-    int dx, dy, dz;
-    const double *spts;
-    const int32_t *sidx;
-    const CellEntry *table;
-    uint64_t mask;
+    const GridHead *g;
+    const int32_t *band;
+    const int32_t *start;
+    const GridPoint *pts;
+    int32_t bands;
 };
-
-__device__ __forceinline__ GridView grid_view(const char *ws, const double *spts,
-                                              const int32_t *sidx, const CellEntry *table,
-                                              uint64_t mask)
-{
-    const GridHead *g = (const GridHead *)ws;
-    GridView v;
-    v.ox = g->origin[0];
-    v.oy = g->origin[1];
-    v.oz = g->origin[2];
-    v.cell = g->cell;
-    v.dx = g->dims[0];
-    v.dy = g->dims[1];
-    v.dz = g->dims[2];
-    v.spts = spts;
-    v.sidx = sidx;
-    v.table = table;
-    v.mask = mask;
-    return v;
-}
 
 __device__ __forceinline__ bool before(double s, int32_t i, double t, int32_t j)
 {
     return s < t || (s == t && i < j);
 }
 
-template <int K>
-__device__ __forceinline__ void visit_cell(const GridView &g, int x, int y, int z, double qx,
-                                           double qy, double qz, double (&bd)[K],
-                                           int32_t (&bi)[K])
+// Points j0..j1-1 against the K best.  HASHED skips points of other cells
+// (another tag) and points already held (another visited cell with this tag).
+template <int K, bool HASHED>
+__device__ __forceinline__ void scan_points(const GridPoint *__restrict__ pts, int j0, int j1,
+                                            uint32_t tag, double qx, double qy, double qz,
+                                            double (&bd)[K], int32_t (&bi)[K])
 {
-    const unsigned long long key = cell_key(x, y, z);
-    uint64_t slot = mix64(key) & g.mask;
-    CellEntry e;
-    for (;;) {
-        e = g.table[slot];
-        if (e.key == key) break;
-        if (e.key == kEmpty) return;
-        slot = (slot + 1) & g.mask;
-    }
-    for (int t = e.start; t < e.start + e.count; ++t) {
+    for (int j = j0; j < j1; ++j) {
+        const GridPoint p = pts[j];
+        if (HASHED && p.tag != tag) continue;
         double s = 0.0, d;
-        d = qx - g.spts[3 * t];
+        d = qx - p.x;
         s += d * d;
-        d = qy - g.spts[3 * t + 1];
+        d = qy - p.y;
         s += d * d;
-        d = qz - g.spts[3 * t + 2];
+        d = qz - p.z;
         s += d * d;
-        const int32_t id = g.sidx[t];
+        const int32_t id = p.idx;
         if (!before(s, id, bd[K - 1], bi[K - 1])) continue;
+        if (HASHED) {
+            bool held = false;
+#pragma unroll
+            for (int m = 0; m < K; ++m) held = held || bi[m] == id;
+            if (held) continue;
+        }
         bd[K - 1] = s;
         bi[K - 1] = id;
 #pragma unroll
-        for (int j = K - 1; j > 0; --j)
-            if (before(bd[j], bi[j], bd[j - 1], bi[j - 1])) {
-                const double td = bd[j];
-                bd[j] = bd[j - 1];
-                bd[j - 1] = td;
-                const int32_t ti = bi[j];
-                bi[j] = bi[j - 1];
-                bi[j - 1] = ti;
+        for (int m = K - 1; m > 0; --m)
+            if (before(bd[m], bi[m], bd[m - 1], bi[m - 1])) {
+                const double td = bd[m];
+                bd[m] = bd[m - 1];
+                bd[m - 1] = td;
+                const int32_t ti = bi[m];
+                bi[m] = bi[m - 1];
+                bi[m - 1] = ti;
             }
     }
 }
 
-// The K nearest points of q: shells of cells around q's cell until the K-th
-// squared distance is within the block's guaranteed radius (the distance
-// from q to the nearest face of the block that does not lie on the grid's
-// border, less a margin for rounding of the cell bounds).
 template <int K>
-__device__ void knn_point(const GridView &g, double qx, double qy, double qz, double (&bd)[K],
-                          int32_t (&bi)[K])
+__device__ __forceinline__ void none_yet(double (&bd)[K], int32_t (&bi)[K])
 {
 #pragma unroll
     for (int j = 0; j < K; ++j) {
         bd[j] = INFINITY;
         bi[j] = INT32_MAX;
     }
-    const int cx = cell_of(qx, g.ox, g.cell, g.dx);
-    const int cy = cell_of(qy, g.oy, g.cell, g.dy);
-    const int cz = cell_of(qz, g.oz, g.cell, g.dz);
-    const int rmax = max(g.dx, max(g.dy, g.dz));
-    const double margin = 1e-9 * g.cell;
+}
+
+// The K nearest points of q among hashed cells: shells of cells around q's
+// cell until the K-th squared distance is within the block's guaranteed
+// radius (the distance from q to the nearest face of the block that does not
+// lie on the grid's border, less a margin for rounding of the cell bounds).
+template <int K>
+__device__ __noinline__ void knn_cells(const GridView &v, double qx, double qy, double qz,
+                                       double (&bd)[K], int32_t (&bi)[K])
+{
+    const GridHead &g = *v.g;
+    const double ox = g.origin[0], oy = g.origin[1], oz = g.origin[2], cell = g.cell;
+    const int dx = g.dims[0], dy = g.dims[1], dz = g.dims[2];
+    const uint64_t mask = (uint64_t)(g.nbins - 1);
+    none_yet<K>(bd, bi);
+    const int cx = cell_of(qx, ox, cell, dx);
+    const int cy = cell_of(qy, oy, cell, dy);
+    const int cz = cell_of(qz, oz, cell, dz);
+    const int rmax = max(dx, max(dy, dz));
+    const double margin = 1e-9 * cell;
     for (int r = 0; r <= rmax; ++r) {
         for (int z = cz - r; z <= cz + r; ++z) {
-            if (z < 0 || z >= g.dz) continue;
+            if (z < 0 || z >= dz) continue;
             for (int y = cy - r; y <= cy + r; ++y) {
-                if (y < 0 || y >= g.dy) continue;
+                if (y < 0 || y >= dy) continue;
                 const bool face = (z == cz - r || z == cz + r || y == cy - r || y == cy + r);
                 const int step = (face || r == 0) ? 1 : 2 * r;
                 for (int x = cx - r; x <= cx + r; x += step) {
-                    if (x < 0 || x >= g.dx) continue;
-                    visit_cell<K>(g, x, y, z, qx, qy, qz, bd, bi);
+                    if (x < 0 || x >= dx) continue;
+                    const uint64_t m = mix64(cell_key(x, y, z));
+                    const int32_t *s = v.start + (m & mask);
+                    scan_points<K, true>(v.pts, s[0], s[1], (uint32_t)(m >> 32), qx, qy, qz, bd,
+                                         bi);
                 }
             }
         }
         double guar = INFINITY;
-        if (cx - r > 0) guar = fmin(guar, qx - (g.ox + (cx - r) * g.cell));
-        if (cx + r + 1 < g.dx) guar = fmin(guar, (g.ox + (cx + r + 1) * g.cell) - qx);
-        if (cy - r > 0) guar = fmin(guar, qy - (g.oy + (cy - r) * g.cell));
-        if (cy + r + 1 < g.dy) guar = fmin(guar, (g.oy + (cy + r + 1) * g.cell) - qy);
-        if (cz - r > 0) guar = fmin(guar, qz - (g.oz + (cz - r) * g.cell));
-        if (cz + r + 1 < g.dz) guar = fmin(guar, (g.oz + (cz + r + 1) * g.cell) - qz);
+        if (cx - r > 0) guar = fmin(guar, qx - (ox + (cx - r) * cell));
+        if (cx + r + 1 < dx) guar = fmin(guar, (ox + (cx + r + 1) * cell) - qx);
+        if (cy - r > 0) guar = fmin(guar, qy - (oy + (cy - r) * cell));
+        if (cy + r + 1 < dy) guar = fmin(guar, (oy + (cy + r + 1) * cell) - qy);
+        if (cz - r > 0) guar = fmin(guar, qz - (oz + (cz - r) * cell));
+        if (cz + r + 1 < dz) guar = fmin(guar, (oz + (cz + r + 1) * cell) - qz);
         if (guar == INFINITY) break;  // the block covers the whole grid
         guar -= margin;
         if (guar > 0.0 && bd[K - 1] <= guar * guar) break;
     }
 }
 
+// The K nearest points of q among latitude bands.  A round of reach r visits
+// the bands within r of q's and, in each, the cells within longitude D of q,
+// sin D = sin(r h) / cos(latitude of q) for a band height h (all cells where
+// that passes 1, near the poles).  Every point not visited then lies at an
+// angle of at least r h from q (its latitude differs by that, or its meridian
+// passes q no nearer), and at an angle a and norms in [rmin, rmax] its squared
+// distance is at least (|q| - t)^2 + 4 |q| t sin^2(a / 2), t = |q| cos a
+// clamped to those norms.
 template <int K>
-__device__ __forceinline__ void knn_store(int64_t p, const double (&bd)[K], const int32_t (&bi)[K],
-                                          int64_t V, double *dists, int64_t *nbrs)
+__device__ __forceinline__ void knn_shell(const GridView &v, double qx, double qy, double qz,
+                                          double (&bd)[K], int32_t (&bi)[K])
 {
+    const GridHead &g = *v.g;
+    const int bands = v.bands;
+    float lat, lon, clat;
+    angles_of(qx, qy, qz, 1.0 / g.rmax, lat, lon, clat);
+    const double qn = sqrt(qx * qx + qy * qy + qz * qz);
+    const int own = band_of(lat, bands);
+    const float h = 3.14159265f / (float)bands;
+    for (int r = K <= 3 ? 1 : 2;; r *= 2) {
+        none_yet<K>(bd, bi);
+        if (!(qn < INFINITY)) break;   // no distance to compare
+        const float a = (float)r * h;
+        const float ratio = a < 1.5f ? sinf(a) / clat : 1.0f;
+        const bool circle = !(ratio < 0.99f);
+        const float D = circle ? 0.0f : asinf(ratio) + 4.0f * kAngleSlack;
+        for (int k = 0; k <= 2 * r; ++k) {   // q's band, then outwards
+            const int b = own + ((k & 1) ? -((k + 1) >> 1) : (k >> 1));
+            if (b < 0 || b >= bands) continue;
+            const int base = v.band[b], n = v.band[b + 1] - base;
+            const int32_t *start = v.start + base;
+            const float per = (float)n * 0.159154943f;
+            int c0 = (int)floorf((lon - D) * per), c1 = (int)floorf((lon + D) * per);
+            if (circle || c1 - c0 >= n - 1) {
+                c0 = 0;
+                c1 = n - 1;
+            }
+            // cells beyond either end of the band continue at the other end
+            if (c0 < 0) {
+                scan_points<K, false>(v.pts, start[c0 + n], start[n], 0, qx, qy, qz, bd, bi);
+                c0 = 0;
+            }
+            if (c1 >= n) {
+                scan_points<K, false>(v.pts, start[0], start[c1 - n + 1], 0, qx, qy, qz, bd, bi);
+                c1 = n - 1;
+            }
+            scan_points<K, false>(v.pts, start[c0], start[c1 + 1], 0, qx, qy, qz, bd, bi);
+        }
+        if (circle && own - r <= 0 && own + r >= bands - 1) break;   // every point visited
+        double ca, s2;
+        if (r <= 2) {
+            ca = g.cosa[r - 1];
+            s2 = g.sin2a[r - 1];
+        } else {
+            const double ad = r * (3.141592653589793 / bands) - 2.0 * kAngleSlack;
+            if (ad >= 3.141592653589793) continue;   // more bands than the sphere has
+            ca = cos(ad);
+            s2 = sin(0.5 * ad) * sin(0.5 * ad);
+        }
+        const double t = fmin(fmax(qn * ca, g.rmin), g.rmax);
+        const double least = (qn - t) * (qn - t) + 4.0 * qn * t * s2;
+        if (bd[K - 1] <= least * (1.0 - kGuardSlack)) break;
+    }
+}
+
+template <int K>
+__device__ __forceinline__ void knn_point(const GridView &v, double qx, double qy, double qz,
+                                          double (&bd)[K], int32_t (&bi)[K])
+{
+    if (v.g->shell)
+        knn_shell<K>(v, qx, qy, qz, bd, bi);
+    else
+        knn_cells<K>(v, qx, qy, qz, bd, bi);
+}
+
+// Results of a block's 256 consecutive queries p0..p0+255 (of n), through
+// LDS so that the stores are contiguous (K doubles per query are not).
+template <int K>
+__device__ __forceinline__ void knn_store(int64_t p0, int64_t n, const double (&bd)[K],
+                                          const int32_t (&bi)[K], int64_t V, double *dists,
+                                          int64_t *nbrs)
+{
+    __shared__ double sd[256 * K];
+    __shared__ int32_t si[256 * K];
+    const int t = threadIdx.x;
 #pragma unroll
     for (int j = 0; j < K; ++j) {
-        dists[p * K + j] = sqrt(bd[j]);  // +inf where fewer than K points exist
-        nbrs[p * K + j] = bi[j] == INT32_MAX ? V : bi[j];
+        sd[t * K + j] = sqrt(bd[j]);  // +inf where fewer than K points exist
+        si[t * K + j] = bi[j];
+    }
+    __syncthreads();
+    const int m = (int)min((int64_t)256, n - p0) * K;
+#pragma unroll
+    for (int j = 0; j < K; ++j) {
+        const int e = j * 256 + t;
+        if (e < m) {
+            dists[p0 * K + e] = sd[e];
+            nbrs[p0 * K + e] = si[e] == INT32_MAX ? V : si[e];
+        }
     }
 }
 
 }  // namespace
 
 template <int K>
-__global__ __launch_bounds__(256) void k_knn_points(const char *__restrict__ ws,
-                                                    const double *__restrict__ spts,
-                                                    const int32_t *__restrict__ sidx,
-                                                    const CellEntry *__restrict__ table,
-                                                    uint64_t mask, int64_t V,
+__global__ __launch_bounds__(256) void k_knn_points(GridView v, int64_t V,
                                                     const double *__restrict__ q, int64_t nq,
                                                     double *__restrict__ dists,
                                                     int64_t *__restrict__ nbrs)
 {
-    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= nq) return;
-    const GridView g = grid_view(ws, spts, sidx, table, mask);
+    const int64_t p0 = (int64_t)blockIdx.x * 256, p = min(p0 + threadIdx.x, nq - 1);
     double bd[K];
     int32_t bi[K];
-    knn_point<K>(g, q[3 * p], q[3 * p + 1], q[3 * p + 2], bd, bi);
-    knn_store<K>(p, bd, bi, V, dists, nbrs);
+    knn_point<K>(v, q[3 * p], q[3 * p + 1], q[3 * p + 2], bd, bi);
+    knn_store<K>(p0, nq, bd, bi, V, dists, nbrs);
 }
 
 // trig: cos(lat_h), sin(lat_h) for each row, then cos(lon_w), sin(lon_w) for
@@ -382,27 +625,21 @@ __global__ __launch_bounds__(256) void k_knn_points(const char *__restrict__ ws,
 // numba code calls; x = (r * cos lat) * cos lon, y = (r * cos lat) * sin lon,
 // z = r * sin lat as util.py:86-88.
 template <int K>
-__global__ __launch_bounds__(256) void k_knn_pixels(const char *__restrict__ ws,
-                                                    const double *__restrict__ spts,
-                                                    const int32_t *__restrict__ sidx,
-                                                    const CellEntry *__restrict__ table,
-                                                    uint64_t mask, int64_t V, int64_t width,
+__global__ __launch_bounds__(256) void k_knn_pixels(GridView v, int64_t V, int64_t width,
                                                     int64_t height, double radius,
                                                     const double *__restrict__ trig,
                                                     double *__restrict__ dists,
                                                     int64_t *__restrict__ nbrs)
 {
-    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= width * height) return;
+    const int64_t n = width * height;
+    const int64_t p0 = (int64_t)blockIdx.x * 256, p = min(p0 + threadIdx.x, n - 1);
     const int64_t h = p / width, w = p - h * width;
     const double clat = trig[2 * h], slat = trig[2 * h + 1];
     const double clon = trig[2 * height + 2 * w], slon = trig[2 * height + 2 * w + 1];
-    const double qx = radius * clat * clon, qy = radius * clat * slon, qz = radius * slat;
-    const GridView g = grid_view(ws, spts, sidx, table, mask);
     double bd[K];
     int32_t bi[K];
-    knn_point<K>(g, qx, qy, qz, bd, bi);
-    knn_store<K>(p, bd, bi, V, dists, nbrs);
+    knn_point<K>(v, radius * clat * clon, radius * clat * slon, radius * slat, bd, bi);
+    knn_store<K>(p0, n, bd, bi, V, dists, nbrs);
 }
 
 __global__ __launch_bounds__(256) void k_ll_arr(int64_t width, int64_t height, double radius,
@@ -469,48 +706,57 @@ int knn_grid_build(nx_ctx *ctx, const double *pts, int64_t V, void *grid, hipStr
     const GridLayout L = grid_layout(V);
     char *w = (char *)grid;
     auto *g = (GridHead *)(w + L.head);
-    auto *kin = (unsigned long long *)(w + L.kin);
-    auto *kout = (unsigned long long *)(w + L.kout);
-    auto *iin = (int32_t *)(w + L.iin);
-    auto *sidx = (int32_t *)(w + L.sidx);
-    auto *spts = (double *)(w + L.spts);
-    auto *table = (CellEntry *)(w + L.table);
+    auto *band = (int32_t *)(w + L.band);
+    auto *start = (int32_t *)(w + L.start);
+    auto *bin = (uint32_t *)(w + L.bin);
+    auto *rank = (int32_t *)(w + L.rank);
+    auto *part = (unsigned long long *)(w + L.part);
+    auto *sums = (int32_t *)(w + L.part);   // the box records are read by then
     const unsigned blocks = (unsigned)((V + 255) / 256);
-    hipLaunchKernelGGL(k_grid_init, dim3(1), dim3(64), 0, stream, g);
-    hipLaunchKernelGGL(k_grid_box, dim3(std::min<unsigned>(blocks, 2048u)), dim3(256), 0, stream,
-                       pts, V, g);
-    hipLaunchKernelGGL(k_grid_setup, dim3(1), dim3(64), 0, stream, g, V);
-    hipLaunchKernelGGL(k_grid_keys, dim3(blocks), dim3(256), 0, stream, pts, V, g, kin, iin);
-    size_t temp = sort_temp_bytes(V);
-    NX_HIP(hipcub::DeviceRadixSort::SortPairs(w + L.temp, temp, (uint64_t *)kin, (uint64_t *)kout,
-                                              iin, sidx, (int)V, 0, 3 * kAxisBits, stream));
-    hipLaunchKernelGGL(k_fill_cells, dim3((unsigned)((L.tsize + 255) / 256)), dim3(256), 0, stream,
-                       table, L.tsize);
-    hipLaunchKernelGGL(k_grid_fill, dim3(blocks), dim3(256), 0, stream, pts, V, kout, sidx, spts,
-                       table, L.tsize - 1);
+    const int parts = (int)std::min<int64_t>((V + 1023) / 1024, kBoxBlocks);
+    hipLaunchKernelGGL(k_grid_box, dim3(parts), dim3(1024), 0, stream, pts, V, part);
+    hipLaunchKernelGGL(k_grid_setup, dim3(1), dim3(1024), 0, stream, g, V,
+                       (const unsigned long long *)part, parts, L.bands, L.tsize, band);
+    hipLaunchKernelGGL(k_grid_clear, dim3(std::min<unsigned>(blocks, 2048u)), dim3(256), 0, stream,
+                       (const GridHead *)g, start);
+    hipLaunchKernelGGL(k_grid_count, dim3(blocks), dim3(256), 0, stream, pts, V,
+                       (const GridHead *)g, (const int32_t *)band, L.bands, start, bin, rank);
+    const unsigned scan = std::min<unsigned>(blocks, kScanBlocks);
+    hipLaunchKernelGGL(k_grid_sums, dim3(scan), dim3(256), 0, stream, (const GridHead *)g,
+                       (const int32_t *)start, sums);
+    hipLaunchKernelGGL(k_grid_starts, dim3(scan), dim3(256), 0, stream, (const GridHead *)g, V,
+                       (const int32_t *)sums, start);
+    hipLaunchKernelGGL(k_grid_place, dim3(blocks), dim3(256), 0, stream, pts, V,
+                       (const GridHead *)g, (const int32_t *)start, (const uint32_t *)bin,
+                       (const int32_t *)rank, (GridPoint *)(w + L.pts));
     NX_HIP(hipGetLastError());
     return NX_OK;
 }
 
-template <int K>
-static void launch_points(const char *w, const GridLayout &L, int64_t V, const double *q,
-                          int64_t nq, double *dists, int64_t *nbrs, hipStream_t stream)
+static GridView grid_view(const void *grid, int64_t V)
 {
-    hipLaunchKernelGGL(k_knn_points<K>, dim3((unsigned)((nq + 255) / 256)), dim3(256), 0, stream,
-                       w, (const double *)(w + L.spts), (const int32_t *)(w + L.sidx),
-                       (const CellEntry *)(w + L.table), L.tsize - 1, V, q, nq, dists, nbrs);
+    const GridLayout L = grid_layout(V);
+    const char *w = (const char *)grid;
+    return GridView{(const GridHead *)(w + L.head), (const int32_t *)(w + L.band),
+                    (const int32_t *)(w + L.start), (const GridPoint *)(w + L.pts), L.bands};
 }
 
 template <int K>
-static void launch_pixels(const char *w, const GridLayout &L, int64_t V, int64_t width,
-                          int64_t height, double radius, const double *trig, double *dists,
-                          int64_t *nbrs, hipStream_t stream)
+static void launch_points(const GridView &v, int64_t V, const double *q, int64_t nq,
+                          double *dists, int64_t *nbrs, hipStream_t stream)
+{
+    hipLaunchKernelGGL(k_knn_points<K>, dim3((unsigned)((nq + 255) / 256)), dim3(256), 0, stream,
+                       v, V, q, nq, dists, nbrs);
+}
+
+template <int K>
+static void launch_pixels(const GridView &v, int64_t V, int64_t width, int64_t height,
+                          double radius, const double *trig, double *dists, int64_t *nbrs,
+                          hipStream_t stream)
 {
     const int64_t n = width * height;
     hipLaunchKernelGGL(k_knn_pixels<K>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream,
-                       w, (const double *)(w + L.spts), (const int32_t *)(w + L.sidx),
-                       (const CellEntry *)(w + L.table), L.tsize - 1, V, width, height, radius,
-                       trig, dists, nbrs);
+                       v, V, width, height, radius, trig, dists, nbrs);
 }
 
 #define NX_K_DISPATCH(FN, ...)                  \
@@ -534,8 +780,7 @@ int knn_query(nx_ctx *ctx, const void *grid, int64_t V, const double *q, int64_t
     if (nq == 0) return NX_OK;
     if (nq > (int64_t)UINT32_MAX * 256) return set_error(NX_EINVAL, "too many query points");
     NX_HIP(hipSetDevice(ctx->device));
-    const GridLayout L = grid_layout(V);
-    NX_K_DISPATCH(launch_points, (const char *)grid, L, V, q, nq, dists, nbrs, stream);
+    NX_K_DISPATCH(launch_points, grid_view(grid, V), V, q, nq, dists, nbrs, stream);
     NX_HIP(hipGetLastError());
     return NX_OK;
 }
@@ -594,8 +839,7 @@ int knn_query_pixels(nx_ctx *ctx, const void *grid, int64_t V, int64_t width, in
     if (k < 1 || k > kKnnMax) return set_error(NX_EINVAL, "k=%d outside 1..%d", k, kKnnMax);
     NX_HIP(hipSetDevice(ctx->device));
     if ((rc = stage_trig(ctx, width, height, ws, stream))) return rc;
-    const GridLayout L = grid_layout(V);
-    NX_K_DISPATCH(launch_pixels, (const char *)grid, L, V, width, height, radius,
+    NX_K_DISPATCH(launch_pixels, grid_view(grid, V), V, width, height, radius,
                   (const double *)ws, dists, nbrs, stream);
     NX_HIP(hipGetLastError());
     return NX_OK;

@@ -150,3 +150,60 @@ def test_export_pipeline_writes_the_oracle_image(oracle, tmp_path):
     ref_m = oracle.make_gray_array(400, 200, qd[0], qd[1],
                                    oracle.rescale_ex(ocean.astype(np.float64), 0, 255))
     assert np.array_equal(m, ref_m.astype(np.float64).astype(np.uint8))
+
+
+def _point_sets():
+    rng = np.random.default_rng(11)
+
+    def ball(n):
+        p = rng.standard_normal((n, 3))
+        return p / np.linalg.norm(p, axis=1, keepdims=True)
+    ico, _ = util.create_mesh(30)
+    thick = ball(4000) * rng.uniform(0.85, 1.0, (4000, 1))
+    return {
+        "icosphere": ico, "world": ico * 6378100.0, "random sphere": ball(5000),
+        "thick shell": thick, "thinner than a shell": ball(3000) * rng.uniform(0.7, 1, (3000, 1)),
+        "offset sphere": ico + [3.0, 0, 0], "cap": ico[ico[:, 2] > 0.9],
+        "duplicates": np.concatenate([ico, ico[::3], ico[::5]]),
+        "poles": np.concatenate([ball(300), np.tile([[0, 0, 1.0], [0, 0, -1.0]], (20, 1))]),
+        "seam": np.concatenate([ball(300), [[-np.cos(t), s * 0.0, np.sin(t)]
+                                            for t in np.linspace(-1.5, 1.5, 41) for s in (1, -1)]]),
+        "volume": rng.uniform(-1, 1, (3000, 3)), "line": np.linspace(-1, 1, 500)[:, None] * [[1, 2, 3]],
+        "one": np.array([[0.0, 0.0, 1.0]]), "six": np.concatenate([np.eye(3), -np.eye(3)]),
+        "with nan": np.concatenate([ico, [[np.nan, 0, 0]]]),
+    }
+
+
+@pytest.mark.parametrize("k", [1, 3, 4, 8])
+def test_query_every_kind_of_point_set(oracle, k):
+    """Both kinds of bins (latitude bands, hashed cells) against brute force:
+    on, near and off the points' surface, at the centre, the poles and the
+    seam of the longitudes, and at exact ties."""
+    rng = np.random.default_rng(12)
+    for name, p in _point_sets().items():
+        print(name, "k", k, flush=True)
+        fine = p[np.isfinite(p).all(axis=1)]
+        r = np.linalg.norm(fine, axis=1).max()
+        u = rng.standard_normal((300, 3))
+        u /= np.linalg.norm(u, axis=1, keepdims=True)
+        q = np.concatenate([u * r, u[:80] * r * 1.05, u[:80] * r * 0.6, u[:20] * r * 7, fine[:50],
+                            0.5 * (fine[:40] + fine[-40:][:len(fine[:40])]),
+                            r * np.array([[0, 0, 1.0], [0, 0, -1.0], [-1, 0, 0], [-1, -0.0, 0],
+                                          [0, 0, 0], [1e-9, 0, -1], [-1, 1e-12, 0.3]])])
+        d, n = util.KnnGrid(p).query(q, k=k)
+        rd, rn = oracle.knn(p, q, k)
+        if k == 1:
+            rd, rn = rd[..., 0], rn[..., 0]
+        assert np.array_equal(d, rd) and np.array_equal(n, rn)
+
+
+@pytest.mark.parametrize("wh", [(1, 2), (7, 3), (255, 2), (257, 5), (130, 131)])
+def test_query_pixels_image_edges(oracle, wh):
+    """Images that do not fill the last block, narrow and tall ones, and a
+    radius other than the points'."""
+    pts, _ = util.create_mesh(21)
+    grid = util.KnnGrid(pts * 2.0)
+    for radius in (2.0, 1.9, -2.0):
+        d, n = grid.query_pixels_device(wh[0], wh[1], radius, 3)
+        rd, rn = oracle.knn(pts * 2.0, oracle.make_ll_arr(wh[0], wh[1], radius), 3)
+        assert np.array_equal(d.cpu().numpy(), rd) and np.array_equal(n.cpu().numpy(), rn)
