@@ -22,6 +22,7 @@
 #include <vector>
 
 #include "nx_ctx.h"
+#include "nx_erosion_dev.h"
 #include "nx_reduce_dev.h"
 
 namespace nx {
@@ -50,15 +51,20 @@ struct GridHead {
     int64_t nbins;
     double rmin, rmax;          // shell: least and largest |p|
     double cosa[2], sin2a[2];   // shell: cos a and sin^2 (a / 2) of blocks of 1 and 2 bands
+    float sina[2];              // sin of 1 and 2 band heights
+    float perband;              // bands per radian
+    double unit, fixed;         // 1 and kFixed over rmax
 };
 static_assert(sizeof(GridHead) <= 256, "grid head must fit its 256 bytes");
 
-// A point in bin order; `tag` is the upper half of its cell's hash (cells).
-struct alignas(16) GridPoint {
-    double x, y, z;
-    int32_t idx;
-    uint32_t tag;
+// A point in bin order.  Shell: its coordinates in units of rmax / 2^29, so a
+// query's differences to it are exact integers (kFixed).  Cells: x is the
+// upper half of its cell's hash.
+struct alignas(16) GridEntry {
+    int32_t x, y, z, idx;
 };
+constexpr double kFixed = 0x1p29;
+constexpr int kStage = 256;   // entries a wave stages (16 KB for a block's four waves)
 
 inline size_t a256(size_t x) { return (x + 255) & ~(size_t)255; }
 
@@ -76,7 +82,7 @@ int32_t band_count(int64_t V)
 }
 
 struct GridLayout {
-    size_t head, band, start, pts, bin, rank, part, total;
+    size_t head, band, start, entry, pts, bin, rank, part, total;
     uint64_t tsize;    // bins for hashed cells
     int32_t bands;
 };
@@ -93,8 +99,10 @@ GridLayout grid_layout(int64_t V)
     o += a256(4 * ((size_t)L.bands + 1));
     L.start = o;
     o += a256(4 * ((size_t)L.tsize + 1));
+    L.entry = o;
+    o += a256(sizeof(GridEntry) * (size_t)V);
     L.pts = o;
-    o += a256(sizeof(GridPoint) * (size_t)V);
+    o += a256(24 * (size_t)V);
     L.bin = o;
     o += a256(4 * (size_t)V);
     L.rank = o;
@@ -143,9 +151,9 @@ __device__ __forceinline__ void angles_of(double x, double y, double z, double s
 
 __device__ __forceinline__ int clamp_cell(float t, int n) { return min(max((int)t, 0), n - 1); }
 
-__device__ __forceinline__ int band_of(float lat, int bands)
+__device__ __forceinline__ int band_of(float lat, int bands, float perband)
 {
-    return clamp_cell(lat * ((float)bands * 0.318309886f), bands);
+    return clamp_cell(lat * perband, bands);
 }
 
 }  // namespace
@@ -173,14 +181,27 @@ __global__ __launch_bounds__(1024) void k_grid_box(const double *__restrict__ pt
             hi[k] = q[k] > hi[k] ? q[k] : hi[k];
         }
     }
+    __shared__ unsigned long long red[16][8];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-        block_minmax(lo[k], hi[k]);
-        if (threadIdx.x == 0) {
-            part[8 * blockIdx.x + 2 * k] = lo[k];
-            part[8 * blockIdx.x + 2 * k + 1] = hi[k];
+        for (int off = 32; off > 0; off >>= 1) {
+            const unsigned long long a = __shfl_xor(lo[k], off, 64), b = __shfl_xor(hi[k], off, 64);
+            lo[k] = a < lo[k] ? a : lo[k];
+            hi[k] = b > hi[k] ? b : hi[k];
         }
-        __syncthreads();
+        if ((threadIdx.x & 63) == 0) {
+            red[threadIdx.x >> 6][2 * k] = lo[k];
+            red[threadIdx.x >> 6][2 * k + 1] = hi[k];
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < 8) {   // minima are even
+        unsigned long long a = red[0][threadIdx.x];
+        for (int w = 1; w < 16; ++w) {
+            const unsigned long long c = red[w][threadIdx.x];
+            a = ((c < a) != (threadIdx.x & 1)) ? c : a;
+        }
+        part[8 * blockIdx.x + threadIdx.x] = a;
     }
 }
 
@@ -199,21 +220,20 @@ __global__ __launch_bounds__(1024) void k_grid_setup(GridHead *__restrict__ g, i
     __shared__ double box[8];
     __shared__ int shell;
     const int t = threadIdx.x;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-        unsigned long long lo = ~0ull, hi = 0ull;
-        for (int i = t; i < parts; i += 1024) {
-            const unsigned long long a = part[8 * i + 2 * k], b = part[8 * i + 2 * k + 1];
-            lo = a < lo ? a : lo;
-            hi = b > hi ? b : hi;
+    if (t < 512) {   // wave w joins key w: minima are even
+        const int w = t >> 6;
+        unsigned long long a = part[w];
+        for (int i = t & 63; i < parts; i += 64) {
+            const unsigned long long c = part[8 * i + w];
+            a = ((c < a) != (w & 1)) ? c : a;
         }
-        block_minmax(lo, hi);
-        if (t == 0) {
-            box[2 * k] = dunkey(lo);
-            box[2 * k + 1] = dunkey(hi);
+        for (int off = 32; off > 0; off >>= 1) {
+            const unsigned long long c = __shfl_xor(a, off, 64);
+            a = ((c < a) != (w & 1)) ? c : a;
         }
-        __syncthreads();
+        if ((t & 63) == 0) box[w] = dunkey(a);
     }
+    __syncthreads();
     const double pi = 3.141592653589793, h = pi / bands;
     if (t == 0) {
         double ext[3], R = 0.0;
@@ -239,12 +259,17 @@ __global__ __launch_bounds__(1024) void k_grid_setup(GridHead *__restrict__ g, i
         g->shell = shell = s;
         g->rmin = sqrt(n0) * (1.0 - kGuardSlack);
         g->rmax = sqrt(n1) * (1.0 + kGuardSlack);
-        for (int r = 1; r <= 2; ++r) {
-            const double a = r * h - 2.0 * kAngleSlack;
-            g->cosa[r - 1] = cos(a);
-            g->sin2a[r - 1] = sin(0.5 * a) * sin(0.5 * a);
-        }
+        g->unit = 1.0 / g->rmax;
+        g->fixed = kFixed / g->rmax;
+        g->perband = (float)bands * 0.318309886f;
         if (!s) g->nbins = (int64_t)tsize;
+    }
+    if ((t & 63) == 0 && (t >> 6) >= 1 && (t >> 6) <= 2) {
+        const int r = t >> 6;
+        const double a = r * h - 2.0 * kAngleSlack, s2 = sin(0.5 * a);
+        g->cosa[r - 1] = 1.0 - 2.0 * s2 * s2;
+        g->sin2a[r - 1] = s2 * s2;
+        g->sina[r - 1] = r * h < 1.5 ? sinf((float)(r * h)) : 2.0f;
     }
     __syncthreads();
     if (!shell) return;
@@ -254,7 +279,7 @@ __global__ __launch_bounds__(1024) void k_grid_setup(GridHead *__restrict__ g, i
     for (int32_t b0 = 0; b0 < bands; b0 += 1024) {
         const int32_t b = b0 + t;
         int32_t n = 0;
-        if (b < bands) n = max(1, (int32_t)(2.0 * bands * cos((b + 0.5) * h - 0.5 * pi)));
+        if (b < bands) n = max(1, (int32_t)(2.0f * (float)bands * sinf(((float)b + 0.5f) * (float)h)));
         int32_t inc = n;
         for (int off = 1; off < 64; off <<= 1) {
             const int32_t o = __shfl_up(inc, off, 64);
@@ -286,7 +311,9 @@ __global__ __launch_bounds__(256) void k_grid_clear(const GridHead *__restrict__
         count[i] = 0;
 }
 
-// Each point's bin and its rank among the bin's points.
+// Each point's bin and its rank among the bin's points.  Bound by the counters'
+// atomics, which run at the memory side: 10,000,002 points take 308 us (337
+// with a contiguous eighth of the points on each XCD).
 __global__ __launch_bounds__(256) void k_grid_count(const double *__restrict__ pts, int64_t V,
                                                     const GridHead *__restrict__ g,
                                                     const int32_t *__restrict__ band, int32_t bands,
@@ -300,8 +327,8 @@ __global__ __launch_bounds__(256) void k_grid_count(const double *__restrict__ p
     uint32_t b;
     if (g->shell) {
         float lat, lon, clat;
-        angles_of(x, y, z, 1.0 / g->rmax, lat, lon, clat);
-        const int r = band_of(lat, bands);
+        angles_of(x, y, z, g->unit, lat, lon, clat);
+        const int r = band_of(lat, bands, g->perband);
         const int n = band[r + 1] - band[r];
         b = (uint32_t)(band[r] + clamp_cell(lon * ((float)n * 0.159154943f), n));
     } else {
@@ -367,28 +394,42 @@ __global__ __launch_bounds__(256) void k_grid_starts(const GridHead *__restrict_
     if (blockIdx.x == 0 && t == 0) start[n] = (int32_t)V;
 }
 
+// Entries in bin order; the points themselves stay in the caller's order for
+// a shell (read once per result) and go into bin order for cells (read once
+// per candidate).
 __global__ __launch_bounds__(256) void k_grid_place(const double *__restrict__ pts, int64_t V,
                                                     const GridHead *__restrict__ g,
                                                     const int32_t *__restrict__ start,
                                                     const uint32_t *__restrict__ bin,
                                                     const int32_t *__restrict__ rank,
-                                                    GridPoint *__restrict__ out)
+                                                    GridEntry *__restrict__ entry,
+                                                    double *__restrict__ out)
 {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t i = xcd_tile(blockIdx.x, gridDim.x) * 256 + threadIdx.x;
     if (i >= V) return;
-    GridPoint p;
-    p.x = pts[3 * i];
-    p.y = pts[3 * i + 1];
-    p.z = pts[3 * i + 2];
-    p.idx = (int32_t)i;
-    p.tag = 0;
-    if (!g->shell) {
+    const double x = pts[3 * i], y = pts[3 * i + 1], z = pts[3 * i + 2];
+    const int64_t at = (int64_t)start[bin[i]] + rank[i];
+    GridEntry e;
+    int64_t to = i;
+    if (g->shell) {
+        const double f = g->fixed;
+        e.x = (int32_t)rint(x * f);
+        e.y = (int32_t)rint(y * f);
+        e.z = (int32_t)rint(z * f);
+    } else {
         const double c = g->cell;
-        p.tag = (uint32_t)(mix64(cell_key(cell_of(p.x, g->origin[0], c, g->dims[0]),
-                                          cell_of(p.y, g->origin[1], c, g->dims[1]),
-                                          cell_of(p.z, g->origin[2], c, g->dims[2]))) >> 32);
+        const uint64_t m = mix64(cell_key(cell_of(x, g->origin[0], c, g->dims[0]),
+                                          cell_of(y, g->origin[1], c, g->dims[1]),
+                                          cell_of(z, g->origin[2], c, g->dims[2])));
+        e.x = (int32_t)(m >> 32);
+        e.y = e.z = 0;
+        to = at;
     }
-    out[(int64_t)start[bin[i]] + rank[i]] = p;
+    e.idx = (int32_t)i;
+    entry[at] = e;
+    out[3 * to] = x;
+    out[3 * to + 1] = y;
+    out[3 * to + 2] = z;
 }
 
 namespace {
@@ -397,7 +438,8 @@ struct GridView {
     const GridHead *g;
     const int32_t *band;
     const int32_t *start;
-    const GridPoint *pts;
+    const GridEntry *entry;
+    const double *pts;
     int32_t bands;
 };
 
@@ -406,44 +448,39 @@ __device__ __forceinline__ bool before(double s, int32_t i, double t, int32_t j)
     return s < t || (s == t && i < j);
 }
 
-// Points j0..j1-1 against the K best.  HASHED skips points of other cells
-// (another tag) and points already held (another visited cell with this tag).
-template <int K, bool HASHED>
-__device__ __forceinline__ void scan_points(const GridPoint *__restrict__ pts, int j0, int j1,
-                                            uint32_t tag, double qx, double qy, double qz,
-                                            double (&bd)[K], int32_t (&bi)[K])
+// Squared distance as the reference's KD-tree sums it.
+__device__ __forceinline__ double dist2(const double *__restrict__ p, double qx, double qy,
+                                        double qz)
 {
-    for (int j = j0; j < j1; ++j) {
-        const GridPoint p = pts[j];
-        if (HASHED && p.tag != tag) continue;
-        double s = 0.0, d;
-        d = qx - p.x;
-        s += d * d;
-        d = qy - p.y;
-        s += d * d;
-        d = qz - p.z;
-        s += d * d;
-        const int32_t id = p.idx;
-        if (!before(s, id, bd[K - 1], bi[K - 1])) continue;
-        if (HASHED) {
-            bool held = false;
+    double s = 0.0, d;
+    d = qx - p[0];
+    s += d * d;
+    d = qy - p[1];
+    s += d * d;
+    d = qz - p[2];
+    s += d * d;
+    return s;
+}
+
+__device__ __forceinline__ void order(double &s, int32_t &i, double &t, int32_t &j)
+{
+    const bool swap = before(t, j, s, i);
+    const double a = swap ? t : s, b = swap ? s : t;
+    const int32_t c = swap ? j : i, d = swap ? i : j;
+    s = a;
+    t = b;
+    i = c;
+    j = d;
+}
+
+// (s, id) into the K best so far, which are in order.
+template <int K>
+__device__ __forceinline__ void insert(double s, int32_t id, double (&bd)[K], int32_t (&bi)[K])
+{
+    bd[K - 1] = s;
+    bi[K - 1] = id;
 #pragma unroll
-            for (int m = 0; m < K; ++m) held = held || bi[m] == id;
-            if (held) continue;
-        }
-        bd[K - 1] = s;
-        bi[K - 1] = id;
-#pragma unroll
-        for (int m = K - 1; m > 0; --m)
-            if (before(bd[m], bi[m], bd[m - 1], bi[m - 1])) {
-                const double td = bd[m];
-                bd[m] = bd[m - 1];
-                bd[m - 1] = td;
-                const int32_t ti = bi[m];
-                bi[m] = bi[m - 1];
-                bi[m - 1] = ti;
-            }
-    }
+    for (int m = K - 1; m > 0; --m) order(bd[m - 1], bi[m - 1], bd[m], bi[m]);
 }
 
 template <int K>
@@ -461,7 +498,7 @@ __device__ __forceinline__ void none_yet(double (&bd)[K], int32_t (&bi)[K])
 // radius (the distance from q to the nearest face of the block that does not
 // lie on the grid's border, less a margin for rounding of the cell bounds).
 template <int K>
-__device__ __noinline__ void knn_cells(const GridView &v, double qx, double qy, double qz,
+__device__ __forceinline__ void knn_cells(const GridView &v, double qx, double qy, double qz,
                                        double (&bd)[K], int32_t (&bi)[K])
 {
     const GridHead &g = *v.g;
@@ -485,8 +522,16 @@ __device__ __noinline__ void knn_cells(const GridView &v, double qx, double qy, 
                     if (x < 0 || x >= dx) continue;
                     const uint64_t m = mix64(cell_key(x, y, z));
                     const int32_t *s = v.start + (m & mask);
-                    scan_points<K, true>(v.pts, s[0], s[1], (uint32_t)(m >> 32), qx, qy, qz, bd,
-                                         bi);
+                    for (int j = s[0]; j < s[1]; ++j) {
+                        const GridEntry e = v.entry[j];
+                        if (e.x != (int32_t)(m >> 32)) continue;   // another cell's
+                        const double s2 = dist2(v.pts + 3 * (int64_t)j, qx, qy, qz);
+                        if (!before(s2, e.idx, bd[K - 1], bi[K - 1])) continue;
+                        bool held = false;   // by another visited cell with this tag
+#pragma unroll
+                        for (int h = 0; h < K; ++h) held = held || bi[h] == e.idx;
+                        if (!held) insert<K>(s2, e.idx, bd, bi);
+                    }
                 }
             }
         }
@@ -503,104 +548,359 @@ __device__ __noinline__ void knn_cells(const GridView &v, double qx, double qy, 
     }
 }
 
-// The K nearest points of q among latitude bands.  A round of reach r visits
-// the bands within r of q's and, in each, the cells within longitude D of q,
-// sin D = sin(r h) / cos(latitude of q) for a band height h (all cells where
-// that passes 1, near the poles).  Every point not visited then lies at an
-// angle of at least r h from q (its latitude differs by that, or its meridian
-// passes q no nearer), and at an angle a and norms in [rmin, rmax] its squared
-// distance is at least (|q| - t)^2 + 4 |q| t sin^2(a / 2), t = |q| cos a
-// clamped to those norms.
-template <int K>
-__device__ __forceinline__ void knn_shell(const GridView &v, double qx, double qy, double qz,
-                                          double (&bd)[K], int32_t (&bi)[K])
+// Latitude bands.  A round of reach r visits the bands within r of q's and,
+// in each, the cells within longitude D of q, sin D = sin(r h) / cos(latitude
+// of q) for a band height h (all cells where that passes 1, near the poles).
+// Every point not visited then lies at an angle of at least r h from q (its
+// latitude differs by that, or its meridian passes q no nearer), and at an
+// angle a and norms in [rmin, rmax] its squared distance is at least
+// (|q| - t)^2 + 4 |q| t sin^2(a / 2), t = |q| cos a clamped to those norms.
+struct ShellQuery {
+    double x, y, z, norm;
+    float lat, lon, clat;
+    int own;   // q's band
+};
+
+// The visited part of a band: entries ja.. (na of them), then jb.. (to n): a
+// window past either end of the band continues at the other end.
+struct Run {
+    int ja, na, jb, n;
+    __device__ __forceinline__ int at(int i) const { return i + (i < na ? ja : jb - na); }
+};
+
+__device__ __forceinline__ Run band_run(const GridView &v, const ShellQuery &q, int b, float D,
+                                        bool circle)
+{
+    Run run{0, 0, 0, 0};
+    if (b < 0 || b >= v.bands) return run;
+    const int base = v.band[b], n = v.band[b + 1] - base;
+    const int32_t *start = v.start + base;
+    const float per = (float)n * 0.159154943f;
+    int c0 = (int)floorf((q.lon - D) * per), c1 = (int)floorf((q.lon + D) * per);
+    if (circle || c1 - c0 >= n - 1) {
+        c0 = 0;
+        c1 = n - 1;
+    }
+    const bool wrap = c0 < 0 || c1 >= n;
+    const int a = c0 < 0 ? c0 + n : c0, e = c1 >= n ? c1 - n : c1;
+    run.ja = start[a];
+    run.na = start[wrap ? n : e + 1] - run.ja;
+    run.n = run.na;
+    if (wrap) {
+        run.jb = start[0];
+        run.n += start[e + 1] - run.jb;
+    }
+    return run;
+}
+
+// asin x <= x + (pi / 2 - 1) x^3 on [0, 1].
+__device__ __forceinline__ float window(float sina, float clat, bool &circle)
+{
+    const float x = sina * __builtin_amdgcn_rcpf(clat);   // within the slack
+    circle = !(x < 0.99f);
+    return circle ? 0.0f : x * (1.0f + 0.5709f * x * x) + 4.0f * kAngleSlack;
+}
+
+// Least squared distance of a point at an angle with these terms or more.
+__device__ __forceinline__ double beyond(const GridHead &g, double qn, double ca, double s2)
+{
+    const double t = fmin(fmax(qn * ca, g.rmin), g.rmax);
+    return ((qn - t) * (qn - t) + 4.0 * qn * t * s2) * (1.0 - kGuardSlack);
+}
+
+// The first round, of reach R: the candidates' squared distances in FP32 from
+// exact integer differences, the K + 1 least kept as one word each (the
+// number of the candidate in the low bits), then FP64 for the K.  False where
+// that does not settle it: more than 64 candidates (not staged), a candidate
+// beyond the K-th that rounding (2^-17 or 2^-15 in the words, 2^-24 in the
+// sum, 2^-29 of rmax in the coordinates) could place before it, or a block
+// too small.
+// STAGED: the wave's queries lie in one row of an image, in order of
+// longitude, so their runs of a band make one run (or two, where it passes
+// the band's end, which LDS joins); where those hold at most kStage entries
+// together they are read once into LDS, as FP32 differences to the wave's
+// first query.  Bound by VALU issue (70% busy: 695 instructions per wave, 14
+// per candidate) and the FP64 points' gathers.  8192 x 4096 on d=1000: 971 us
+// (1666 with every candidate loaded by its query, 2392 with every candidate
+// in FP64); 2048 x 1024 on d=320: 76 (86, 137).
+template <int K, int R, bool STAGED>
+__device__ __forceinline__ bool knn_near(const GridView &v, const ShellQuery &q, float4 *lds,
+                                         double (&bd)[K], int32_t (&bi)[K])
+{
+    constexpr int kBands = 2 * R + 1, kMost = 64;
+    const GridHead &g = *v.g;
+    if (!(q.norm <= 2.0 * g.rmax)) return false;   // the differences stay within 31 bits
+    const double f = g.fixed;
+    const int fx = (int)rint(q.x * f), fy = (int)rint(q.y * f), fz = (int)rint(q.z * f);
+    bool circle;
+    const float D = window(g.sina[R - 1], q.clat, circle);
+    const int own = STAGED ? __builtin_amdgcn_readfirstlane(q.own) : q.own;
+    Run run[kBands];
+    int total = 0;
+    // Most waves' windows are parts of their bands, with no end in between:
+    // then each band's runs are one, from the first query's start to the last's end.
+    bool simple = STAGED && !__any(circle);
+    if (simple) {
+        int c0[kBands], c1[kBands];
+        const int32_t *start[kBands];
+#pragma unroll
+        for (int k = 0; k < kBands; ++k) {
+            const int b = own + k - R;
+            c0[k] = 0;
+            c1[k] = -1;
+            start[k] = v.start;
+            if (b < 0 || b >= v.bands) continue;
+            const int first = v.band[b], n = v.band[b + 1] - first;
+            const float per = (float)n * 0.159154943f;
+            start[k] += first;
+            c0[k] = (int)floorf((q.lon - D) * per);
+            c1[k] = (int)floorf((q.lon + D) * per);
+            simple = simple && c0[k] >= 0 && c1[k] < n && c1[k] - c0[k] < n - 1;
+        }
+        simple = __all(simple);
+        if (simple) {
+#pragma unroll
+            for (int k = 0; k < kBands; ++k) {
+                run[k].ja = start[k][(uint32_t)c0[k]];
+                run[k].n = run[k].na = start[k][(uint32_t)(c1[k] + 1)] - run[k].ja;
+                run[k].jb = 0;
+                total += run[k].n;
+            }
+        }
+    }
+    if (!simple) {
+#pragma unroll
+        for (int k = 0; k < kBands; ++k) {
+            run[k] = band_run(v, q, own + k - R, D, circle);
+            total += run[k].n;
+        }
+    }
+    // words as floats: positive, never subnormal (the squares start from 1),
+    // so a median of three places a word among the best
+    float best[K + 1];
+#pragma unroll
+    for (int m = 0; m <= K; ++m) best[m] = INFINITY;
+    uint32_t low = kMost - 1;   // the words' low bits
+    auto take = [&](float dx, float dy, float dz, uint32_t number) {
+        const float d2 = fmaf(dz, dz, fmaf(dy, dy, fmaf(dx, dx, 1.0f)));
+        const float w = __uint_as_float((__float_as_uint(d2) & ~low) | (number & low));
+#pragma unroll
+        for (int m = K; m > 0; --m) best[m] = __builtin_amdgcn_fmed3f(best[m - 1], best[m], w);
+        best[0] = __builtin_amdgcn_fmed3f(0.0f, best[0], w);
+    };
+    // each difference is off by at most 1 per axis, so a distance by 1.74, and
+    // by 1 more for the squares' 1
+    float slack = 5.0f;
+    bool staged = false;
+    if (STAGED) {
+        const int lane = threadIdx.x & 63;
+        // per band: the joined run's first piece (len entries from base), the
+        // second's start, its length, and this query's place in it
+        int base[kBands], len[kBands], from[kBands], joined[kBands], place[kBands], all = 0;
+        if (simple) {
+#pragma unroll
+            for (int k = 0; k < kBands; ++k) {
+                base[k] = __builtin_amdgcn_readfirstlane(run[k].ja);
+                len[k] = joined[k] = __builtin_amdgcn_readlane(run[k].ja + run[k].n, 63) - base[k];
+                from[k] = 0;
+                place[k] = run[k].ja - base[k];
+                all += joined[k];
+            }
+            staged = all <= kStage;
+        } else {
+            bool inside = true;
+#pragma unroll
+            for (int k = 0; k < kBands; ++k) {
+                const bool wraps = run[k].n > run[k].na;
+                const unsigned long long some = __ballot(wraps);
+                base[k] = __builtin_amdgcn_readfirstlane(run[k].ja);
+                const int last = __builtin_amdgcn_readlane(
+                    wraps ? run[k].jb + run[k].n - run[k].na : run[k].ja + run[k].na, 63);
+                if (some) {
+                    const int l = __builtin_ctzll(some);
+                    from[k] = __builtin_amdgcn_readlane(run[k].jb, l);
+                    len[k] = __builtin_amdgcn_readlane(run[k].ja + run[k].na, l) - base[k];
+                    joined[k] = len[k] + last - from[k];
+                } else {
+                    from[k] = last;
+                    len[k] = joined[k] = last - base[k];
+                }
+                all += joined[k];
+                const bool second = run[k].ja < base[k];
+                place[k] = run[k].ja + (second ? len[k] - from[k] : -base[k]);
+                // (not so near the poles, where a window may be a whole band for
+                // some of the queries only)
+                inside = inside && place[k] >= 0 && place[k] + run[k].n <= joined[k] &&
+                         !(second && wraps) && len[k] >= 0 && last <= base[k] + (some ? 0 : len[k]);
+            }
+            staged = all <= kStage && __all(inside);
+        }
+        if (staged) {
+            const int ox = __builtin_amdgcn_readfirstlane(fx);
+            const int oy = __builtin_amdgcn_readfirstlane(fy);
+            const int oz = __builtin_amdgcn_readfirstlane(fz);
+            const float qx = (float)(fx - ox), qy = (float)(fy - oy), qz = (float)(fz - oz);
+            // rounding of the differences to the first query, of either end
+            slack += (fabsf(qx) + fabsf(qy) + fabsf(qz)) * 0x1p-21f;
+            int at = 0;
+#pragma unroll
+            for (int k = 0; k < kBands; ++k) {
+                for (int t = lane; t < joined[k]; t += 64) {
+                    const GridEntry p =
+                        v.entry[(uint32_t)(simple || t < len[k] ? base[k] + t : from[k] + t - len[k])];
+                    lds[at + t] = make_float4((float)(p.x - ox), (float)(p.y - oy),
+                                              (float)(p.z - oz), __int_as_float(p.idx));
+                }
+                run[k].ja = at + place[k];
+                at += joined[k];
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            low = kStage - 1;   // a candidate's number is its place in LDS
+#pragma unroll
+            for (int k = 0; k < kBands; ++k) {
+                int j = run[k].ja;
+                const int e = j + run[k].n;
+                for (; j < e; ++j) {
+                    const float4 p = lds[j];
+                    take(qx - p.x, qy - p.y, qz - p.z, (uint32_t)j);
+                }
+            }
+        }
+    }
+    if (!staged) {
+        if (total > kMost) return false;
+        uint32_t number = 0;
+        auto visit = [&](int j, int e) {
+            for (; j < e; ++j, ++number) {
+                const GridEntry p = v.entry[j];
+                take((float)(fx - p.x), (float)(fy - p.y), (float)(fz - p.z), number);
+            }
+        };
+#pragma unroll
+        for (int k = 0; k < kBands; ++k) {
+            visit(run[k].ja, run[k].ja + run[k].na);
+            if (run[k].n > run[k].na) visit(run[k].jb, run[k].jb + run[k].n - run[k].na);
+        }
+    }
+    if (total > K) {
+        // d of the K-th rounded up and of the next rounded down, in units of
+        // rmax / 2^29
+        const float dk = __builtin_amdgcn_sqrtf(__uint_as_float(__float_as_uint(best[K - 1]) | low));
+        const float dn = __builtin_amdgcn_sqrtf(__uint_as_float(__float_as_uint(best[K]) & ~low));
+        if (!(dn > dk * (1.0f + 2e-6f) + slack)) return false;
+    }
+#pragma unroll
+    for (int m = 0; m < K; ++m) {
+        int i = (int)(__float_as_uint(best[m]) & low), j = i;
+        if (!staged) {
+#pragma unroll
+            for (int k = 0; k < kBands; ++k) {
+                if (i >= 0 && i < run[k].n) j = run[k].at(i);
+                i -= run[k].n;
+            }
+        }
+        bd[m] = INFINITY;
+        bi[m] = INT32_MAX;
+        if (m < total) {
+            bi[m] = staged ? __float_as_int(lds[j].w) : v.entry[j].idx;
+            bd[m] = dist2(v.pts + 3 * (int64_t)bi[m], q.x, q.y, q.z);
+        }
+    }
+    // in order but for rounding
+#pragma unroll
+    for (int e = 1; e < K; ++e)
+#pragma unroll
+        for (int m = e; m > 0; --m) order(bd[m - 1], bi[m - 1], bd[m], bi[m]);
+    if (circle && q.own - R <= 0 && q.own + R >= v.bands - 1) return true;   // all points visited
+    return bd[K - 1] <= beyond(g, q.norm, g.cosa[R - 1], g.sin2a[R - 1]);
+}
+
+// Rounds of doubling reach in FP64, for queries knn_near does not settle.
+// The angles' terms double with the reach (sin 2a = 2 sin a cos a).
+template <int K, int R>
+__device__ __forceinline__ void knn_rounds(const GridView &v, const ShellQuery &q, double (&bd)[K],
+                                           int32_t (&bi)[K])
 {
     const GridHead &g = *v.g;
-    const int bands = v.bands;
-    float lat, lon, clat;
-    angles_of(qx, qy, qz, 1.0 / g.rmax, lat, lon, clat);
-    const double qn = sqrt(qx * qx + qy * qy + qz * qz);
-    const int own = band_of(lat, bands);
-    const float h = 3.14159265f / (float)bands;
-    for (int r = K <= 3 ? 1 : 2;; r *= 2) {
+    const float h = 3.14159265f / (float)v.bands;
+    float sina = g.sina[R - 1];
+    double ca = g.cosa[R - 1], s2 = g.sin2a[R - 1];
+    none_yet<K>(bd, bi);
+    if (!(q.norm < INFINITY)) return;   // no distance to compare
+    for (int r = R;; r *= 2) {
         none_yet<K>(bd, bi);
-        if (!(qn < INFINITY)) break;   // no distance to compare
-        const float a = (float)r * h;
-        const float ratio = a < 1.5f ? sinf(a) / clat : 1.0f;
-        const bool circle = !(ratio < 0.99f);
-        const float D = circle ? 0.0f : asinf(ratio) + 4.0f * kAngleSlack;
+        bool circle;
+        const float D = window((float)r * h < 1.5f ? sina : 2.0f, q.clat, circle);
         for (int k = 0; k <= 2 * r; ++k) {   // q's band, then outwards
-            const int b = own + ((k & 1) ? -((k + 1) >> 1) : (k >> 1));
-            if (b < 0 || b >= bands) continue;
-            const int base = v.band[b], n = v.band[b + 1] - base;
-            const int32_t *start = v.start + base;
-            const float per = (float)n * 0.159154943f;
-            int c0 = (int)floorf((lon - D) * per), c1 = (int)floorf((lon + D) * per);
-            if (circle || c1 - c0 >= n - 1) {
-                c0 = 0;
-                c1 = n - 1;
+            const Run run = band_run(v, q, q.own + ((k & 1) ? -((k + 1) >> 1) : (k >> 1)), D, circle);
+            for (int i = 0; i < run.n; ++i) {
+                const int32_t id = v.entry[run.at(i)].idx;
+                const double s = dist2(v.pts + 3 * (int64_t)id, q.x, q.y, q.z);
+                if (before(s, id, bd[K - 1], bi[K - 1])) insert<K>(s, id, bd, bi);
             }
-            // cells beyond either end of the band continue at the other end
-            if (c0 < 0) {
-                scan_points<K, false>(v.pts, start[c0 + n], start[n], 0, qx, qy, qz, bd, bi);
-                c0 = 0;
-            }
-            if (c1 >= n) {
-                scan_points<K, false>(v.pts, start[0], start[c1 - n + 1], 0, qx, qy, qz, bd, bi);
-                c1 = n - 1;
-            }
-            scan_points<K, false>(v.pts, start[c0], start[c1 + 1], 0, qx, qy, qz, bd, bi);
         }
-        if (circle && own - r <= 0 && own + r >= bands - 1) break;   // every point visited
-        double ca, s2;
-        if (r <= 2) {
-            ca = g.cosa[r - 1];
-            s2 = g.sin2a[r - 1];
-        } else {
-            const double ad = r * (3.141592653589793 / bands) - 2.0 * kAngleSlack;
-            if (ad >= 3.141592653589793) continue;   // more bands than the sphere has
-            ca = cos(ad);
-            s2 = sin(0.5 * ad) * sin(0.5 * ad);
-        }
-        const double t = fmin(fmax(qn * ca, g.rmin), g.rmax);
-        const double least = (qn - t) * (qn - t) + 4.0 * qn * t * s2;
-        if (bd[K - 1] <= least * (1.0 - kGuardSlack)) break;
+        if (circle && q.own - r <= 0 && q.own + r >= v.bands - 1) return;   // all points visited
+        // a reach of pi or more passes every band: the next round covers all
+        if ((float)r * h < 3.14f && bd[K - 1] <= beyond(g, q.norm, ca, s2)) return;
+        sina = 2.0f * sina * sqrtf(fmaxf(1.0f - sina * sina, 0.0f));
+        s2 = 4.0 * s2 * (1.0 - s2);
+        ca = 1.0 - 2.0 * s2;
     }
 }
 
-template <int K>
-__device__ __forceinline__ void knn_point(const GridView &v, double qx, double qy, double qz,
+template <int K, bool STAGED>
+__device__ __forceinline__ void knn_shell(const GridView &v, const ShellQuery &q, float4 *lds,
                                           double (&bd)[K], int32_t (&bi)[K])
 {
-    if (v.g->shell)
-        knn_shell<K>(v, qx, qy, qz, bd, bi);
-    else
-        knn_cells<K>(v, qx, qy, qz, bd, bi);
+    constexpr int R = K <= 3 ? 1 : 2;
+    if (!knn_near<K, R, STAGED>(v, q, lds, bd, bi)) knn_rounds<K, R>(v, q, bd, bi);
 }
 
-// Results of a block's 256 consecutive queries p0..p0+255 (of n), through
-// LDS so that the stores are contiguous (K doubles per query are not).
-template <int K>
-__device__ __forceinline__ void knn_store(int64_t p0, int64_t n, const double (&bd)[K],
-                                          const int32_t (&bi)[K], int64_t V, double *dists,
-                                          int64_t *nbrs)
+__device__ __forceinline__ ShellQuery shell_query(const GridView &v, double x, double y, double z)
 {
-    __shared__ double sd[256 * K];
-    __shared__ int32_t si[256 * K];
+    ShellQuery q{x, y, z, sqrt(x * x + y * y + z * z), 0.0f, 0.0f, 0.0f, 0};
+    angles_of(x, y, z, v.g->unit, q.lat, q.lon, q.clat);
+    q.own = band_of(q.lat, v.bands, v.g->perband);
+    return q;
+}
+
+// LDS of a query block: the staged entries of its four waves, then its results.
+template <int K>
+union KnnLds {
+    float4 entry[4][kStage];
+    struct {
+        double d[256 * K];
+        int32_t i[256 * K];
+    } out;
+};
+
+// Results of a block's `count` (up to 256) consecutive queries from p0 on,
+// through LDS so that the stores are contiguous (K doubles per query are not).
+template <int K>
+__device__ __forceinline__ void knn_store(KnnLds<K> &lds, int64_t p0, int count,
+                                          const double (&bd)[K], const int32_t (&bi)[K], int64_t V,
+                                          double *dists, int64_t *nbrs)
+{
+    double *sd = lds.out.d;
+    int32_t *si = lds.out.i;
     const int t = threadIdx.x;
+    __syncthreads();   // every wave is done with its entries
 #pragma unroll
     for (int j = 0; j < K; ++j) {
         sd[t * K + j] = sqrt(bd[j]);  // +inf where fewer than K points exist
         si[t * K + j] = bi[j];
     }
     __syncthreads();
-    const int m = (int)min((int64_t)256, n - p0) * K;
+    dists += p0 * K;
+    nbrs += p0 * K;
+    const int m = count * K;
 #pragma unroll
     for (int j = 0; j < K; ++j) {
         const int e = j * 256 + t;
         if (e < m) {
-            dists[p0 * K + e] = sd[e];
-            nbrs[p0 * K + e] = si[e] == INT32_MAX ? V : si[e];
+            dists[e] = sd[e];
+            nbrs[e] = si[e] == INT32_MAX ? V : si[e];
         }
     }
 }
@@ -614,32 +914,69 @@ __global__ __launch_bounds__(256) void k_knn_points(GridView v, int64_t V,
                                                     int64_t *__restrict__ nbrs)
 {
     const int64_t p0 = (int64_t)blockIdx.x * 256, p = min(p0 + threadIdx.x, nq - 1);
+    __shared__ KnnLds<K> lds;
     double bd[K];
     int32_t bi[K];
-    knn_point<K>(v, q[3 * p], q[3 * p + 1], q[3 * p + 2], bd, bi);
-    knn_store<K>(p0, nq, bd, bi, V, dists, nbrs);
+    const double x = q[3 * p], y = q[3 * p + 1], z = q[3 * p + 2];
+    if (v.g->shell)
+        knn_shell<K, false>(v, shell_query(v, x, y, z), nullptr, bd, bi);
+    else
+        knn_cells<K>(v, x, y, z, bd, bi);
+    knn_store<K>(lds, p0, (int)min((int64_t)256, nq - p0), bd, bi, V, dists, nbrs);
 }
 
 // trig: cos(lat_h), sin(lat_h) for each row, then cos(lon_w), sin(lon_w) for
 // each column, computed on the host with the C library the reference's
 // numba code calls; x = (r * cos lat) * cos lon, y = (r * cos lat) * sin lon,
 // z = r * sin lat as util.py:86-88.
-template <int K>
+// ROWS: a block's pixels lie in one row, and stripes of 1 << stripe rows go to
+// the XCDs in turn (blockIdx.x is the XCD: consecutive blocks go round them),
+// so that an XCD's L2 reads the points of its stripes once: 8192 x 4096 on
+// d=1000 STRIPES.  Otherwise blocks take 256 pixels across rows.
+template <int K, bool ROWS>
 __global__ __launch_bounds__(256) void k_knn_pixels(GridView v, int64_t V, int64_t width,
-                                                    int64_t height, double radius,
-                                                    const double *__restrict__ trig,
+                                                    int64_t height, double radius, int stripe,
+                                                    float dlat, float dlon, const double *__restrict__ trig,
                                                     double *__restrict__ dists,
                                                     int64_t *__restrict__ nbrs)
 {
-    const int64_t n = width * height;
-    const int64_t p0 = (int64_t)blockIdx.x * 256, p = min(p0 + threadIdx.x, n - 1);
-    const int64_t h = p / width, w = p - h * width;
+    int64_t p0, h, w;
+    int count;
+    if (ROWS) {
+        const int z = blockIdx.z, row = z & ((1 << stripe) - 1);
+        h = ((((z >> stripe) << 3) + (int)blockIdx.x) << stripe) + row;
+        if (h >= height) return;
+        const int w0 = blockIdx.y * 256;
+        count = min(256, (int)width - w0);
+        w = w0 + min((int)threadIdx.x, count - 1);
+        p0 = h * width + w0;
+    } else {
+        const int64_t n = width * height;
+        p0 = (int64_t)blockIdx.x * 256;
+        count = (int)min((int64_t)256, n - p0);
+        const int64_t p = p0 + min((int)threadIdx.x, count - 1);
+        h = p / width;
+        w = p - h * width;
+    }
     const double clat = trig[2 * h], slat = trig[2 * h + 1];
     const double clon = trig[2 * height + 2 * w], slon = trig[2 * height + 2 * w + 1];
+    const double x = radius * clat * clon, y = radius * clat * slon, z = radius * slat;
+    __shared__ KnnLds<K> lds;
     double bd[K];
     int32_t bi[K];
-    knn_point<K>(v, radius * clat * clon, radius * clat * slon, radius * slat, bd, bi);
-    knn_store<K>(p0, n, bd, bi, V, dists, nbrs);
+    if (!v.g->shell) {
+        knn_cells<K>(v, x, y, z, bd, bi);
+    } else if (radius > 0.0) {
+        // the angles are the pixel's own
+        ShellQuery q{x, y, z, radius, 0.0f, 0.0f, (float)clat, 0};
+        q.lat = 3.14159265f - (float)(int)h * dlat;
+        q.lon = (float)(int)w * dlon;
+        q.own = band_of(q.lat, v.bands, v.g->perband);
+        knn_shell<K, ROWS>(v, q, lds.entry[threadIdx.x >> 6], bd, bi);
+    } else {
+        knn_shell<K, false>(v, shell_query(v, x, y, z), nullptr, bd, bi);
+    }
+    knn_store<K>(lds, p0, count, bd, bi, V, dists, nbrs);
 }
 
 __global__ __launch_bounds__(256) void k_ll_arr(int64_t width, int64_t height, double radius,
@@ -656,39 +993,81 @@ __global__ __launch_bounds__(256) void k_ll_arr(int64_t width, int64_t height, d
     out[3 * p + 2] = radius * slat;
 }
 
-// util.py:356-364 over k neighbours: sd = sum(d); w_i = 1 / ((d_i + 0.00001)
+// util.py:356-364 over K neighbours: sd = sum(d); w_i = 1 / ((d_i + 0.00001)
 // / sd); t = sum(w); value = int(sum(colors[n_i] * (w_i / t))), each sum
 // accumulated from 0 in neighbour order; truncation toward zero.
-__global__ __launch_bounds__(256) void k_gray(int64_t npix, int k, const double *__restrict__ dists,
+template <int K>
+__device__ __forceinline__ int32_t gray_value(const double (&d)[K], const int64_t (&n)[K],
+                                              const double *__restrict__ colors, int64_t ncolors,
+                                              bool &bad)
+{
+    double c[K], w[K];
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+        const bool out = n[i] < 0 || n[i] >= ncolors;
+        bad = bad || out;
+        c[i] = out ? 0.0 : colors[n[i]];
+    }
+    double sd = 0.0, t = 0.0, v = 0.0;
+#pragma unroll
+    for (int i = 0; i < K; ++i) sd += d[i];
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+        w[i] = 1.0 / ((d[i] + 0.00001) / sd);
+        t += w[i];
+    }
+#pragma unroll
+    for (int i = 0; i < K; ++i)
+        if (n[i] >= 0 && n[i] < ncolors) v += c[i] * (w[i] / t);
+    return (int32_t)(int64_t)v;
+}
+
+// A block's 256 K distances and indices come through LDS, so that the loads
+// are contiguous (K doubles per pixel are not).  Bound by reading 16 K bytes
+// per pixel: 8192 x 4096, K = 3: 409 us, 500 with a pixel's own loads.
+template <int K>
+__global__ __launch_bounds__(256) void k_gray(int64_t npix, const double *__restrict__ dists,
                                               const int64_t *__restrict__ nbrs,
                                               const double *__restrict__ colors, int64_t ncolors,
                                               int32_t *__restrict__ out, int *__restrict__ err)
 {
-    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= npix) return;
-    double d[kKnnMax], ws[kKnnMax];
-    double sd = 0.0;
-    for (int i = 0; i < k; ++i) {
-        d[i] = dists[p * k + i];
-        sd += d[i];
+    __shared__ double sd[256 * K];
+    __shared__ int64_t sn[256 * K];
+    const int t = threadIdx.x;
+    const int64_t p0 = (int64_t)blockIdx.x * 256;
+    const int count = (int)min((int64_t)256, npix - p0), m = count * K;
+    double a[K];
+    int64_t b[K];
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+        const int e = min(i * 256 + t, m - 1);
+        b[i] = __builtin_nontemporal_load(&nbrs[p0 * K + e]);
+        a[i] = __builtin_nontemporal_load(&dists[p0 * K + e]);
     }
-    double t = 0.0;
-    for (int i = 0; i < k; ++i) {
-        ws[i] = 1.0 / ((d[i] + 0.00001) / sd);
-        t += ws[i];
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+        sn[i * 256 + t] = b[i];
+        sd[i * 256 + t] = a[i];
     }
-    double v = 0.0;
+    __syncthreads();
+    if (t >= count) return;
+#pragma unroll
+    for (int i = 0; i < K; ++i) {
+        b[i] = sn[t * K + i];
+        a[i] = sd[t * K + i];
+    }
     bool bad = false;
-    for (int i = 0; i < k; ++i) {
-        const int64_t n = nbrs[p * k + i];
-        if (n < 0 || n >= ncolors) {
-            bad = true;
-            continue;
-        }
-        v += colors[n] * (ws[i] / t);
-    }
-    out[p] = (int32_t)(int64_t)v;
+    out[p0 + t] = gray_value<K>(a, b, colors, ncolors, bad);
     if (bad) __hip_atomic_fetch_or(err, NX_ERR_INDEX_BIT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+template <int K>
+static void launch_gray(int64_t npix, const double *dists, const int64_t *nbrs,
+                        const double *colors, int64_t ncolors, int32_t *out, int *err,
+                        hipStream_t stream)
+{
+    hipLaunchKernelGGL(k_gray<K>, dim3((unsigned)((npix + 255) / 256)), dim3(256), 0, stream, npix,
+                       dists, nbrs, colors, ncolors, out, err);
 }
 
 size_t knn_grid_bytes(int64_t V)
@@ -712,7 +1091,7 @@ int knn_grid_build(nx_ctx *ctx, const double *pts, int64_t V, void *grid, hipStr
     auto *rank = (int32_t *)(w + L.rank);
     auto *part = (unsigned long long *)(w + L.part);
     auto *sums = (int32_t *)(w + L.part);   // the box records are read by then
-    const unsigned blocks = (unsigned)((V + 255) / 256);
+    const unsigned blocks = (unsigned)((V + 255) / 256), by8 = (blocks + 7) / 8 * 8;
     const int parts = (int)std::min<int64_t>((V + 1023) / 1024, kBoxBlocks);
     hipLaunchKernelGGL(k_grid_box, dim3(parts), dim3(1024), 0, stream, pts, V, part);
     hipLaunchKernelGGL(k_grid_setup, dim3(1), dim3(1024), 0, stream, g, V,
@@ -726,9 +1105,10 @@ int knn_grid_build(nx_ctx *ctx, const double *pts, int64_t V, void *grid, hipStr
                        (const int32_t *)start, sums);
     hipLaunchKernelGGL(k_grid_starts, dim3(scan), dim3(256), 0, stream, (const GridHead *)g, V,
                        (const int32_t *)sums, start);
-    hipLaunchKernelGGL(k_grid_place, dim3(blocks), dim3(256), 0, stream, pts, V,
+    hipLaunchKernelGGL(k_grid_place, dim3(by8), dim3(256), 0, stream, pts, V,
                        (const GridHead *)g, (const int32_t *)start, (const uint32_t *)bin,
-                       (const int32_t *)rank, (GridPoint *)(w + L.pts));
+                       (const int32_t *)rank, (GridEntry *)(w + L.entry),
+                       (double *)(w + L.pts));
     NX_HIP(hipGetLastError());
     return NX_OK;
 }
@@ -738,7 +1118,8 @@ static GridView grid_view(const void *grid, int64_t V)
     const GridLayout L = grid_layout(V);
     const char *w = (const char *)grid;
     return GridView{(const GridHead *)(w + L.head), (const int32_t *)(w + L.band),
-                    (const int32_t *)(w + L.start), (const GridPoint *)(w + L.pts), L.bands};
+                    (const int32_t *)(w + L.start), (const GridEntry *)(w + L.entry),
+                    (const double *)(w + L.pts), L.bands};
 }
 
 template <int K>
@@ -754,9 +1135,20 @@ static void launch_pixels(const GridView &v, int64_t V, int64_t width, int64_t h
                           double radius, const double *trig, double *dists, int64_t *nbrs,
                           hipStream_t stream)
 {
-    const int64_t n = width * height;
-    hipLaunchKernelGGL(k_knn_pixels<K>, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream,
-                       v, V, width, height, radius, trig, dists, nbrs);
+    const float dlat = 3.14159265f / (float)(height - 1), dlon = 6.28318531f / (float)width;
+    if (width >= 256 && width <= (1 << 23) && height <= (1 << 18)) {
+        int stripe = 4;
+        while (stripe > 0 && (64 << stripe) > height) --stripe;   // 8 stripes or more to an XCD
+        const int64_t groups = (height + (8 << stripe) - 1) >> (3 + stripe);
+        hipLaunchKernelGGL((k_knn_pixels<K, true>),
+                           dim3(8, (unsigned)((width + 255) / 256), (unsigned)(groups << stripe)),
+                           dim3(256), 0, stream, v, V, width, height, radius, stripe, dlat, dlon,
+                           trig, dists, nbrs);
+        return;
+    }
+    hipLaunchKernelGGL((k_knn_pixels<K, false>), dim3((unsigned)((width * height + 255) / 256)),
+                       dim3(256), 0, stream, v, V, width, height, radius, 0, dlat, dlon,
+                       trig, dists, nbrs);
 }
 
 #define NX_K_DISPATCH(FN, ...)                  \
@@ -869,8 +1261,7 @@ int make_gray_array(nx_ctx *ctx, int64_t npix, int k, const double *dists, const
     if (npix == 0) return NX_OK;
     if (npix > (int64_t)UINT32_MAX * 256) return set_error(NX_EINVAL, "too many pixels");
     NX_HIP(hipSetDevice(ctx->device));
-    hipLaunchKernelGGL(k_gray, dim3((unsigned)((npix + 255) / 256)), dim3(256), 0, stream, npix, k,
-                       dists, nbrs, colors, ncolors, out, ctx->d_err);
+    NX_K_DISPATCH(launch_gray, npix, dists, nbrs, colors, ncolors, out, ctx->d_err, stream);
     NX_HIP(hipGetLastError());
     return NX_OK;
 }

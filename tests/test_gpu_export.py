@@ -207,3 +207,15 @@ def test_query_pixels_image_edges(oracle, wh):
         d, n = grid.query_pixels_device(wh[0], wh[1], radius, 3)
         rd, rn = oracle.knn(pts * 2.0, oracle.make_ll_arr(wh[0], wh[1], radius), 3)
         assert np.array_equal(d.cpu().numpy(), rd) and np.array_equal(n.cpu().numpy(), rn)
+
+
+@pytest.mark.parametrize("d,wh", [(3, (256, 64)), (9, (256, 200)), (33, (257, 131)), (64, (300, 77)),
+                                  (40, (1000, 400)), (150, (512, 90))])
+def test_query_pixels_rows_share_their_points(oracle, d, wh):
+    """Images at least a block wide, whose rows read their points together:
+    few and many points to a wave, windows that pass the ends of a band, and
+    whole bands near the poles for some pixels of a wave only."""
+    pts, _ = util.create_mesh(d)
+    d_, n_ = util.KnnGrid(pts).query_pixels_device(wh[0], wh[1], 1.0, 3)
+    rd, rn = oracle.knn(pts, oracle.make_ll_arr(wh[0], wh[1], 1.0), 3)
+    assert np.array_equal(d_.cpu().numpy(), rd) and np.array_equal(n_.cpu().numpy(), rn)
