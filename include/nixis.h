@@ -366,6 +366,19 @@ int nx_tile_plan_build_chunk(const int32_t *col, const double *elen, int64_t V,
                              int steps, int chunk, void *out, int64_t cap,
                              nx_tile_plan *plan);
 
+/* nx_tile_plan_build_chunk for four steps, made on the device from col and
+ * elen there: the same image byte for byte.  ws: 256-byte aligned device
+ * memory of nx_tile_plan_device_workspace_bytes(V, chunk) bytes.  With out ==
+ * NULL it cuts the tiles, waits for the stream and fills `plan`; called again
+ * with the same workspace and plan and a zeroed device buffer of plan->bytes
+ * it writes the image there, on the stream.  NX_ERANGE also for a neighbour
+ * table that is not symmetric, which only the host planner takes. */
+size_t nx_tile_plan_device_workspace_bytes(int64_t V, int chunk);
+int nx_tile_plan_build_device(nx_ctx *ctx, const int32_t *col,
+                              const double *elen, int64_t V, int chunk,
+                              void *ws, void *out, int64_t cap,
+                              nx_tile_plan *plan, void *stream);
+
 /* nx_erosion_run with a tile plan (NULL plan: exactly nx_erosion_run).
  * Steps go plan->steps per launch; with a 4-step plan a remainder of 2 or 3
  * steps takes one launch, and a last single step runs alone. */

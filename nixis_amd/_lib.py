@@ -151,6 +151,10 @@ SIGNATURES = {
                                     ctypes.POINTER(NxTilePlan)]),
     "nx_tile_plan_build_steps": (_c_int, [_c_void_p, _c_void_p, _c_i64, _c_int, _c_void_p, _c_i64,
                                           ctypes.POINTER(NxTilePlan)]),
+    "nx_tile_plan_device_workspace_bytes": (_c_size, [_c_i64, _c_int]),
+    "nx_tile_plan_build_device": (_c_int, [_c_void_p, _c_void_p, _c_void_p, _c_i64, _c_int,
+                                           _c_void_p, _c_void_p, _c_i64,
+                                           ctypes.POINTER(NxTilePlan), _c_void_p]),
     "nx_tile_plan_build_chunk": (_c_int, [_c_void_p, _c_void_p, _c_i64, _c_int, _c_int, _c_void_p,
                                           _c_i64, ctypes.POINTER(NxTilePlan)]),
     "nx_erosion_run_tiled": (_c_int, [_c_void_p, _c_void_p, _c_i64, _c_void_p, _c_void_p,

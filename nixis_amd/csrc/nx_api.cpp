@@ -437,6 +437,19 @@ int nx_tile_plan_build_chunk(const int32_t *col, const double *elen, int64_t V, 
     return tile_plan_build(col, elen, V, steps, out, cap, plan, chunk);
 }
 
+size_t nx_tile_plan_device_workspace_bytes(int64_t V, int chunk)
+{
+    return tile_plan_device_workspace_bytes(V, chunk);
+}
+
+int nx_tile_plan_build_device(nx_ctx *ctx, const int32_t *col, const double *elen, int64_t V,
+                              int chunk, void *ws, void *out, int64_t cap, nx_tile_plan *plan,
+                              void *stream)
+{
+    return tile_plan_build_device(ctx, col, elen, V, chunk, ws, out, cap, plan,
+                                  (hipStream_t)stream);
+}
+
 int nx_erosion_store(nx_ctx *ctx, const void *state, int64_t V, double *h, double *w, double *s,
                      void *stream)
 {

@@ -135,6 +135,10 @@ int interpolate_insolation(nx_ctx *ctx, const double *verts, int64_t V, const fl
                            double radius, float *out, hipStream_t stream);
 int yearly_insolation(nx_ctx *ctx, const double *verts, int64_t V, double radius,
                       double axial_tilt, float *out, void *ws, hipStream_t stream);
+size_t tile_plan_device_workspace_bytes(int64_t V, int chunk);
+int tile_plan_build_device(nx_ctx *ctx, const int32_t *col, const double *elen, int64_t V,
+                           int chunk, void *ws, void *out, int64_t cap, nx_tile_plan *plan,
+                           hipStream_t stream);
 size_t knn_grid_bytes(int64_t V);
 int knn_grid_build(nx_ctx *ctx, const double *pts, int64_t V, void *grid, hipStream_t stream);
 int knn_query(nx_ctx *ctx, const void *grid, int64_t V, const double *q, int64_t nq, int k,

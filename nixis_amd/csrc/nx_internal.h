@@ -44,6 +44,8 @@ int ell_from_adjacency(const int32_t *adj, int64_t V, const double *verts,
                        const int64_t *order, int32_t *col, double *elen);
 
 // Tile plan for two steps per launch (nx_tiles.cpp).
+// Section offsets, tile count, steps and size of a plan image.
+void plan_layout(nx_tile_plan &q, int64_t nt, int64_t nring, int64_t ncs, int64_t nlen, int K);
 int tile_plan_build(const int32_t *col, const double *elen, int64_t V, int K, void *out,
                     int64_t cap, nx_tile_plan *plan, int chunk = 0);
 

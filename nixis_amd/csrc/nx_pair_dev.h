@@ -92,6 +92,18 @@ NX_EHD int len_index(int col, int owner, int cs, int T)
     return col < kLenFull ? mul_small(col, cs) + owner
                           : kLenFull * cs + mul_small(col - kLenFull, cs - T) + (owner - T);
 }
+// Doubles of a tile's length block: kt columns over c step-1 vertices, the
+// columns from kLenFull on over the ring vertices T..c-1 only.
+NX_EHD int64_t len_block(int kt, int c, int T)
+{
+    return (int64_t)(kt < kLenFull ? kt : kLenFull) * c +
+           (int64_t)(kt > kLenFull ? kt - kLenFull : 0) * (c - T);
+}
+// The choice of the lengths' owners (nx_tiles.cpp, tile_edges): first cap of
+// a ring vertex, rounds before giving up, the label of a vertex without a path.
+constexpr int kOwnRing = 4;
+constexpr int kOwnRounds = 2000;
+constexpr int kOwnFar = 255;
 NX_EHD int slot_nbr(int code) { return code & 4095; }
 template <class P>
 NX_EHD double slot_len(int code, int li, int cs, int T, P len)

@@ -112,48 +112,38 @@ bool cut(const int32_t *col, int64_t V, int64_t a, int64_t len, int K, int limit
            cut(col, V, a + h, len - h, K, limit, step1_limit, out);
 }
 
-// Doubles of a tile's length block: kt columns over c step-1 vertices, the
-// columns from kLenFull on over the ring vertices T..c-1 only.
-inline int64_t len_block(int kt, int c, int T)
-{
-    return (int64_t)std::min(kt, kLenFull) * c + (int64_t)std::max(kt - kLenFull, 0) * (c - T);
-}
-
 // Edge lengths of one tile, stored once per undirected edge.  Every length
 // the tile's step-1 vertices (local 0..c-1, the tile's own 0..T-1 first)
 // read belongs to one of them: an edge to a vertex outside that set to the
 // vertex inside it, an edge between two of them to one of the two.  The
 // owners are chosen so that each of the tile's own vertices holds at most
-// kLenFull edges and the ring vertices as few as possible: greedy (an edge
-// between an own and a ring vertex to the ring vertex, else to the end that
-// holds fewer), then augmenting paths move ownership away from vertices over
-// their cap (kLenFull for own vertices, kr for ring vertices, kr growing
-// where no path exists).  Owner o's j-th owned edge (in slot order) has its
-// length at len_index(j, o, c, T) (nx_pair_dev.h): columns below kLenFull
-// hold all c vertices, later ones the ring vertices only.  The slot code is
-// the neighbour's local index (bits 0-11), the length's column (bits 12-14)
-// and bit 15 set when the slot's own vertex is the owner.  A pad slot (the
-// vertex itself) is coded as owned, column 0: a tie adds nothing, whatever
-// the length.  lc [6][c]: local neighbour index of each slot; len [6][c]:
-// its length.  Returns the number of columns kt, or -1 when an own vertex
-// cannot be held to kLenFull edges (a neighbour table that is not symmetric
-// can force more on it); writes codes [6][c] and the len_block(kt, c, T)
-// lengths when given.
-int tile_edges(const int32_t *lc, const double *len, int c, int T, uint16_t *codes,
-               double *lens)
+// kLenFull edges and the ring vertices as few as possible: an edge between an
+// own and a ring vertex starts with the ring vertex, any other with its end
+// of lower device index, then synchronous rounds move ownership away from
+// vertices over their cap (kLenFull for own vertices, kr for ring vertices):
+// each round labels every vertex with its distance to one under its cap along
+// owned edges, and each vertex over its cap passes its first edge towards
+// one; kr grows where none has a path.  A round's moves do not depend on
+// their order, so the device's planner (nx_plan_dev.hip), where a tile's
+// vertices move at once, makes the same plan.  Owner o's j-th owned edge (in
+// slot order) has its length at len_index(j, o, c, T) (nx_pair_dev.h): columns
+// below kLenFull hold all c vertices, later ones the ring vertices only.  The
+// slot code is the neighbour's local index (bits 0-11), the length's column
+// (bits 12-14) and bit 15 set when the slot's own vertex is the owner.  A pad
+// slot (the vertex itself) is coded as owned, column 0: a tie adds nothing,
+// whatever the length.  lc [6][c]: local neighbour index of each slot; len
+// [6][c]: its length; dev [c]: the vertices' device indices.  Returns the
+// number of columns kt, or -1 when an own vertex cannot be held to kLenFull
+// edges (a neighbour table that is not symmetric can force more on it);
+// writes codes [6][c] and the len_block(kt, c, T) lengths when given.
+int tile_edges(const int32_t *lc, const double *len, const int32_t *dev, int c, int T,
+               uint16_t *codes, double *lens)
 {
-    struct Edge {
-        int32_t u, v;
-        int8_t ku, kv;
-        int32_t owner;
-    };
-    std::vector<Edge> E;
-    std::vector<int32_t> own((size_t)c, 0);
-    std::vector<std::vector<int32_t>> inc((size_t)c);   // internal edges at each vertex
-    // a slot whose edge its own vertex must hold: the neighbour is outside
-    // the step-1 set, or (a table that is not symmetric) has no slot back
-    std::vector<int8_t> forced((size_t)6 * c, 0);
-    auto back = [&](int32_t n, int32_t j) {
+    // bit k of own[j]: j holds the edge of its slot k; of movable[j]: the
+    // other end could hold it (the neighbour is in the set and the two slots
+    // name each other first)
+    std::vector<uint8_t> own((size_t)c, 0), movable((size_t)c, 0), back((size_t)6 * c, 0);
+    auto first = [&](int32_t n, int32_t j) {
         for (int q = 0; q < 6; ++q)
             if (lc[(size_t)q * c + n] == j) return q;
         return -1;
@@ -162,87 +152,71 @@ int tile_edges(const int32_t *lc, const double *len, int c, int T, uint16_t *cod
         for (int k = 0; k < 6; ++k) {
             const int32_t n = lc[(size_t)k * c + j];
             if (n == j) continue;
-            if (n >= c || back(n, j) < 0) {
-                forced[(size_t)k * c + j] = 1;
-                ++own[(size_t)j];
+            const int q = n < c ? first(n, j) : -1;
+            bool mine = true;
+            if (q >= 0 && first(j, n) == k) {
+                back[(size_t)k * c + j] = (uint8_t)q;
+                movable[(size_t)j] |= (uint8_t)(1 << k);
+                mine = (j >= T) != (n >= T) ? j >= T : dev[j] < dev[n];
             }
+            if (mine) own[(size_t)j] |= (uint8_t)(1 << k);
         }
-    for (int32_t j = 0; j < c; ++j)
-        for (int k = 0; k < 6; ++k) {
-            const int32_t n = lc[(size_t)k * c + j];
-            if (n == j || forced[(size_t)k * c + j] || j > n) continue;
-            const int kv = back(n, j);
-            if (forced[(size_t)kv * c + n]) continue;
-            const bool jr = j >= T, nr = n >= T;
-            const int32_t o = jr != nr ? (jr ? j : n) : (own[(size_t)j] <= own[(size_t)n] ? j : n);
-            ++own[(size_t)o];
-            inc[(size_t)j].push_back((int32_t)E.size());
-            inc[(size_t)n].push_back((int32_t)E.size());
-            E.push_back(Edge{j, n, (int8_t)k, (int8_t)kv, o});
-        }
-    int kr = kLenFull;
-    auto cap = [&](int32_t v) { return v < T ? kLenFull : kr; };
-    std::vector<int32_t> prev((size_t)c);
-    std::vector<int32_t> queue;
-    for (int32_t s = 0; s < c; ++s) {
-        while (own[(size_t)s] > cap(s)) {
-            // breadth-first search over owned edges (x owns e: e can move to the
-            // other end) for a vertex holding fewer than its cap
-            std::fill(prev.begin(), prev.end(), -2);
-            prev[(size_t)s] = -1;
-            queue.assign(1, s);
-            int32_t found = -1;
-            for (size_t h = 0; h < queue.size() && found < 0; ++h) {
-                const int32_t x = queue[h];
-                for (int32_t e : inc[(size_t)x]) {
-                    if (E[(size_t)e].owner != x) continue;
-                    const int32_t y = E[(size_t)e].u == x ? E[(size_t)e].v : E[(size_t)e].u;
-                    if (prev[(size_t)y] != -2) continue;
-                    prev[(size_t)y] = e;
-                    if (own[(size_t)y] < cap(y)) {
-                        found = y;
+    auto held = [&](int32_t j) { return __builtin_popcount(own[(size_t)j]); };
+    int kr = kOwnRing;
+    auto cap = [&](int32_t j) { return j < T ? kLenFull : kr; };
+    std::vector<uint8_t> dist((size_t)c);
+    std::vector<int32_t> over, moves;   // vertices over their cap; slots that pass an edge
+    for (int round = 0;; ++round) {
+        over.clear();
+        for (int32_t j = 0; j < c; ++j)
+            if (held(j) > cap(j)) over.push_back(j);
+        if (over.empty()) break;
+        if (round == kOwnRounds) return -1;
+        for (int32_t j = 0; j < c; ++j) dist[(size_t)j] = held(j) < cap(j) ? 0 : kOwnFar;
+        for (int s = 1; s < kOwnFar; ++s) {
+            bool changed = false;
+            for (int32_t j = 0; j < c; ++j) {
+                if (dist[(size_t)j] != kOwnFar) continue;
+                const int m = own[(size_t)j] & movable[(size_t)j];
+                for (int k = 0; k < 6; ++k)
+                    if ((m >> k & 1) && dist[(size_t)lc[(size_t)k * c + j]] == s - 1) {
+                        dist[(size_t)j] = (uint8_t)s;
+                        changed = true;
                         break;
                     }
-                    queue.push_back(y);
+            }
+            if (!changed) break;
+            if (std::none_of(over.begin(), over.end(),
+                             [&](int32_t j) { return dist[(size_t)j] == kOwnFar; }))
+                break;
+        }
+        moves.clear();
+        for (int32_t j : over) {
+            if (dist[(size_t)j] == kOwnFar) continue;
+            const int m = own[(size_t)j] & movable[(size_t)j];
+            for (int k = 0; k < 6; ++k)
+                if ((m >> k & 1) &&
+                    dist[(size_t)lc[(size_t)k * c + j]] == dist[(size_t)j] - 1) {
+                    moves.push_back(6 * j + k);
+                    break;
                 }
-            }
-            if (found < 0) {
-                if (s < T) return -1;
-                ++kr;
-                continue;
-            }
-            for (int32_t y = found; y != s;) {
-                Edge &e = E[(size_t)prev[(size_t)y]];
-                const int32_t x = e.u == y ? e.v : e.u;
-                e.owner = y;
-                y = x;
-            }
-            --own[(size_t)s];
-            ++own[(size_t)found];
+        }
+        if (moves.empty()) {
+            if (kr >= 6) return -1;
+            ++kr;
+        }
+        for (int32_t e : moves) {
+            const int32_t j = e / 6, k = e % 6;
+            own[(size_t)j] &= (uint8_t)~(1 << k);
+            own[(size_t)lc[(size_t)k * c + j]] |= (uint8_t)(1 << back[(size_t)k * c + j]);
         }
     }
     int kt = 1;
-    for (int32_t j = 0; j < c; ++j) kt = std::max(kt, own[(size_t)j]);
+    for (int32_t j = 0; j < c; ++j) kt = std::max(kt, held(j));
     if (!codes) return kt;
     // columns in slot order of each owner
-    std::vector<int8_t> owns(forced);                  // slot (k, j) holds j's own edge
-    for (const Edge &e : E) {
-        if (e.owner == e.u)
-            owns[(size_t)e.ku * c + e.u] = 1;
-        else
-            owns[(size_t)e.kv * c + e.v] = 1;
-    }
-    std::vector<int8_t> colof((size_t)6 * c, 0);
+    auto column = [&](int32_t j, int k) { return __builtin_popcount(own[(size_t)j] & ((1 << k) - 1)); };
     std::fill(lens, lens + len_block(kt, c, T), 0.0);
-    for (int32_t j = 0; j < c; ++j) {
-        int m = 0;
-        for (int k = 0; k < 6; ++k)
-            if (owns[(size_t)k * c + j]) {
-                colof[(size_t)k * c + j] = (int8_t)m;
-                lens[len_index(m, j, c, T)] = len[(size_t)k * c + j];
-                ++m;
-            }
-    }
     for (int32_t j = 0; j < c; ++j)
         for (int k = 0; k < 6; ++k) {
             const size_t sl = (size_t)k * c + j;
@@ -250,11 +224,11 @@ int tile_edges(const int32_t *lc, const double *len, int c, int T, uint16_t *cod
             uint32_t code;
             if (n == j) {
                 code = (uint32_t)j | 0x8000u;
-            } else if (owns[sl]) {
-                code = (uint32_t)n | (uint32_t)colof[sl] << 12 | 0x8000u;
-            } else {
-                const int q = back(n, j);   // n owns the edge, in its slot back to j
-                code = (uint32_t)n | (uint32_t)colof[(size_t)q * c + n] << 12;
+            } else if (own[(size_t)j] >> k & 1) {
+                code = (uint32_t)n | (uint32_t)column(j, k) << 12 | 0x8000u;
+                lens[len_index(column(j, k), j, c, T)] = len[sl];
+            } else {   // n owns the edge, in its slot back to j
+                code = (uint32_t)n | (uint32_t)column(n, back[sl]) << 12;
             }
             codes[sl] = (uint16_t)code;
         }
@@ -264,6 +238,24 @@ int tile_edges(const int32_t *lc, const double *len, int c, int T, uint16_t *cod
 inline int64_t a256(int64_t x) { return (x + 255) & ~(int64_t)255; }
 
 }  // namespace
+
+void plan_layout(nx_tile_plan &q, int64_t nt, int64_t nring, int64_t ncs, int64_t nlen, int K)
+{
+    q.ntiles = nt;
+    q.steps = K;
+    int64_t o = 0;
+    q.off_start = o; o = a256(o + 4 * (nt + 1));
+    q.off_cs = o;    o = a256(o + 4 * nt);
+    q.off_load = o;  o = a256(o + 4 * nt);
+    q.off_rbase = o; o = a256(o + 8 * (nt + 1));
+    q.off_ring = o;  o = a256(o + 4 * nring);
+    q.off_cbase = o; o = a256(o + 8 * (nt + 1));
+    q.off_lcol = o;  o = a256(o + 2 * 6 * ncs);
+    q.off_lel = o;   o = a256(o + 8 * nlen);
+    q.off_pref = o;  o = a256(o + 4 * (K + 1) * nt);
+    q.off_ebase = o; o = a256(o + 8 * (nt + 1));
+    q.bytes = o;
+}
 
 int tile_plan_build(const int32_t *col, const double *elen, int64_t V, int K, void *out,
                     int64_t cap, nx_tile_plan *plan, int chunk_in)
@@ -325,7 +317,7 @@ int tile_plan_build(const int32_t *col, const double *elen, int64_t V, int K, vo
     // vertices (the tile, then rings 1..K-1).
     std::atomic<int> bad{0};
     auto local_table = [&](const Tile &t, std::vector<int32_t> &flat, std::vector<int32_t> &lc,
-                           std::vector<double> &ln) {
+                           std::vector<double> &ln, std::vector<int32_t> &dev) {
         const int64_t a = t.a, b = t.a + t.T;
         flat.clear();
         for (auto &x : t.r) flat.insert(flat.end(), x.begin(), x.end());
@@ -342,8 +334,10 @@ int tile_plan_build(const int32_t *col, const double *elen, int64_t V, int K, vo
         const int32_t c = t.T + t.ring_total() - (int32_t)t.r.back().size();
         lc.resize((size_t)6 * c);
         ln.resize((size_t)6 * c);
+        dev.resize((size_t)c);
         for (int32_t j = 0; j < c; ++j) {
             const int64_t v = j < t.T ? a + j : flat[(size_t)(j - t.T)];
+            dev[(size_t)j] = (int32_t)v;
             for (int k = 0; k < 6; ++k) {
                 const int32_t l = local(col[(int64_t)k * V + v]);
                 if (l < 0) bad.store(1);
@@ -357,12 +351,12 @@ int tile_plan_build(const int32_t *col, const double *elen, int64_t V, int K, vo
     // so the writing pass below recomputes the same orientation).
     std::vector<int32_t> kts((size_t)nt, 0);
     parallel_for(nt, [&](int64_t t0, int64_t t1) {
-        std::vector<int32_t> flat, lc;
+        std::vector<int32_t> flat, lc, dev;
         std::vector<double> ln;
         for (int64_t i = t0; i < t1; ++i) {
-            const int32_t c = local_table(*tiles[(size_t)i], flat, lc, ln);
-            kts[(size_t)i] = tile_edges(lc.data(), ln.data(), c, tiles[(size_t)i]->T, nullptr,
-                                        nullptr);
+            const int32_t c = local_table(*tiles[(size_t)i], flat, lc, ln, dev);
+            kts[(size_t)i] = tile_edges(lc.data(), ln.data(), dev.data(), c,
+                                        tiles[(size_t)i]->T, nullptr, nullptr);
         }
     }, 64);
     if (bad.load()) return set_error(NX_EINVAL, "tile plan: a neighbour fell outside its tile's rings");
@@ -380,23 +374,10 @@ int tile_plan_build(const int32_t *col, const double *elen, int64_t V, int K, vo
     nx_tile_plan q;
     std::memset(&q, 0, sizeof(q));
     q.V = V;
-    q.ntiles = nt;
     q.max_tile = max_tile;
     q.max_load = max_load;
     q.max_step1 = max_step1;
-    int64_t o = 0;
-    q.off_start = o; o = a256(o + 4 * (nt + 1));
-    q.off_cs = o;    o = a256(o + 4 * nt);
-    q.off_load = o;  o = a256(o + 4 * nt);
-    q.off_rbase = o; o = a256(o + 8 * (nt + 1));
-    q.off_ring = o;  o = a256(o + 4 * nring);
-    q.off_cbase = o; o = a256(o + 8 * (nt + 1));
-    q.off_lcol = o;  o = a256(o + 2 * 6 * ncs);
-    q.off_lel = o;   o = a256(o + 8 * nlen);
-    q.off_pref = o;  o = a256(o + 4 * (K + 1) * nt);
-    q.off_ebase = o; o = a256(o + 8 * (nt + 1));
-    q.steps = K;
-    q.bytes = o;
+    plan_layout(q, nt, nring, ncs, nlen, K);
     q.blob = plan->blob;
     *plan = q;
     if (!out || cap < q.bytes) return NX_OK;
@@ -432,13 +413,14 @@ int tile_plan_build(const int32_t *col, const double *elen, int64_t V, int K, vo
     }
     start[nt] = (int32_t)V;
     parallel_for(nt, [&](int64_t t0, int64_t t1) {
-        std::vector<int32_t> flat, lc;
+        std::vector<int32_t> flat, lc, dev;
         std::vector<double> ln;
         for (int64_t i = t0; i < t1; ++i) {
             const Tile &t = *tiles[(size_t)i];
-            const int32_t c = local_table(t, flat, lc, ln);
+            const int32_t c = local_table(t, flat, lc, ln, dev);
             std::copy(flat.begin(), flat.end(), ring + rbase[i]);
-            tile_edges(lc.data(), ln.data(), c, t.T, lcol + 6 * cbase[i], lel + ebase[i]);
+            tile_edges(lc.data(), ln.data(), dev.data(), c, t.T, lcol + 6 * cbase[i],
+                       lel + ebase[i]);
         }
     }, 64);
     if (bad.load()) return set_error(NX_EINVAL, "tile plan: a neighbour fell outside its tile's rings");

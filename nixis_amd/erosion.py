@@ -97,7 +97,7 @@ class ErosionGraph:
         self.elen = torch.from_numpy(elen).to(device)
         self.device = self.col.device
         self.plan = None
-        self.stream_bytes_per_launch = None
+        self._stream_bytes = None
         self._plan_blob = None
         self.steps = int(steps)
         self._tuning(chunk, variant, graph_chunk)
@@ -114,7 +114,8 @@ class ErosionGraph:
                     chunk=0, variant=None, graph_chunk=None):
         """The same graph from device tensors (verts float64 [V,3], neighbours
         int32 [V,6]), built on the device (nx_sfc_order_device,
-        nx_ell_from_adjacency_device); the tile plan is cut on the host from
+        nx_ell_from_adjacency_device, nx_tile_plan_build_device); a two-step
+        plan, or one the device planner refuses, is cut on the host from
         copies of the device tables."""
         import torch
         from . import util
@@ -142,13 +143,55 @@ class ErosionGraph:
         self._odev = order
         self.order = order.cpu().numpy() if order is not None else None
         self.plan = None
-        self.stream_bytes_per_launch = None
+        self._stream_bytes = None
         self._plan_blob = None
         self.steps = int(steps)
         self._tuning(chunk, variant, graph_chunk)
-        if tiled:
+        if tiled and not (self.steps == 4 and self._build_plan_device(stream)):
             self._build_plan(col.cpu().numpy(), elen.cpu().numpy())
         return self
+
+    def _build_plan_device(self, stream):
+        """The four-step plan from the device tables; False when refused."""
+        import torch
+        L = _lib.lib()
+        plan = _lib.NxTilePlan()
+        ctx = _lib.Context.get(self.device)
+        with torch.cuda.stream(stream):      # the buffers belong to the planner's stream
+            ws = torch.empty(int(L.nx_tile_plan_device_workspace_bytes(self.V, self.chunk)),
+                             dtype=torch.uint8, device=self.device)
+
+            def build(out, cap):
+                return L.nx_tile_plan_build_device(
+                    ctx.handle, _lib.ptr(self.col), _lib.ptr(self.elen), self.V, self.chunk,
+                    _lib.ptr(ws), _lib.ptr(out), cap, ctypes.byref(plan), _lib.stream_ptr(stream))
+            rc = build(None, 0)
+            if rc == _lib.NX_ERANGE:
+                return False
+            _lib.check(rc)
+            blob = torch.zeros(plan.bytes, dtype=torch.uint8, device=self.device)
+            _lib.check(build(blob, plan.bytes))
+        if stream is not None:
+            ctx.sync_check(stream)
+        self._set_plan(plan, blob)
+        return True
+
+    def _set_plan(self, plan, blob):
+        if blob.data_ptr() % 256:
+            raise RuntimeError("tile plan copy is not 256-byte aligned")
+        plan.blob = blob.data_ptr()
+        self.plan = plan
+        self._plan_blob = blob
+
+    @property
+    def stream_bytes_per_launch(self):
+        """Contiguous bytes one launch reads (_plan_stream_bytes), from the
+        plan's image; None without a plan."""
+        if self.plan is None:
+            return None
+        if self._stream_bytes is None:
+            self._stream_bytes = _plan_stream_bytes(self.plan, self._plan_blob.cpu().numpy(), self.V)
+        return self._stream_bytes
 
     def _build_plan(self, col, elen):
         import torch
@@ -167,13 +210,8 @@ class ErosionGraph:
         _lib.check(L.nx_tile_plan_build_chunk(_lib.ptr(col), _lib.ptr(elen), self.V, self.steps,
                                               self.chunk, _lib.ptr(img), plan.bytes,
                                               ctypes.byref(plan)))
-        self.stream_bytes_per_launch = _plan_stream_bytes(plan, img, self.V)
-        blob = torch.from_numpy(img).to(self.device)
-        if blob.data_ptr() % 256:
-            raise RuntimeError("tile plan copy is not 256-byte aligned")
-        plan.blob = blob.data_ptr()
-        self.plan = plan
-        self._plan_blob = blob
+        self._stream_bytes = _plan_stream_bytes(plan, img, self.V)
+        self._set_plan(plan, torch.from_numpy(img).to(self.device))
 
     @property
     def nbytes(self):
