@@ -54,8 +54,9 @@ int nx_abi_version(void);
 int nx_ctx_create(int device, nx_ctx **out);
 int nx_ctx_destroy(nx_ctx *ctx);
 /* Context options (nx_ctx_set_option). */
-#define NX_OPT_GRAPH_CHUNK 1 /* erosion steps per captured hipGraph; 0 = eager
-                                launches (default 32)                        */
+#define NX_OPT_GRAPH_CHUNK 1 /* erosion steps per captured hipGraph of a run
+                                without a tile plan; 0 = eager launches
+                                (default 32)                                 */
 #define NX_OPT_PAIR_KERNEL 2 /* two-step erosion kernel variant, 0..6 (0 =
                                 default); a tuning knob, results identical   */
 #define NX_OPT_MULTI_KERNEL 3 /* four-step erosion kernel variant, 0..4 (0 =
@@ -299,7 +300,8 @@ int nx_erosion_load(nx_ctx *ctx, void *state, int64_t V, const double *h,
  * (erosion_iteration3): `iters` Jacobi steps; before each step `rain` is
  * added to every vertex's water (the reference's water += 0.3/320; pass 0
  * for a bare erosion_iteration3).  Multi-step runs replay captured
- * hipGraphs of NX_OPT_GRAPH_CHUNK steps, cached per context.
+ * hipGraphs of NX_OPT_GRAPH_CHUNK steps, cached per context (runs over a tile
+ * plan, whose launches outlast their submission, launch eagerly).
  *   col   device int32 [6,V]  neighbour of each slot (self for a pad slot)
  *   elen  device f64 [6,V]    edge length of each slot (0 for a pad) */
 int nx_erosion_run(nx_ctx *ctx, void *state, int64_t V, const int32_t *col,
@@ -356,8 +358,10 @@ int nx_tile_plan_build_steps(const int32_t *col, const double *elen, int64_t V,
                              nx_tile_plan *plan);
 
 /* nx_tile_plan_build_steps with the starting tile size `chunk` (kTileMin =
- * 32 .. 1024 vertices for 2 steps, .. 2048 for 4; 0 for the default, 768 for
- * 2 steps and 1152 for 4).
+ * 32 .. 1024 vertices for 2 steps, .. 2048 for 4; 0 for the default: 768 for
+ * 2 steps; for 4 steps 1152, or less for planets of up to 1.2 million vertices,
+ * so that a launch fills the GPU; batches of planets, which fill it together,
+ * are faster with 1152).
  * Tiles are halved from there until their rings fit, so the chunk trades
  * ring overhead against the number of blocks per launch; the erosion
  * autotuner picks it per mesh size.  The results of erosion do not depend on

@@ -59,6 +59,12 @@ def _L():
     return L
 
 
+# Starting tile size of a batch's plans: planets that share launches fill the
+# GPU together, so their tiles are full ones (the library's default makes a
+# small planet's tiles smaller to spread them over an otherwise idle GPU).
+BATCH_CHUNK = 1152
+
+
 def even_divisions(d):
     """nixis.py:142-146: odd subdivision counts are rounded up to even."""
     d = int(d)
@@ -158,7 +164,7 @@ class MeshCache:
             if tuning is None:
                 from . import autotune
                 tuning = autotune.lookup_erosion(10 * d * d + 2)
-            kw = tuning.graph_kwargs() if tuning is not None else {}
+            kw = tuning.graph_kwargs() if tuning is not None else {"chunk": BATCH_CHUNK}
             g = self._build_graph(d, **kw)
             self._graphs[d] = g
         return g

@@ -53,20 +53,39 @@ static ErosionBufs bufs(void *state, int64_t V)
     return b;
 }
 
-// Launch j of a sequence reads the buffer that j earlier launches flipped
-// to; the step counter and buffer come from the workspace so that replays
-// of a captured sequence stay correct.  RULE 3 or 4 (nx_erosion_dev.h).
+// The buffer that launch j of a run reads: the current one for launch 0, and
+// what j launches flipped it to for later ones, which take it from meta->base
+// (left there by launch 0) so that the last launch can advance the step
+// counter and the current buffer by itself: no launch reads the field that
+// it, or one beside it, writes.  `done` is the run's steps in its last launch
+// (never launch 0, k_advance follows that one) and 0 in the others.
+__device__ __forceinline__ int launch_buffer(ErosionMeta *meta, int j, int64_t done)
+{
+    const int p = j ? (meta->base + j) & 1 : meta->buf;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        if (j == 0) meta->base = p;
+        if (done) {
+            meta->it += done;
+            meta->buf = p ^ 1;
+        }
+    }
+    return p;
+}
+
+// The step counter and buffer come from the workspace so that replays of a
+// captured sequence stay correct.  RULE 3 or 4 (nx_erosion_dev.h).
 template <int RULE>
-__global__ __launch_bounds__(256) void k_erode_step(const ErosionMeta *__restrict__ meta,
+__global__ __launch_bounds__(256) void k_erode_step(ErosionMeta *__restrict__ meta,
                                                     double2 *__restrict__ hw0,
                                                     double2 *__restrict__ hw1,
                                                     double *__restrict__ s0,
                                                     double *__restrict__ s1, int64_t V,
                                                     const int32_t *__restrict__ col,
                                                     const double *__restrict__ elen,
-                                                    int64_t nblocks, int j, double rain_next)
+                                                    int64_t nblocks, int j, int64_t done,
+                                                    double rain_next)
 {
-    const int p = (meta->buf + j) & 1;
+    const int p = launch_buffer(meta, j, done);
     const int64_t tile = xcd_tile(blockIdx.x, nblocks);
     const int64_t i = tile * blockDim.x + threadIdx.x;
     if (tile < nblocks && i < V)
@@ -77,25 +96,27 @@ __global__ __launch_bounds__(256) void k_erode_step(const ErosionMeta *__restric
 // Two steps per launch, one block per tile of the plan (nx_pair_dev.h).
 // B holds step one's results, at most kStepOneMax (tile + ring 1) vertices.
 template <int THREADS, bool KEEP, int RULE = 3>
-__global__ __launch_bounds__(THREADS) void k_erode_pair(const ErosionMeta *__restrict__ meta,
+__global__ __launch_bounds__(THREADS) void k_erode_pair(ErosionMeta *__restrict__ meta,
                                                        double2 *__restrict__ hw0,
                                                        double2 *__restrict__ hw1,
                                                        double *__restrict__ s0,
-                                                       double *__restrict__ s1, TilePlanDev P,
-                                                       int j, double rain_mid, double rain_next)
+                                                       double *__restrict__ s1, TilePlanDev P, int j,
+                                                       int64_t done, double rain_first,
+                                                       double rain_mid, double rain_next)
 {
     __shared__ double2 A[kLoadMax];
     __shared__ double2 B[THREADS == 1024 ? kStepOneMax : 1];
+    const int p = launch_buffer(meta, j, done);
     const int64_t tile = xcd_tile(blockIdx.x, P.ntiles);
     if (tile >= P.ntiles) return;
     erode_tile_pair<THREADS, KEEP, RULE>(A, THREADS == 1024 ? B : nullptr, hw0, hw1, s0, s1,
-                                         (meta->buf + j) & 1, P, tile, rain_mid, rain_next);
+                                         p, P, tile, rain_mid, rain_next);
 }
 
 // Kernel variants (NX_OPT_PAIR_KERNEL): block size and register use.
 struct PairVariant {
-    void (*fn)(const ErosionMeta *, double2 *, double2 *, double *, double *, TilePlanDev, int,
-               double, double);
+    void (*fn)(ErosionMeta *, double2 *, double2 *, double *, double *, TilePlanDev, int, int64_t,
+               double, double, double);
     int threads;
 };
 static const PairVariant kPairVariants[] = {
@@ -109,17 +130,19 @@ static const PairVariant kPairRule4 = {k_erode_pair<1024, true, 4>, 1024};
 
 // kMultiSteps steps per launch over a plan built for them (nx_pair_dev.h).
 template <int THREADS, bool KEEP, int RULE = 3>
-__global__ __launch_bounds__(THREADS) void k_erode_multi(const ErosionMeta *__restrict__ meta,
+__global__ __launch_bounds__(THREADS) void k_erode_multi(ErosionMeta *__restrict__ meta,
                                                         double2 *__restrict__ hw0,
                                                         double2 *__restrict__ hw1,
                                                         double *__restrict__ s0,
-                                                        double *__restrict__ s1, TilePlanDev P,
-                                                        int j, double rain_mid, double rain_next)
+                                                        double *__restrict__ s1, TilePlanDev P, int j,
+                                                       int64_t done, double rain_first,
+                                                       double rain_mid, double rain_next)
 {
     __shared__ double2 A[kLoadMaxMulti];
+    const int p = launch_buffer(meta, j, done);
     const int64_t tile = xcd_tile(blockIdx.x, P.ntiles);
     if (tile >= P.ntiles) return;
-    erode_tile_multi<THREADS, kMultiSteps, KEEP, RULE>(A, hw0, hw1, s0, s1, (meta->buf + j) & 1, P,
+    erode_tile_multi<THREADS, kMultiSteps, KEEP, RULE>(A, hw0, hw1, s0, s1, p, P,
                                                       tile, rain_mid, rain_next);
 }
 
@@ -127,20 +150,22 @@ __global__ __launch_bounds__(THREADS) void k_erode_multi(const ErosionMeta *__re
 // the steps alternating between two LDS buffers (nx_pair_dev.h); the plan
 // keeps tile + rings 1..3 within kQuadStepOne and tile + rings within
 // kQuadLoadMax.  NS = 2 or 3: the last two or three of those steps.
-template <int RULE = 3, int NS = 4>
-__global__ __launch_bounds__(1024) void k_erode_quad(const ErosionMeta *__restrict__ meta,
+template <int RULE = 3, int NS = 4, bool FIRST = false>
+__global__ __launch_bounds__(1024) void k_erode_quad(ErosionMeta *__restrict__ meta,
                                                     double2 *__restrict__ hw0,
                                                     double2 *__restrict__ hw1,
                                                     double *__restrict__ s0,
                                                     double *__restrict__ s1, TilePlanDev P, int j,
-                                                    double rain_mid, double rain_next)
+                                                       int64_t done, double rain_first,
+                                                       double rain_mid, double rain_next)
 {
     __shared__ double2 A[kQuadLoadMax];
     __shared__ double2 B[kQuadStepOne];
+    const int p = launch_buffer(meta, j, done);
     const int64_t tile = xcd_tile(blockIdx.x, P.ntiles);
     if (tile >= P.ntiles) return;
-    erode_tile_quad<RULE, NS>(A, B, hw0, hw1, s0, s1, (meta->buf + j) & 1, P, tile, rain_mid,
-                              rain_next);
+    erode_tile_quad<RULE, NS, FIRST>(A, B, hw0, hw1, s0, s1, p, P, tile, rain_mid,
+                              rain_next, rain_first);
 }
 
 // NX_OPT_MULTI_KERNEL variants: 0 keeps each thread's first-step data in
@@ -157,6 +182,11 @@ static const PairVariant kMultiRule4 = {k_erode_quad<4>, 1024};
 static const PairVariant kQuadTails[2][2] = {   // [rule 4][steps 3]
     {{k_erode_quad<3, 2>, 1024}, {k_erode_quad<3, 3>, 1024}},
     {{k_erode_quad<4, 2>, 1024}, {k_erode_quad<4, 3>, 1024}},
+};
+// The first launch of a run with rain, by its steps 2..4.
+static const PairVariant kQuadFirst[2][3] = {
+    {{k_erode_quad<3, 2, true>, 1024}, {k_erode_quad<3, 3, true>, 1024}, {k_erode_quad<3, 4, true>, 1024}},
+    {{k_erode_quad<4, 2, true>, 1024}, {k_erode_quad<4, 3, true>, 1024}, {k_erode_quad<4, 4, true>, 1024}},
 };
 
 // erosion.py:76-99 (erosion_iteration1): w[i] = r[i] + amt with amt moved
@@ -313,93 +343,60 @@ int erosion_load(nx_ctx *ctx, void *state, int64_t V, const double *h, const dou
 }
 
 // Launch n consecutive steps (the launches read the step counter and the
-// current buffer from the workspace) and advance the workspace by n steps.
+// current buffer from the workspace, and the last of several advances them).
 // With a two-step plan, steps go two per launch and an odd last step runs
 // alone; with a four-step plan, four per launch and a last two or three in
 // one tail launch.  The last step's rain for a following step is `rain`
-// unless `last`.
+// unless `last`; `rain` is also added before the first step when `first`, by
+// the first launch itself where that is a k_erode_quad.
 static void launch_steps(const ErosionBufs &b, int64_t V, const int32_t *col, const double *elen,
                          const nx_tile_plan *plan, int variant, int mvariant, int rule, int n,
-                         double rain, bool last, hipStream_t stream)
+                         double rain, bool first, bool last, hipStream_t stream)
 {
     const int64_t nblocks = (V + 255) / 256;
     const int64_t grid = ((nblocks + 7) / 8) * 8;
-    int k = 0, j = 0;
-    if (plan && plan->steps == kMultiSteps) {
-        const TilePlanDev P = plan_dev(*plan);
-        const int64_t tgrid = ((P.ntiles + 7) / 8) * 8;
-        const PairVariant &mv = rule == 4 ? kMultiRule4 : kMultiVariants[mvariant];
-        for (; k + kMultiSteps <= n; k += kMultiSteps, ++j) {
-            const double rain_next = (last && k + kMultiSteps == n) ? 0.0 : rain;
-            hipLaunchKernelGGL(mv.fn, dim3((unsigned)tgrid), dim3(mv.threads), 0, stream, b.meta,
-                               b.hw[0], b.hw[1], b.s[0], b.s[1], P, j, rain, rain_next);
+    const int per = plan ? plan->steps : 1;       // steps of a full launch
+    const bool quad = plan && per == kMultiSteps && n >= 2 && (rule == 4 || mvariant == 0);
+    const int tail = per == kMultiSteps && n % per >= 2 ? 1 : 0;
+    const int launches = n / per + (tail ? 1 : n % per);
+    if (first && rain != 0.0 && !quad)
+        hipLaunchKernelGGL(k_add_rain, dim3((unsigned)nblocks), dim3(256), 0, stream, b.meta,
+                           b.hw[0], b.hw[1], V, rain);
+    const TilePlanDev P = plan ? plan_dev(*plan) : TilePlanDev{};
+    const unsigned tgrid = (unsigned)(((P.ntiles + 7) / 8) * 8);
+    for (int k = 0, j = 0; k < n; ++j) {
+        const int steps = n - k >= per ? per : tail ? n - k : 1;
+        const bool end = k + steps == n;
+        const double rain_next = last && end ? 0.0 : rain;
+        const int64_t done = end && j > 0 ? n : 0;
+        if (steps == 1) {
+            hipLaunchKernelGGL(rule == 4 ? k_erode_step<4> : k_erode_step<3>, dim3((unsigned)grid),
+                               dim3(256), 0, stream, b.meta, b.hw[0], b.hw[1], b.s[0], b.s[1], V,
+                               col, elen, nblocks, j, done, rain_next);
+        } else {
+            const bool wet = first && j == 0 && quad && rain != 0.0;
+            const PairVariant &v = wet          ? kQuadFirst[rule == 4][steps - 2]
+                                   : steps < per ? kQuadTails[rule == 4][steps - 2]
+                                   : per == 2    ? (rule == 4 ? kPairRule4 : kPairVariants[variant])
+                                                 : (rule == 4 ? kMultiRule4 : kMultiVariants[mvariant]);
+            hipLaunchKernelGGL(v.fn, dim3(tgrid), dim3(v.threads), 0, stream, b.meta, b.hw[0],
+                               b.hw[1], b.s[0], b.s[1], P, j, done, rain, rain, rain_next);
         }
-        if (n - k >= 2) {
-            const PairVariant &tv = kQuadTails[rule == 4][n - k - 2];
-            const double rain_next = last ? 0.0 : rain;
-            hipLaunchKernelGGL(tv.fn, dim3((unsigned)tgrid), dim3(tv.threads), 0, stream, b.meta,
-                               b.hw[0], b.hw[1], b.s[0], b.s[1], P, j, rain, rain_next);
-            k = n;
-            ++j;
-        }
-    } else if (plan) {
-        const TilePlanDev P = plan_dev(*plan);
-        const int64_t tgrid = ((P.ntiles + 7) / 8) * 8;
-        for (; k + 2 <= n; k += 2, ++j) {
-            const double rain_next = (last && k + 2 == n) ? 0.0 : rain;
-            const PairVariant &pv = rule == 4 ? kPairRule4 : kPairVariants[variant];
-            hipLaunchKernelGGL(pv.fn, dim3((unsigned)tgrid), dim3(pv.threads), 0, stream, b.meta,
-                               b.hw[0], b.hw[1], b.s[0], b.s[1], P, j, rain, rain_next);
-        }
+        k += steps;
     }
-    for (; k < n; ++k, ++j) {
-        const double rain_next = (last && k + 1 == n) ? 0.0 : rain;
-        hipLaunchKernelGGL(rule == 4 ? k_erode_step<4> : k_erode_step<3>, dim3((unsigned)grid),
-                           dim3(256), 0, stream, b.meta, b.hw[0], b.hw[1], b.s[0], b.s[1], V, col,
-                           elen, nblocks, j, rain_next);
-    }
-    hipLaunchKernelGGL(k_advance, dim3(1), dim3(1), 0, stream, b.meta, (int64_t)n, j);
+    if (launches == 1)
+        hipLaunchKernelGGL(k_advance, dim3(1), dim3(1), 0, stream, b.meta, (int64_t)n, 1);
 }
 
-// Everything a captured launch takes from the plan by value (TilePlanDev:
-// the blob address, the section offsets, the tile count) plus the kernel
-// variant and rule, folded into one 64-bit tag (FNV-1a).  Two plans that
-// differ in any of these get different graphs even when a later plan's
-// image lands at a freed plan's address.
-static uint64_t plan_tag(const nx_tile_plan *plan, int variant, int rule)
-{
-    uint64_t h = 1469598103934665603ull;
-    auto mix = [&h](uint64_t v) {
-        for (int k = 0; k < 8; ++k) {
-            h ^= (v >> (8 * k)) & 0xff;
-            h *= 1099511628211ull;
-        }
-    };
-    mix((uint64_t)rule);
-    mix((uint64_t)variant);
-    if (plan) {
-        mix((uint64_t)(uintptr_t)plan->blob);
-        const int64_t f[] = {plan->bytes,   plan->V,        plan->ntiles,    plan->max_tile,
-                             plan->max_load, plan->off_start, plan->off_cs,   plan->off_load,
-                             plan->off_rbase, plan->off_ring, plan->off_cbase, plan->off_lcol,
-                             plan->off_lel,  plan->steps,    plan->max_step1, plan->off_pref,
-                             plan->off_ebase};
-        for (int64_t v : f) mix((uint64_t)v);
-    }
-    return h;
-}
-
-// Captured chunk of steps, cached per (workspace, graph, plan contents,
-// length, rain, last).  Replays stay correct because every launch reads the
+// Captured chunk of one-step launches, cached per (workspace, graph, length,
+// rain, last, rule).  Replays stay correct because every launch reads the
 // step counter and current buffer from the workspace rather than from its
 // arguments.  No memset is recorded into the graph.
 static int chunk_graph(nx_ctx *ctx, const ErosionBufs &b, void *state, int64_t V,
-                       const int32_t *col, const double *elen, const nx_tile_plan *plan, int rule,
-                       int n, double rain, bool last, hipGraphExec_t *out)
+                       const int32_t *col, const double *elen, int rule, int n, double rain,
+                       bool last, hipGraphExec_t *out)
 {
-    const int variant =
-        plan ? (plan->steps == kMultiSteps ? 8 + ctx->multi_variant : ctx->pair_variant) : -1;
-    GraphKey key{state, V, col, elen, n, rain, last, plan_tag(plan, variant, rule)};
+    GraphKey key{state, V, col, elen, n, rain, last, (uint64_t)rule};
     std::lock_guard<std::mutex> lk(ctx->mu);
     auto it = ctx->graphs.find(key);
     if (it != ctx->graphs.end()) {
@@ -409,8 +406,7 @@ static int chunk_graph(nx_ctx *ctx, const ErosionBufs &b, void *state, int64_t V
     ctx->make_room_for_graph();
     hipGraph_t g = nullptr;
     NX_HIP(hipStreamBeginCapture(ctx->capture_stream, hipStreamCaptureModeThreadLocal));
-    launch_steps(b, V, col, elen, plan, ctx->pair_variant, ctx->multi_variant, rule, n, rain, last,
-                 ctx->capture_stream);
+    launch_steps(b, V, col, elen, nullptr, 0, 0, rule, n, rain, false, last, ctx->capture_stream);
     const hipError_t le = hipGetLastError();
     const hipError_t ce = hipStreamEndCapture(ctx->capture_stream, &g);
     if (le != hipSuccess || ce != hipSuccess) {
@@ -471,24 +467,27 @@ int erosion_run_rule(nx_ctx *ctx, void *state, int64_t V, const int32_t *col, co
     if (iters == 0) return NX_OK;
     NX_HIP(hipSetDevice(ctx->device));
     ErosionBufs b = bufs(state, V);
-    const int64_t nblocks = (V + 255) / 256;
-    if (rain != 0.0)
-        hipLaunchKernelGGL(k_add_rain, dim3((unsigned)nblocks), dim3(256), 0, stream, b.meta,
-                           b.hw[0], b.hw[1], V, rain);
-    const int chunk = ctx->graph_chunk;
+    // Runs over a plan launch eagerly: a launch takes 8 us or more, submitting
+    // it about 4, and a captured chunk of 32 steps adds 3 to 60 us of its own
+    // (64 to 1000 divisions: 2.0 against 2.1 us per step, 79.8 against 81.8)
+    // after a capture for each new workspace.
+    const int chunk = plan ? 0 : ctx->graph_chunk;
     if (chunk <= 0 || iters < 2) {
         launch_steps(b, V, col, elen, plan, ctx->pair_variant, ctx->multi_variant, rule, iters, rain,
-                     true, stream);
+                     true, true, stream);
         NX_HIP(hipGetLastError());
         return NX_OK;
     }
+    if (rain != 0.0)
+        hipLaunchKernelGGL(k_add_rain, dim3((unsigned)((V + 255) / 256)), dim3(256), 0, stream,
+                           b.meta, b.hw[0], b.hw[1], V, rain);
     // Full chunks, then the remainder; the final piece does not pre-add rain.
     int done = 0;
     while (done < iters) {
         const int n = std::min(chunk, iters - done);
         const bool last = done + n == iters;
         hipGraphExec_t ex = nullptr;
-        rc = chunk_graph(ctx, b, state, V, col, elen, plan, rule, n, rain, last, &ex);
+        rc = chunk_graph(ctx, b, state, V, col, elen, rule, n, rain, last, &ex);
         if (rc) return rc;
         NX_HIP(hipGraphLaunch(ex, stream));
         done += n;

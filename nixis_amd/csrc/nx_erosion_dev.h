@@ -36,7 +36,7 @@ namespace nx {
 struct ErosionMeta {
     int64_t it;           // steps taken so far
     int32_t buf;          // which of the two buffers holds the current fields
-    int32_t pad;
+    int32_t base;         // buf when the run now on the stream began
 };
 
 // erosion.py:205-207

@@ -35,6 +35,24 @@ constexpr int kLoadMaxMulti = 3072; // tile + its kMultiSteps rings
 constexpr int kQuadStepOne = 2048;
 constexpr int kQuadLoadMax = 2688;
 constexpr int kQuadChunk = 1152;
+// Default chunk of a four-step plan over V vertices.  A launch takes as long
+// as its fullest CU: up to about two tiles per CU of kCus, the tiles are made
+// equal in size and just enough to go round the CUs once, or twice (2% over,
+// for the shorter last one), which measured faster than fewer, full tiles at
+// 64 to 200 divisions (us per step: 41k vertices 2.0 against 3.4, 100k 2.5
+// against 3.4, 225k 3.4 against 3.5, 400k 5.0 against 5.5); beyond two rounds
+// of two tiles per CU full tiles win (1000 divisions: 79.8, 81.6 at 1024, 101
+// at 512).  Below kQuadSmall the rings outgrow the tiles.
+constexpr int kCus = 256;
+constexpr int kQuadSmall = 256;
+inline int quad_chunk(int64_t V)
+{
+    for (int64_t round : {kCus, 2 * kCus, 4 * kCus}) {
+        const int64_t chunk = (V + round - 1) / round * 51 / 50;
+        if (chunk <= kQuadChunk) return chunk < kQuadSmall ? kQuadSmall : (int)chunk;
+    }
+    return kQuadChunk;
+}
 
 // Device view of a plan image (pointers into nx_tile_plan::blob).
 struct TilePlanDev {
@@ -341,12 +359,14 @@ __device__ __forceinline__ void erode_tile_multi(double2 *A, double2 *hw0, doubl
 // theirs.  NS = 3 or 2 runs the last three or two of those steps (a run's
 // tail of steps that does not fill a four-step launch): the first step then
 // covers tile + rings 1..2 or tile + ring 1, and only the vertices it reads
-// are staged.
-template <int RULE = 3, int NS = 4>
+// are staged.  FIRST adds rain_first to the water as it is staged (the first
+// rain of a run, erosion.py:182).
+template <int RULE = 3, int NS = 4, bool FIRST = false>
 __device__ __forceinline__ void erode_tile_quad(double2 *A, double2 *B, double2 *hw0, double2 *hw1,
                                                 double *s0, double *s1, int p,
                                                 const TilePlanDev &P, int64_t tile,
-                                                double rain_mid, double rain_next)
+                                                double rain_mid, double rain_next,
+                                                double rain_first = 0.0)
 {
     constexpr int TH = 1024;
     constexpr int kPer = kQuadStepOne / TH;
@@ -368,8 +388,11 @@ __device__ __forceinline__ void erode_tile_quad(double2 *A, double2 *B, double2 
     const auto lcol = gmem(P.lcol) + 6 * cb;
     const auto lel = gmem(P.lel) + gmem(P.ebase)[tile];
 
-    for (int li = threadIdx.x; li < cl; li += TH)
-        A[li] = hw_src[li < T ? a + li : ring[li - T]];
+    for (int li = threadIdx.x; li < cl; li += TH) {
+        double2 v = hw_src[li < T ? a + li : ring[li - T]];
+        if (FIRST) v.y = v.y + rain_first;
+        A[li] = v;
+    }
     double sed[kPer];
     int code[kPer][6];
 #pragma unroll

@@ -14,7 +14,8 @@
 // A tile takes about 20 synchronous steps to collect and number and 40 to
 // settle its owners, so the kernels are bound by barriers and LDS latency, two
 // tiles to a CU.  Neighbour tables, order and plan of a new mesh of 316,842
-// vertices: 178 ms with the host planner, 0.99 ms so.  A table that is not symmetric is left to the host planner.
+// vertices: 178 ms with the host planner, 0.99 ms so.  A table that is not
+// symmetric is left to the host planner.
 #include <hip/hip_runtime.h>
 
 #include <cstring>
@@ -587,7 +588,7 @@ __global__ __launch_bounds__(kThreads) void k_plan_write(
 size_t tile_plan_device_workspace_bytes(int64_t V, int chunk)
 {
     if (V <= 0 || V > INT32_MAX || chunk < 0 || (chunk != 0 && chunk < kTileMin)) return 256;
-    return plan_scratch(V, chunk ? chunk : kQuadChunk).total;
+    return plan_scratch(V, chunk ? chunk : quad_chunk(V)).total;
 }
 
 int tile_plan_build_device(nx_ctx *ctx, const int32_t *col, const double *elen, int64_t V,
@@ -601,7 +602,7 @@ int tile_plan_build_device(nx_ctx *ctx, const int32_t *col, const double *elen, 
         return set_error(NX_EINVAL, "tile chunk %d outside %d..%d (0 for the default)", chunk_in,
                          kTileMin, kQuadStepOne);
     NX_HIP(hipSetDevice(ctx->device));
-    const int64_t chunk = chunk_in ? chunk_in : kQuadChunk;
+    const int64_t chunk = chunk_in ? chunk_in : quad_chunk(V);
     const PlanScratch L = plan_scratch(V, chunk);
     char *w = (char *)ws;
     auto *totals = (PlanTotals *)(w + L.totals);

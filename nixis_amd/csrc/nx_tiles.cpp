@@ -6,7 +6,7 @@
 // the fields of the tile and K rings (erosion.py:197-279 reads only the
 // one-ring of each vertex): step j runs on the tile and rings 1..K-j.  Tiles
 // start at `chunk` vertices (by default kPairChunk for two steps,
-// kQuadChunk for four; an autotuner may pick another per mesh size) and are
+// quad_chunk for four; an autotuner may pick another per mesh size) and are
 // halved until tile + rings fit the kernel's load limit and the first step's
 // vertices (tile + rings 1..K-1) its step-one limit (kStepOneMax, or
 // kQuadStepOne for four steps); a space-filling-curve order (compact tiles,
@@ -277,7 +277,7 @@ int tile_plan_build(const int32_t *col, const double *elen, int64_t V, int K, vo
                          kTileMin, tile_max);
     const int limit = K == 2 ? kLoadMax : kQuadLoadMax;
     const int step1_limit = K == 2 ? kStepOneMax : kQuadStepOne;
-    const int64_t chunk = chunk_in ? chunk_in : (K == 2 ? kPairChunk : kQuadChunk);
+    const int64_t chunk = chunk_in ? chunk_in : (K == 2 ? kPairChunk : quad_chunk(V));
     for (int64_t i = 0; i < 6 * V; ++i)
         if (col[i] < 0 || col[i] >= V) return set_error(NX_EINVAL, "col[%lld] = %d outside 0..V-1", (long long)i, col[i]);
 
