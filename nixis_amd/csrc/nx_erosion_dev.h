@@ -69,6 +69,33 @@ NX_EHD void erode_accumulate(double h, double hn, double wn, double d, double &S
     }
 }
 
+// Heights of at least this size: a neighbour's height then differs by 0 or by
+// 2^-993 and more (both are multiples of the smaller one's last place), so the
+// slope has the difference's sign and comparing the heights gives it.
+constexpr double kCompare = 0x1p-940;
+
+// erode_accumulate for |h| >= kCompare: the products take the difference's
+// sign (S - t is S + -t, and -w k is -(w k)), so one comparison and two sums
+// serve both directions.
+template <int RULE = 3>
+NX_EHD void erode_compare(double h, double hn, double wn, double d, double &S, double &W)
+{
+    const uint64_t down = __builtin_bit_cast(uint64_t, hn - h) & 0x8000000000000000ull;
+    double ts, tw;
+    if (RULE == 4) {
+        ts = __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, max0(kSol * wn)) ^ down);
+        tw = __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, max0(wn * d)) ^ down);
+    } else {
+        const double w = __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, wn) ^ down);
+        ts = kSol * w;
+        tw = w * d;
+    }
+    if (hn < h || hn > h) {   // neither for a tie or a NaN
+        S += ts;
+        W += tw;
+    }
+}
+
 // Finish the vertex; `rain` (0 for none) is the next iteration's rainfall,
 // added to the new water as the reference's water += rain would.
 template <int RULE = 3>

@@ -33,6 +33,7 @@ constexpr int kLoadMaxMulti = 3072; // tile + its kMultiSteps rings
 // 1..4 within kQuadLoadMax, so that both LDS buffers of erode_tile_quad fit
 // two blocks per CU; they start from tiles of kQuadChunk vertices.
 constexpr int kQuadStepOne = 2048;
+static_assert(16 * 2688 <= 65536, "a staged vertex's byte offset fits 16 bits");
 constexpr int kQuadLoadMax = 2688;
 constexpr int kQuadChunk = 1152;
 // Default chunk of a four-step plan over V vertices.  A launch takes as long
@@ -349,7 +350,7 @@ __device__ __forceinline__ void erode_tile_multi(double2 *A, double2 *hw0, doubl
 // Four steps of tile `tile` (a four-step plan within kQuadStepOne and
 // kQuadLoadMax) by a 1024-thread block, reading buffer p and writing p ^ 1.
 // Each thread keeps up to two first-step vertices (li and li + 1024): their
-// sediment, neighbour indices (two to a word) and edge lengths are loaded
+// sediment, neighbours (LDS byte offsets, two to a word) and edge lengths are loaded
 // before the first barrier, while the field gathers are in flight, and stay
 // in registers for all four steps.  h and w of the tile and its four rings
 // are staged in A; step 1 (tile + rings 1..3) writes B, step 2 (tile + rings
@@ -417,8 +418,8 @@ __device__ __forceinline__ void erode_tile_quad(double2 *A, double2 *B, double2 
             for (int q = 0; q < 6; ++q) len[m][q] = slot_len(code[m][q], li, c1, T, lel);
 #pragma unroll
             for (int q = 0; q < 3; ++q)
-                nbp[m][q] = (uint32_t)slot_nbr(code[m][2 * q]) |
-                            (uint32_t)slot_nbr(code[m][2 * q + 1]) << 16;
+                nbp[m][q] = (uint32_t)slot_nbr(code[m][2 * q]) << 4 |
+                            (uint32_t)slot_nbr(code[m][2 * q + 1]) << 20;
         }
     }
     __syncthreads();
@@ -431,11 +432,26 @@ __device__ __forceinline__ void erode_tile_quad(double2 *A, double2 *B, double2 
             if (li < n) {
                 const double2 me = src[li];
                 double S = sed[m], W = me.y;
+                auto nb = [&](int q) {
+                    const uint32_t at = q & 1 ? nbp[m][q >> 1] >> 16 : nbp[m][q >> 1] & 0xffffu;
+                    return *(const double2 *)((const char *)src + at);
+                };
+                if (fabs(me.x) >= kCompare) {
+                    // the next neighbour's read is in flight during an update
+                    double2 v = nb(0);
 #pragma unroll
-                for (int q = 0; q < 6; ++q) {
-                    const int nb_i = (int)((nbp[m][q >> 1] >> (16 * (q & 1))) & 0xffffu);
-                    const double2 nb = src[nb_i];
-                    erode_accumulate<RULE>(me.x, nb.x, nb.y, len[m][q], S, W);
+                    for (int q = 0; q < 6; ++q) {
+                        const double2 next = nb(q < 5 ? q + 1 : 5);
+                        asm volatile("" ::: "memory");
+                        erode_compare<RULE>(me.x, v.x, v.y, len[m][q], S, W);
+                        v = next;
+                    }
+                } else {
+#pragma unroll
+                    for (int q = 0; q < 6; ++q) {
+                        const double2 v = nb(q);
+                        erode_accumulate<RULE>(me.x, v.x, v.y, len[m][q], S, W);
+                    }
                 }
                 double ho, wo, so;
                 erode_finish<RULE>(me.x, me.y, sed[m], S, W, rain, ho, wo, so);

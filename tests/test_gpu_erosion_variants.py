@@ -108,3 +108,53 @@ def test_v4_full_size_tiled_equals_single_steps():
     for x, y in zip(a, b):
         assert np.array_equal(x, y)
     assert np.isfinite(a[0]).all() and (a[1] >= 0).all()
+
+
+def _edge_heights(kind, h, rng):
+    if kind == "ties":                   # many neighbours at equal heights
+        return np.round(h / 3000.0)
+    if kind == "edge":                   # magnitudes on both sides of 2^-940
+        return np.sign(h) * 2.0 ** rng.uniform(-944, -936, h.size)
+    if kind == "tiny":                   # differences whose slope can underflow
+        return h / 9000.0 * 2.0 ** -1062
+    if kind == "zeros":
+        return np.where(rng.uniform(size=h.size) < 0.5, 0.0, h) * np.where(h < 0, -1.0, 1.0)
+    h = h.copy()
+    h[rng.integers(0, h.size, 20)] = rng.choice([np.nan, np.inf, -np.inf, 1e308, -1e308], 20)
+    return h
+
+
+@pytest.mark.parametrize("radius", [1.0, 6378100.0])
+@pytest.mark.parametrize("kind", ["ties", "edge", "tiny", "zeros", "special"])
+@pytest.mark.parametrize("rule", [3, 4])
+def test_slot_update_at_the_comparison_edges(oracle, rule, kind, radius):
+    """Four-step launches and their tails, where heights tie, are zero, are so
+    small that a slope underflows, straddle the size from which heights are
+    compared directly, or are not finite: finite values and infinities bit for
+    bit, NaN where the oracle has NaN."""
+    rng = np.random.default_rng(8)
+    pts, nb, h = _planet(26)
+    pts = pts * radius
+    h = _edge_heights(kind, h, rng)
+    w = rng.uniform(-0.5, 1.0, h.size)
+    s = rng.uniform(-0.01, 0.02, h.size)
+    g = erosion.ErosionGraph(pts, nb)
+    assert g.plan is not None and g.plan.steps == 4
+    for n, rain in ((2, 0.0), (3, 0.5), (4, 0.0), (6, 0.3 / 320)):
+        st = erosion.ErosionState(g.V)
+        st.load(*[torch.from_numpy(g.permute(a)).cuda() for a in (h, w, s)])
+        st.run(g, n, rain, rule=rule)
+        out = [torch.empty(g.V, dtype=torch.float64, device="cuda") for _ in range(3)]
+        st.store(*out)
+        st.ctx.sync_check()
+        ref = [h.copy(), w.copy(), s.copy()]
+        step = oracle.erosion_iteration3 if rule == 3 else oracle.erosion_iteration4
+        for _ in range(n):
+            if rain:
+                ref[1] += rain
+            step(pts, nb, *ref)
+        for t, r in zip(out, ref):
+            a = g.unpermute(t.cpu().numpy())
+            nan = np.isnan(r)
+            assert np.array_equal(nan, np.isnan(a))
+            assert np.array_equal(a[~nan].view(np.int64), r[~nan].view(np.int64))
