@@ -108,7 +108,7 @@ int power_rescale(nx_ctx *ctx, const double *x, const uint8_t *mask, int64_t n, 
 int sample_octaves_keys(nx_ctx *ctx, const double *verts, int64_t V, const int32_t *perm,
                         const int32_t *pgi, int n_oct, const double *rough,
                         const double *strength, double radius, double *elev, int accumulate,
-                        float *dbg_noise, int32_t *dbg_sel, unsigned long long *keys,
+                        float *dbg_noise, int32_t *dbg_sel, unsigned long long *rec, int *nrec,
                         hipStream_t stream);
 int terrain_heights(nx_ctx *ctx, const double *verts, int64_t V, const int32_t *perm,
                     const int32_t *pgi, int n_oct, const double *rough, const double *strength,

@@ -26,8 +26,9 @@ struct OctaveArgs {
     int accumulate;
 };
 
-// keys (nullable): order-preserving min/max keys of the elevations written,
-// reduced here so a rescale after noise needs no pass of its own.
+// rec (nullable): order-preserving min/max keys of the elevations a block
+// writes, one pair per block, so a rescale after noise needs no pass of its
+// own.
 template <bool DBG>
 __device__ __forceinline__ void sample_octaves_body(const OctaveArgs &a,
                                                     const double *__restrict__ verts, int64_t V,
@@ -35,7 +36,7 @@ __device__ __forceinline__ void sample_octaves_body(const OctaveArgs &a,
                                                     float *__restrict__ dbg_noise,
                                                     int32_t *__restrict__ dbg_sel,
                                                     int *__restrict__ err,
-                                                    unsigned long long *__restrict__ keys)
+                                                    unsigned long long *__restrict__ rec)
 {
     unsigned long long lo = ~0ull, hi = 0ull;
     __shared__ NoiseTables T;
@@ -57,18 +58,18 @@ __device__ __forceinline__ void sample_octaves_body(const OctaveArgs &a,
             }
         });
         elev[i] = acc;
-        if (keys) {
+        if (rec) {
             const unsigned long long k = dkey(acc);
             lo = k < lo ? k : lo;
             hi = k > hi ? k : hi;
         }
     }
     if (bad) __hip_atomic_fetch_or(err, NX_ERR_RANGE_BIT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (keys) {
+    if (rec) {
         block_minmax(lo, hi);
         if (threadIdx.x == 0) {
-            __hip_atomic_fetch_min(&keys[0], lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_fetch_max(&keys[1], hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            rec[2 * blockIdx.x] = lo;
+            rec[2 * blockIdx.x + 1] = hi;
         }
     }
 }
@@ -77,9 +78,9 @@ __device__ __forceinline__ void sample_octaves_body(const OctaveArgs &a,
 // keeps enough waves in flight to cover the dependent LDS hash lookups.
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_sample_octaves(
     OctaveArgs a, const double *__restrict__ verts, int64_t V, double *__restrict__ elev,
-    int *__restrict__ err, unsigned long long *__restrict__ keys)
+    int *__restrict__ err, unsigned long long *__restrict__ rec)
 {
-    sample_octaves_body<false>(a, verts, V, elev, nullptr, nullptr, err, keys);
+    sample_octaves_body<false>(a, verts, V, elev, nullptr, nullptr, err, rec);
 }
 
 // Debug launch: per-octave noise values and selection records.
@@ -178,13 +179,13 @@ int sample_octaves(nx_ctx *ctx, const double *verts, int64_t V, const int32_t *p
                    int32_t *dbg_sel, hipStream_t stream)
 {
     return sample_octaves_keys(ctx, verts, V, perm, pgi, n_oct, rough, strength, radius, elev,
-                               accumulate, dbg_noise, dbg_sel, nullptr, stream);
+                               accumulate, dbg_noise, dbg_sel, nullptr, nullptr, stream);
 }
 
 int sample_octaves_keys(nx_ctx *ctx, const double *verts, int64_t V, const int32_t *perm,
                         const int32_t *pgi, int n_oct, const double *rough,
                         const double *strength, double radius, double *elev, int accumulate,
-                        float *dbg_noise, int32_t *dbg_sel, unsigned long long *keys,
+                        float *dbg_noise, int32_t *dbg_sel, unsigned long long *rec, int *nrec,
                         hipStream_t stream)
 {
     if (!ctx) return set_error(NX_EINVAL, "null context");
@@ -202,13 +203,17 @@ int sample_octaves_keys(nx_ctx *ctx, const double *verts, int64_t V, const int32
     if (V == 0) return NX_OK;
     NX_HIP(hipSetDevice(ctx->device));
     const int grid = grid_for(ctx, V, 8);
+    if (rec) {   // one pair per block, at most *nrec
+        if (grid > *nrec) return set_error(NX_EINVAL, "%d blocks for %d min/max records", grid, *nrec);
+        *nrec = grid;
+    }
     if (dbg_noise || dbg_sel) {
-        if (keys) return set_error(NX_EINVAL, "min/max keys are not reduced with debug output");
+        if (rec) return set_error(NX_EINVAL, "min/max keys are not reduced with debug output");
         hipLaunchKernelGGL(k_sample_octaves_dbg, dim3(grid), dim3(256), 0, stream, a, verts, V,
                            elev, dbg_noise, dbg_sel, ctx->d_err);
     } else {
         hipLaunchKernelGGL(k_sample_octaves, dim3(grid), dim3(256), 0, stream, a, verts, V, elev,
-                           ctx->d_err, keys);
+                           ctx->d_err, rec);
     }
     NX_HIP(hipGetLastError());
     return NX_OK;

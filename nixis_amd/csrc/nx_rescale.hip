@@ -56,8 +56,10 @@ __global__ void k_minmax_init(unsigned long long *keys)
 // (four slices of 128, lane l holding values 2l and 2l + 1 of each, so every
 // load instruction covers one contiguous range) with the next chunk's loads
 // in flight while it reduces the current one.  vec: x is 16-byte aligned.
+// keys null: the block's pair goes to rec instead (joined by k_pr_summary).
 __global__ __launch_bounds__(kMinmaxThreads) void k_minmax(const double *__restrict__ x, int64_t n,
-                                                unsigned long long *__restrict__ keys, int vec)
+                                                unsigned long long *__restrict__ keys, int vec,
+                                                unsigned long long *__restrict__ rec)
 {
     unsigned long long lo = ~0ull, hi = 0ull;
     auto upd = [&](double v) {
@@ -102,9 +104,12 @@ __global__ __launch_bounds__(kMinmaxThreads) void k_minmax(const double *__restr
             if (off(j) < left) upd(v[j]);
     }
     block_minmax(lo, hi);
-    if (threadIdx.x == 0) {
+    if (threadIdx.x == 0 && keys) {
         __hip_atomic_fetch_min(&keys[0], lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __hip_atomic_fetch_max(&keys[1], hi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    } else if (threadIdx.x == 0) {
+        rec[2 * blockIdx.x] = lo;
+        rec[2 * blockIdx.x + 1] = hi;
     }
 }
 
@@ -168,7 +173,8 @@ int rescale(nx_ctx *ctx, const double *x, int64_t n, double lower, double upper,
     unsigned long long *keys = ctx->d_keys + 2 * (ctx->key_slot.fetch_add(1) % kKeySlots);
     const unsigned grid = (unsigned)std::min<int64_t>((n + 255) / 256, (int64_t)ctx->num_cus * 8);
     hipLaunchKernelGGL(k_minmax_init, dim3(1), dim3(64), 0, stream, keys);
-    hipLaunchKernelGGL(k_minmax, dim3(mm_grid(ctx, n)), dim3(kMinmaxThreads), 0, stream, x, n, keys, vec16(x));
+    hipLaunchKernelGGL(k_minmax, dim3(mm_grid(ctx, n)), dim3(kMinmaxThreads), 0, stream, x, n, keys, vec16(x),
+                       (unsigned long long *)nullptr);
     hipLaunchKernelGGL(k_rescale_map, dim3(grid), dim3(256), 0, stream, x, n, keys, lower, upper,
                        out, minmax, ctx->d_err, vec16(x) & vec16(out));
     NX_HIP(hipGetLastError());
@@ -259,7 +265,8 @@ static int rescale_ex_launch(nx_ctx *ctx, const double *x, int64_t n, const Resc
     unsigned long long *keys = key_slot(ctx);
     const unsigned grid = red_grid(ctx, n);
     hipLaunchKernelGGL(k_minmax_init, dim3(1), dim3(64), 0, stream, keys);
-    hipLaunchKernelGGL(k_minmax, dim3(mm_grid(ctx, n)), dim3(kMinmaxThreads), 0, stream, x, n, keys, vec16(x));
+    hipLaunchKernelGGL(k_minmax, dim3(mm_grid(ctx, n)), dim3(kMinmaxThreads), 0, stream, x, n, keys, vec16(x),
+                       (unsigned long long *)nullptr);
     hipLaunchKernelGGL(k_rescale_ex, dim3(grid), dim3(256), 0, stream, x, n, keys, a, out,
                        minmax, ctx->d_err, vec16(x) & vec16(out), (const int32_t *)nullptr);
     NX_HIP(hipGetLastError());
@@ -651,14 +658,22 @@ __device__ __forceinline__ PSum wave_run_summary(const WaveRun &R, double mn, do
 // its own suf) joined with the max of every later run; without one, last is
 // the last non-empty run's.  A lane scan finds each run's predecessor,
 // ballots the first break and the first and last runs.
+// The block is two groups of NT threads, one for each half's runs; every
+// thread gets its group's result.
 template <int NT>
 __device__ PSum psum_join_block(const PSum &P)
 {
     constexpr int NW = NT / 64;
-    __shared__ double s_last[NW], s_mn[NW], s_mx[NW], s_sf[NW];
-    __shared__ int s_has[NW], s_k[NW], s_f[NW], s_l[NW];
-    __shared__ double s_first, s_lastv;
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    struct Join {
+        double last[NW], mn[NW], mx[NW], sf[NW], first, lastv;
+        int has[NW], k[NW], f[NW], l[NW];
+    };
+    __shared__ Join joins[2];
+    Join &J = joins[threadIdx.x / NT];
+    auto &s_last = J.last, &s_mn = J.mn, &s_mx = J.mx, &s_sf = J.sf;
+    auto &s_has = J.has, &s_k = J.k, &s_f = J.f, &s_l = J.l;
+    auto &s_first = J.first, &s_lastv = J.lastv;
+    const int t = threadIdx.x % NT, lane = t & 63, w = t >> 6;
     const int ne = P.ne;
     // inclusive scan over the wave: the last value of the latest non-empty run
     double pv = P.last;
@@ -741,23 +756,23 @@ __device__ PSum psum_join_block(const PSum &P)
 }
 
 // In-order reduction of the nsum pairs of block summaries sum[2c], sum[2c+1]
-// by one block of NT threads: each thread joins a run of ceil(nsum / NT)
-// consecutive pairs, then the block joins the threads' results in parallel;
-// the results are valid in every thread.
+// by one block of 2 NT threads: the first NT threads join the pairs' first
+// halves, the others the second, each a run of ceil(nsum / NT) consecutive
+// ones, then each group joins its threads' results in parallel (one after the
+// other by the whole block took 13 us instead of 7.5); s[0] and s[1] (in
+// LDS) are valid in every thread afterwards.
 template <int NT>
-__device__ void pr_reduce_sums(const PSum *sum, int64_t nsum, PSum &s0, PSum &s1)
+__device__ void pr_reduce_sums(const PSum *sum, int64_t nsum, PSum *s)
 {
+    const int half = threadIdx.x / NT, t = threadIdx.x % NT;
     const int64_t per = (nsum + NT - 1) / NT;
-    const int64_t c0 = (int64_t)threadIdx.x * per;
+    const int64_t c0 = (int64_t)t * per;
     const int64_t c1 = c0 + per < nsum ? c0 + per : nsum;
-    s0 = psum_empty();
-    s1 = psum_empty();
-    for (int64_t c = c0; c < c1; ++c) {
-        s0 = psum_join(s0, sum[2 * c]);
-        s1 = psum_join(s1, sum[2 * c + 1]);
-    }
-    s0 = psum_join_block<NT>(s0);
-    s1 = psum_join_block<NT>(s1);
+    PSum r = psum_empty();
+    for (int64_t c = c0; c < c1; ++c) r = psum_join(r, sum[2 * c + half]);
+    r = psum_join_block<NT>(r);
+    if (t == 0) s[half] = r;
+    __syncthreads();
 }
 
 // Summaries of the values whose mask is unset (sum[2b]) and set (sum[2b + 1])
@@ -773,7 +788,9 @@ __device__ void pr_reduce_sums(const PSum *sum, int64_t nsum, PSum &s0, PSum &s1
 // inside one region see a single half for all of it, and every wave must
 // stream at the same rate.  The eight waves join in order.
 // CHAIN: x holds the noise heights; each value is the standard rescale
-// (util.py:139) with min/max from head->keys0, the rescaled min/max and the
+// (util.py:139) with min/max joined from the nrec block records rec (closing
+// atomics of 2,048 noise blocks on two keys took about 28 us) and left in
+// head->keys0 by block 0; the rescaled min/max and the
 // ocean level are derived from the same keys (the map is monotone, so its
 // extremes are the images of x's), and mask = t <= level (terrain.py:61-72);
 // WRITE: t and the mask are written back.  vec: x is 16-byte and mask
@@ -783,13 +800,34 @@ __global__ __launch_bounds__(kPrThreads) void k_pr_summary(double *x, uint8_t *m
                                                            int64_t nunits, int64_t cpw, int vec,
                                                            PSum *__restrict__ sum,
                                                            PrHead *__restrict__ head, ChainArgs ca,
-                                                           int *__restrict__ err)
+                                                           int *__restrict__ err,
+                                                           const unsigned long long *__restrict__ rec,
+                                                           int nrec)
 {
     __shared__ PSum lds[2][kPrThreads / 64];
     double x_min = 0.0, xr = 1.0, nr = 0.0, level = 0.0;
     if (CHAIN) {
-        x_min = dunkey(head->keys0[0]);
-        const double x_max = dunkey(head->keys0[1]);
+        __shared__ unsigned long long keys[2];
+        unsigned long long lo = ~0ull, hi = 0ull;
+        for (int i = threadIdx.x; i < nrec; i += kPrThreads) {
+            const unsigned long long a = rec[2 * i], b = rec[2 * i + 1];
+            lo = a < lo ? a : lo;
+            hi = b > hi ? b : hi;
+        }
+        block_minmax(lo, hi);
+        if (threadIdx.x == 0) {
+            keys[0] = lo;
+            keys[1] = hi;
+            if (blockIdx.x == 0) {
+                head->keys0[0] = lo;
+                head->keys0[1] = hi;
+                head->keys1[0] = head->keys2[0] = ~0ull;   // for the later passes' reductions
+                head->keys1[1] = head->keys2[1] = 0ull;
+            }
+        }
+        __syncthreads();
+        x_min = dunkey(keys[0]);
+        const double x_max = dunkey(keys[1]);
         xr = x_max - x_min;
         nr = ca.upper - ca.lower;
         const double fa = ((x_min - x_min) / xr) * nr + ca.lower;
@@ -943,35 +981,38 @@ __global__ __launch_bounds__(kPrThreads) void k_pr_summary(double *x, uint8_t *m
     }
 }
 
+// The two-pass chain's constants into head (one thread).
+__device__ void chain_publish(PrHead *head, const PSum *s, const ChainConsts &cc)
+{
+    head->s[0] = s[0];
+    head->s[1] = s[1];
+    head->lo1 = cc.lo1;
+    head->r1 = cc.r1;
+    head->lo0 = cc.lo0;
+    head->r0 = cc.r0;
+    head->h4min = cc.h4min;
+    head->h4max = cc.h4max;
+    head->fast = cc.fast;
+}
+
 // One block: in-order reduction of the per-block summaries into head->s;
 // from_keys: head->xmin/xmax = (min, max) of x from head->keys0; chain: the
-// two-pass height chain's constants (chain_derive) into head, and the
-// five-pass kernels' reduction keys reset for the case they run.
+// two-pass height chain's constants (chain_derive) into head.
 __global__ __launch_bounds__(1024) void k_pr_finish(const PSum *__restrict__ sum, int64_t nsum,
                                                     PrHead *__restrict__ head, int from_keys,
                                                     int chain)
 {
-    PSum s0, s1;
-    pr_reduce_sums<1024>(sum, nsum, s0, s1);
+    __shared__ PSum s[2];
+    pr_reduce_sums<512>(sum, nsum, s);
     if (threadIdx.x == 0) {
-        head->s[0] = s0;
-        head->s[1] = s1;
+        head->s[0] = s[0];
+        head->s[1] = s[1];
         if (from_keys) {
             head->xmin = dunkey(head->keys0[0]);
             head->xmax = dunkey(head->keys0[1]);
         }
-        if (chain) {
-            const ChainConsts cc = chain_derive(s1, s0, head->xmin, head->xmax, head->level);
-            head->lo1 = cc.lo1;
-            head->r1 = cc.r1;
-            head->lo0 = cc.lo0;
-            head->r0 = cc.r0;
-            head->h4min = cc.h4min;
-            head->h4max = cc.h4max;
-            head->fast = cc.fast;
-            head->keys1[0] = head->keys2[0] = ~0ull;
-            head->keys1[1] = head->keys2[1] = 0ull;
-        }
+        if (chain)
+            chain_publish(head, s, chain_derive(s[1], s[0], head->xmin, head->xmax, head->level));
     }
 }
 
@@ -1054,24 +1095,58 @@ __global__ __launch_bounds__(256) void k_pr_map(const double *x, double *out,
 // shift by the level and the split rescale around 0 with the shifted
 // heights' min/max.  Heights and mask are written once.  Every operation is
 // the one the five-pass kernels apply to that value, in the same order.
-// vec: h 16-byte and mask 2-byte aligned.
+// vec: h 16-byte and mask 2-byte aligned.  JOIN: every block joins the nsum
+// summaries and derives the constants itself, and block 0 publishes them, in
+// place of a k_pr_finish launch: few summaries (kJoinMax, planets of up to
+// 131,072 vertices) cost less to join in every block than a launch of one block
+// takes (10,242 heights: 7 us against 5 + 4 and a launch's gap; 1,024,002, 251
+// summaries: 21 against 7 + 10).
+template <bool JOIN>
 __global__ __launch_bounds__(kFinalThreads) void k_chain_final(double *h, uint8_t *__restrict__ mask,
-                                                               int64_t n,
-                                                               const PrHead *__restrict__ head,
-                                                               double min_alt, double max_alt,
+                                                               int64_t n, PrHead *__restrict__ head,
+                                                               const PSum *__restrict__ sum,
+                                                               int64_t nsum, double min_alt,
+                                                               double max_alt,
                                                                int *__restrict__ err, int vec)
 {
     const double x_min = dunkey(head->keys0[0]), x_max = dunkey(head->keys0[1]);
     const double xr = x_max - x_min, nr = max_alt - min_alt;
     const double level = head->level;
-    const double lo1 = head->lo1, r1 = head->r1, lo0 = head->lo0, r0 = head->r0;
-    const double h4min = head->h4min, h4max = head->h4max;
-    const bool fast = head->fast != 0;
+    __shared__ ChainConsts own;
+    __shared__ PSum s[2];
+    if (JOIN) {
+        pr_reduce_sums<kFinalThreads / 2>(sum, nsum, s);
+        if (threadIdx.x == 0) {
+            own = chain_derive(s[1], s[0], head->xmin, head->xmax, level);
+            if (blockIdx.x == 0) chain_publish(head, s, own);
+        }
+        __syncthreads();
+    }
+    double lo1 = JOIN ? own.lo1 : head->lo1, r1 = JOIN ? own.r1 : head->r1;
+    const double lo0 = JOIN ? own.lo0 : head->lo0, r0 = JOIN ? own.r0 : head->r0;
+    const double h4min = JOIN ? own.h4min : head->h4min, h4max = JOIN ? own.h4max : head->h4max;
+    const bool fast = (JOIN ? own.fast : head->fast) != 0;
     bool zero = false;
+    unsigned long long klo = ~0ull, khi = 0ull;
+    if (!fast) {   // the ocean's bounds as k_pr_map takes them, mode 1
+        double upper = head->xmin;
+        lo1 = head->xmax;
+        psum_bounds(JOIN ? s[1] : head->s[1], head->xmin, head->xmax, lo1, upper);
+        r1 = upper - lo1;
+    }
     auto f = [&](double v, uint8_t &m) {
-        const double t = ((v - x_min) / xr) * nr + min_alt;
+        double t = ((v - x_min) / xr) * nr + min_alt;
         m = t <= level ? 1 : 0;
-        if (!fast) return t;  // the five-pass kernels continue from here
+        if (!fast) {   // the five-pass kernels continue from here
+            if (m) {
+                zero = zero | (r1 == 0.0);
+                t = pr_power_map(t, lo1, r1, 0.5);
+            }
+            const unsigned long long k = dkey(t);
+            klo = k < klo ? k : klo;
+            khi = k > khi ? k : khi;
+            return t;
+        }
         double r = m ? pr_power_map(t, lo1, r1, 0.5) : pr_power_map(t, lo0, r0, 2.0);
         r = r - level;
         return split_rescale(r, h4min, h4max, min_alt, max_alt, zero);
@@ -1100,6 +1175,13 @@ __global__ __launch_bounds__(kFinalThreads) void k_chain_final(double *h, uint8_
     // chain_derive sets fast only when no range is zero; kept as a check.
     if (__any(zero) && (threadIdx.x & 63) == 0)
         __hip_atomic_fetch_or(err, NX_ERR_DIV0_BIT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (!fast) {
+        block_minmax(klo, khi);
+        if (threadIdx.x == 0) {
+            __hip_atomic_fetch_min(&head->keys1[0], klo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_fetch_max(&head->keys1[1], khi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
 }
 
 static size_t a256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -1107,6 +1189,17 @@ static size_t a256(size_t x) { return (x + 255) & ~(size_t)255; }
 // Summary blocks: at most kPrMaxBlocks; each wave takes a contiguous run of
 // wave chunks.
 constexpr int64_t kPrMaxBlocks = 2048;
+// The height chain's workspace holds its block records of the min/max behind
+// the summaries, of which it makes at most kChainBlocks pairs.
+constexpr int kMaxRec = 2048;
+constexpr int64_t kChainBlocks = 1664;
+constexpr int64_t kJoinMax = 32;
+static_assert(sizeof(PSum) * 2 * kChainBlocks + 16 * kMaxRec <= sizeof(PSum) * 2 * kPrMaxBlocks,
+              "records beside the summaries");
+static unsigned long long *chain_records(void *ws)
+{
+    return (unsigned long long *)((char *)ws + 256 + sizeof(PSum) * 2 * kPrMaxBlocks) - 2 * kMaxRec;
+}
 
 struct PrGrid {
     int64_t nunits, cpw, blocks;
@@ -1132,12 +1225,12 @@ static int pr_blocks_per_cu()
     return v;
 }
 
-static PrGrid pr_grid(nx_ctx *ctx, int64_t n, int blocks_per_cu)
+static PrGrid pr_grid(nx_ctx *ctx, int64_t n, int blocks_per_cu, int64_t most = kPrMaxBlocks)
 {
     constexpr int64_t wpb = kPrThreads / 64;
     PrGrid g;
     g.nunits = (n + kPrUnit - 1) / kPrUnit;
-    const int64_t want = wpb * std::max<int64_t>(1, std::min<int64_t>(kPrMaxBlocks, (int64_t)ctx->num_cus * blocks_per_cu));
+    const int64_t want = wpb * std::max<int64_t>(1, std::min<int64_t>(most, (int64_t)ctx->num_cus * blocks_per_cu));
     g.cpw = (g.nunits + want - 1) / want;
     const int64_t waves = (g.nunits + g.cpw - 1) / g.cpw;
     g.blocks = (waves + wpb - 1) / wpb;
@@ -1167,11 +1260,11 @@ int power_rescale(nx_ctx *ctx, const double *x, const uint8_t *mask, int64_t n, 
     const unsigned grid = red_grid(ctx, n);
     hipLaunchKernelGGL(k_minmax_init, dim3(1), dim3(64), 0, stream, head->keys0);
     hipLaunchKernelGGL(k_minmax, dim3(mm_grid(ctx, n)), dim3(kMinmaxThreads), 0, stream, x, n, head->keys0,
-                       vec16(x));
+                       vec16(x), (unsigned long long *)nullptr);
     hipLaunchKernelGGL((k_pr_summary<false, false>), dim3((unsigned)g.blocks), dim3(kPrThreads), 0,
                        stream, const_cast<double *>(x), const_cast<uint8_t *>(mask), n, g.nunits,
                        g.cpw, pr_vec(x, mask), sum, head, ChainArgs{0.0, 0.0, 0.0, nullptr},
-                       ctx->d_err);
+                       ctx->d_err, (const unsigned long long *)nullptr, 0);
     hipLaunchKernelGGL(k_pr_finish, dim3(1), dim3(1024), 0, stream, sum, g.blocks, head, 1, 0);
     hipLaunchKernelGGL(k_pr_map, dim3(grid), dim3(256), 0, stream, x, out, mask, n, mode, power,
                        head, (const unsigned long long *)nullptr, 0,
@@ -1189,19 +1282,19 @@ int power_rescale(nx_ctx *ctx, const double *x, const uint8_t *mask, int64_t n, 
 // the block summaries and derives every later bound and min/max from them
 // (k_pr_finish, chain_derive); the second pass applies the whole chain to
 // each value and writes heights and mask.  When the derivation does not hold (a zero range,
-// a zero or non-finite extreme), the second pass writes the rescaled heights
-// and mask instead, and the kernels of the five-pass form, which otherwise
-// return at once, finish the chain: the ocean power_rescale with the min/max
-// of its result; the land power_rescale with the shift by the ocean level and
-// the min/max of its result; the final split rescale around 0.  The
+// a zero or non-finite extreme), the second pass writes the heights after the
+// ocean power_rescale, the mask and those heights' min/max instead, and the
+// kernels of the five-pass form, which otherwise return at once, finish the
+// chain: the land power_rescale with the shift by the ocean level and the
+// min/max of its result; the final split rescale around 0.  The
 // five-pass form itself (NX_OPT_CHAIN_PASSES 5) writes in its summary pass
 // and reduces the summaries in a kernel of its own.  Both forms give the same
 // bits.
 
 size_t height_chain_workspace_bytes(int64_t n) { return power_rescale_workspace_bytes(n); }
 
-// The chain after head->keys0 holds the min/max keys of h.
-static int chain_after_keys(nx_ctx *ctx, double *h, int64_t n, double min_alt, double max_alt,
+// The chain after the nrec block records of the min/max of h.
+static int chain_after_keys(nx_ctx *ctx, int nrec, double *h, int64_t n, double min_alt, double max_alt,
                             double ocean_percent, uint8_t *mask, double *level, void *ws,
                             hipStream_t stream)
 {
@@ -1209,32 +1302,36 @@ static int chain_after_keys(nx_ctx *ctx, double *h, int64_t n, double min_alt, d
     auto *head = (PrHead *)ws;
     auto *sum = (PSum *)((char *)ws + 256);
     const int two = ctx->chain_passes == 2 ? 1 : 0;
-    const PrGrid g = pr_grid(ctx, n, two ? pr_blocks_per_cu<true, false>() : pr_blocks_per_cu<true, true>());
+    const PrGrid g = pr_grid(ctx, n, two ? pr_blocks_per_cu<true, false>() : pr_blocks_per_cu<true, true>(),
+                             kChainBlocks);
+    const unsigned long long *rec = chain_records(ws);
     const unsigned grid = red_grid(ctx, n);
     const ChainArgs ca{min_alt, max_alt, ocean_percent, level};
     const int vsum = pr_vec(h, mask), vmap = vec16(h) & vec2(mask);
     if (ctx->chain_passes == 2) {
         // The summary pass, the join and derivation, then the writing pass;
-        // the five-pass kernels after it return at once when head->fast,
-        // else continue from the rescaled heights and mask the writing pass
-        // left (k_pr_finish resets keys1 and keys2).
+        // the last two of the five-pass kernels after it return at once when
+        // head->fast, else continue from the heights after the ocean's map
+        // that the writing pass left.
         hipLaunchKernelGGL((k_pr_summary<true, false>), dim3((unsigned)g.blocks), dim3(kPrThreads),
-                           0, stream, h, mask, n, g.nunits, g.cpw, vsum, sum, head, ca, ctx->d_err);
-        hipLaunchKernelGGL(k_pr_finish, dim3(1), dim3(1024), 0, stream, sum, g.blocks, head, 0, 1);
-        hipLaunchKernelGGL(k_chain_final, dim3(grid), dim3(kFinalThreads), 0, stream, h, mask, n,
-                           (const PrHead *)head, min_alt, max_alt, ctx->d_err, vmap);
+                           0, stream, h, mask, n, g.nunits, g.cpw, vsum, sum, head, ca, ctx->d_err,
+                           rec, nrec);
+        const bool join = g.blocks <= kJoinMax;
+        if (!join)
+            hipLaunchKernelGGL(k_pr_finish, dim3(1), dim3(1024), 0, stream, sum, g.blocks, head, 0, 1);
+        hipLaunchKernelGGL((join ? k_chain_final<true> : k_chain_final<false>), dim3(grid),
+                           dim3(kFinalThreads), 0, stream, h, mask, n, head, (const PSum *)sum,
+                           g.blocks, min_alt, max_alt, ctx->d_err, vmap);
     } else {
         // nixis.py:332-346 in one pass
         hipLaunchKernelGGL((k_pr_summary<true, true>), dim3((unsigned)g.blocks),
                            dim3(kPrThreads), 0, stream, h, mask, n, g.nunits, g.cpw, vsum, sum, head,
-                           ca, ctx->d_err);
+                           ca, ctx->d_err, rec, nrec);
         hipLaunchKernelGGL(k_pr_finish, dim3(1), dim3(1024), 0, stream, sum, g.blocks, head, 0, 0);
-        hipLaunchKernelGGL(k_minmax_init, dim3(1), dim3(64), 0, stream, head->keys1);
-        hipLaunchKernelGGL(k_minmax_init, dim3(1), dim3(64), 0, stream, head->keys2);
+        // nixis.py:352: the ocean floor, power 0.5
+        hipLaunchKernelGGL(k_pr_map, dim3(grid), dim3(256), 0, stream, h, h, mask, n, 1, 0.5, head,
+                           (const unsigned long long *)nullptr, 0, head->keys1, ctx->d_err, vmap, 0);
     }
-    // nixis.py:352: the ocean floor, power 0.5
-    hipLaunchKernelGGL(k_pr_map, dim3(grid), dim3(256), 0, stream, h, h, mask, n, 1, 0.5, head,
-                       (const unsigned long long *)nullptr, 0, head->keys1, ctx->d_err, vmap, two);
     // nixis.py:355 and 362: the land, power 2.0, then the shift
     hipLaunchKernelGGL(k_pr_map, dim3(grid), dim3(256), 0, stream, h, h, mask, n, 0, 2.0, head,
                        (const unsigned long long *)head->keys1, 1, head->keys2, ctx->d_err, vmap,
@@ -1263,11 +1360,11 @@ int height_chain(nx_ctx *ctx, double *h, int64_t n, double min_alt, double max_a
     int rc = chain_check(ctx, h, n, mask, level, ws);
     if (rc) return rc;
     NX_HIP(hipSetDevice(ctx->device));
-    auto *head = (PrHead *)ws;
-    hipLaunchKernelGGL(k_minmax_init, dim3(1), dim3(64), 0, stream, head->keys0);
-    hipLaunchKernelGGL(k_minmax, dim3(mm_grid(ctx, n)), dim3(kMinmaxThreads), 0, stream, h, n, head->keys0,
-                       vec16(h));
-    return chain_after_keys(ctx, h, n, min_alt, max_alt, ocean_percent, mask, level, ws, stream);
+    const unsigned blocks = mm_grid(ctx, n);
+    if (blocks > (unsigned)kMaxRec) return set_error(NX_EINVAL, "%u min/max blocks", blocks);
+    hipLaunchKernelGGL(k_minmax, dim3(blocks), dim3(kMinmaxThreads), 0, stream, h, n,
+                       (unsigned long long *)nullptr, vec16(h), chain_records(ws));
+    return chain_after_keys(ctx, (int)blocks, h, n, min_alt, max_alt, ocean_percent, mask, level, ws, stream);
 }
 
 // terrain.py:32-59 into h (starting from zero, as nixis.py:330 passes no
@@ -1280,12 +1377,11 @@ int terrain_heights(nx_ctx *ctx, const double *verts, int64_t V, const int32_t *
     int rc = chain_check(ctx, h, V, mask, level, ws);
     if (rc) return rc;
     NX_HIP(hipSetDevice(ctx->device));
-    auto *head = (PrHead *)ws;
-    hipLaunchKernelGGL(k_minmax_init, dim3(1), dim3(64), 0, stream, head->keys0);
+    int nrec = kMaxRec;
     rc = sample_octaves_keys(ctx, verts, V, perm, pgi, n_oct, rough, strength, radius, h, 0,
-                             nullptr, nullptr, head->keys0, stream);
+                             nullptr, nullptr, chain_records(ws), &nrec, stream);
     if (rc) return rc;
-    return chain_after_keys(ctx, h, V, min_alt, max_alt, ocean_percent, mask, level, ws, stream);
+    return chain_after_keys(ctx, nrec, h, V, min_alt, max_alt, ocean_percent, mask, level, ws, stream);
 }
 
 // ---- terrain_heights without a caller workspace ---------------------------
