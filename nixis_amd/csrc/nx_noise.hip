@@ -83,6 +83,66 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
     sample_octaves_body<false>(a, verts, V, elev, nullptr, nullptr, err, rec);
 }
 
+// Few vertices: a block takes 64 of them, one per lane, and its waves share
+// the octaves; the first wave then adds the octaves' values up in order, so the
+// result is that of one lane per vertex bit for bit (an octave's own
+// coordinates equal the doubled ones, see doubles_exactly).  With one wave or
+// two per SIMD a launch takes as long as one wave's octaves do one after the
+// other, about 0.85 us each (us a launch, this way and without: 10,242 vertices
+// and 2, 8, 16 octaves 3.4 / 4.5, 3.8 / 9.4, 5.0 / 16.4; 64,002: 4.1 / 4.6, 5.5 /
+// 9.7, 8.6 / 16.9).  More vertices fill the GPU by themselves unless there are
+// several octaves (127,692 and 2, 4, 8, 16: 6.5 / 4.9, 7.2 / 6.7, 8.8 / 11.0, 14.0
+// / 19.3).
+constexpr int kSplitWaves = 8;
+static bool split_octaves(int64_t V, int n_oct)
+{
+    return n_oct > 1 && (V <= 64 * 1024 || (V <= 64 * 2048 && n_oct >= 6));
+}
+__global__ __launch_bounds__(64 * kSplitWaves) __attribute__((amdgpu_waves_per_eu(8))) void
+k_sample_octaves_split(OctaveArgs a, const double *__restrict__ verts, int64_t V,
+                       double *__restrict__ elev, int *__restrict__ err,
+                       unsigned long long *__restrict__ rec)
+{
+    __shared__ NoiseTables T;
+    __shared__ float value[NX_MAX_OCTAVES][64];
+    load_tables(T, a.tables);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t i = (int64_t)blockIdx.x * 64 + lane, at = i < V ? i : V - 1;
+    const double x = verts[3 * at], y = verts[3 * at + 1], z = verts[3 * at + 2];
+    __syncthreads();
+    for (int o = wave; o < a.oct.n_oct; o += kSplitWaves) {
+        const double r = a.oct.rough[o];
+        const Skewed s = skew3(x * r, y * r, z * r);
+        value[o][lane] = noise3_sum<false>(s.x, s.y, s.z, T, nullptr);
+    }
+    __syncthreads();
+    if (wave != 0) return;
+    double acc = a.accumulate ? elev[at] : 0.0;
+    bool bad = false;
+    if (a.oct.n_oct > 0) {
+        const double rc = a.oct.rough[a.oct.check_oct];
+        bad = !in_domain(skew3(x * rc, y * rc, z * rc));
+        acc += a.oct.base;
+        float accf = 0.0f;
+        for (int o = 0; o < a.oct.n_oct; ++o) accf = fmaf(value[o][lane], a.oct.wsumf[o], accf);
+        acc = acc + (double)accf;
+    }
+    if (i < V) elev[i] = acc;
+    if (bad) __hip_atomic_fetch_or(err, NX_ERR_RANGE_BIT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (rec) {
+        unsigned long long lo = dkey(acc), hi = lo;
+        for (int off = 32; off > 0; off >>= 1) {
+            const unsigned long long b = __shfl_xor(lo, off, 64), c = __shfl_xor(hi, off, 64);
+            lo = b < lo ? b : lo;
+            hi = c > hi ? c : hi;
+        }
+        if (lane == 0) {
+            rec[2 * blockIdx.x] = lo;
+            rec[2 * blockIdx.x + 1] = hi;
+        }
+    }
+}
+
 // Debug launch: per-octave noise values and selection records.
 __global__ __launch_bounds__(256) void k_sample_octaves_dbg(
     OctaveArgs a, const double *__restrict__ verts, int64_t V, double *__restrict__ elev,
@@ -202,7 +262,8 @@ int sample_octaves_keys(nx_ctx *ctx, const double *verts, int64_t V, const int32
     a.accumulate = accumulate ? 1 : 0;
     if (V == 0) return NX_OK;
     NX_HIP(hipSetDevice(ctx->device));
-    const int grid = grid_for(ctx, V, 8);
+    const bool split = split_octaves(V, n_oct) && !dbg_noise && !dbg_sel;
+    const int grid = split ? (int)((V + 63) / 64) : grid_for(ctx, V, 8);
     if (rec) {   // one pair per block, at most *nrec
         if (grid > *nrec) return set_error(NX_EINVAL, "%d blocks for %d min/max records", grid, *nrec);
         *nrec = grid;
@@ -211,6 +272,9 @@ int sample_octaves_keys(nx_ctx *ctx, const double *verts, int64_t V, const int32
         if (rec) return set_error(NX_EINVAL, "min/max keys are not reduced with debug output");
         hipLaunchKernelGGL(k_sample_octaves_dbg, dim3(grid), dim3(256), 0, stream, a, verts, V,
                            elev, dbg_noise, dbg_sel, ctx->d_err);
+    } else if (split) {
+        hipLaunchKernelGGL(k_sample_octaves_split, dim3(grid), dim3(64 * kSplitWaves), 0, stream, a,
+                           verts, V, elev, ctx->d_err, rec);
     } else {
         hipLaunchKernelGGL(k_sample_octaves, dim3(grid), dim3(256), 0, stream, a, verts, V, elev,
                            ctx->d_err, rec);

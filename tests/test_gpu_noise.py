@@ -159,3 +159,29 @@ def test_noise_empty_and_zero_octaves():
     assert terrain.sample_octaves(np.zeros((0, 3)), None, perm, pgi, 3).shape == (0,)
     e = terrain.sample_octaves(util.create_points(4), None, perm, pgi, 0)
     assert (e == 0).all()
+
+
+@pytest.mark.parametrize("n_oct,lacunarity", [(2, 2.0), (3, 2.5), (6, 2.0), (8, 2.5), (9, 2.0),
+                                              (17, 1.3), (32, 1.1)])
+def test_octaves_shared_by_waves_equal_one_lane_each(n_oct, lacunarity):
+    """Few vertices share their octaves among a block's waves; the same
+    vertices at the head of a set too large for that give the same elevations
+    bit for bit, from zero and added to given ones, and so do the min/max that
+    the height chain takes from either launch."""
+    perm, pgi = osx.init(77)
+    rough, strength = terrain.octave_scalars(n_oct, 1.5, 0.4, lacunarity, 0.5, 1.0)
+    gen = torch.Generator(device="cuda").manual_seed(n_oct)
+    pts = torch.randn((140000, 3), dtype=torch.float64, device="cuda", generator=gen)
+    base = torch.randn(140000, dtype=torch.float64, device="cuda", generator=gen)
+    whole = terrain.sample_octaves_device(pts, None, perm, pgi, rough, strength, 1.0)
+    added = terrain.sample_octaves_device(pts, base.clone(), perm, pgi, rough, strength, 1.0)
+    for V in (1, 63, 64, 65, 1000, 65536, 65537, 131072, 131073):
+        e = terrain.sample_octaves_device(pts[:V], None, perm, pgi, rough, strength, 1.0)
+        assert torch.equal(e, whole[:V])
+        e = terrain.sample_octaves_device(pts[:V], base[:V].clone(), perm, pgi, rough, strength, 1.0)
+        assert torch.equal(e, added[:V])
+        if V >= 1000:
+            h, mask, level = terrain.terrain_heights_device(pts[:V], perm, pgi, rough, strength)
+            h2, mask2, level2 = util.height_chain_device(whole[:V].clone(), -4000.0, 8850.0, 55.0)
+            assert torch.equal(h, h2) and torch.equal(mask, mask2) and torch.equal(level, level2)
+    _lib.Context.get(pts.device).sync_check()
