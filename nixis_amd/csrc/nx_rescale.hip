@@ -57,9 +57,12 @@ __global__ void k_minmax_init(unsigned long long *keys)
 // load instruction covers one contiguous range) with the next chunk's loads
 // in flight while it reduces the current one.  vec: x is 16-byte aligned.
 // keys null: the block's pair goes to rec instead (joined by k_pr_summary).
+// COPY: x is also written to copy (k_chain_small's input).
+template <bool COPY = false>
 __global__ __launch_bounds__(kMinmaxThreads) void k_minmax(const double *__restrict__ x, int64_t n,
                                                 unsigned long long *__restrict__ keys, int vec,
-                                                unsigned long long *__restrict__ rec)
+                                                unsigned long long *__restrict__ rec,
+                                                double *__restrict__ copy = nullptr)
 {
     unsigned long long lo = ~0ull, hi = 0ull;
     auto upd = [&](double v) {
@@ -101,7 +104,10 @@ __global__ __launch_bounds__(kMinmaxThreads) void k_minmax(const double *__restr
         if (u + 1 < u1) load(u + 1, vn, leftn);
 #pragma unroll
         for (int j = 0; j < 8; ++j)
-            if (off(j) < left) upd(v[j]);
+            if (off(j) < left) {
+                upd(v[j]);
+                if (COPY) copy[u * 512 + 2 * lane + off(j)] = v[j];
+            }
     }
     block_minmax(lo, hi);
     if (threadIdx.x == 0 && keys) {
@@ -173,7 +179,7 @@ int rescale(nx_ctx *ctx, const double *x, int64_t n, double lower, double upper,
     unsigned long long *keys = ctx->d_keys + 2 * (ctx->key_slot.fetch_add(1) % kKeySlots);
     const unsigned grid = (unsigned)std::min<int64_t>((n + 255) / 256, (int64_t)ctx->num_cus * 8);
     hipLaunchKernelGGL(k_minmax_init, dim3(1), dim3(64), 0, stream, keys);
-    hipLaunchKernelGGL(k_minmax, dim3(mm_grid(ctx, n)), dim3(kMinmaxThreads), 0, stream, x, n, keys, vec16(x),
+    hipLaunchKernelGGL(k_minmax<>, dim3(mm_grid(ctx, n)), dim3(kMinmaxThreads), 0, stream, x, n, keys, vec16(x),
                        (unsigned long long *)nullptr);
     hipLaunchKernelGGL(k_rescale_map, dim3(grid), dim3(256), 0, stream, x, n, keys, lower, upper,
                        out, minmax, ctx->d_err, vec16(x) & vec16(out));
@@ -265,7 +271,7 @@ static int rescale_ex_launch(nx_ctx *ctx, const double *x, int64_t n, const Resc
     unsigned long long *keys = key_slot(ctx);
     const unsigned grid = red_grid(ctx, n);
     hipLaunchKernelGGL(k_minmax_init, dim3(1), dim3(64), 0, stream, keys);
-    hipLaunchKernelGGL(k_minmax, dim3(mm_grid(ctx, n)), dim3(kMinmaxThreads), 0, stream, x, n, keys, vec16(x),
+    hipLaunchKernelGGL(k_minmax<>, dim3(mm_grid(ctx, n)), dim3(kMinmaxThreads), 0, stream, x, n, keys, vec16(x),
                        (unsigned long long *)nullptr);
     hipLaunchKernelGGL(k_rescale_ex, dim3(grid), dim3(256), 0, stream, x, n, keys, a, out,
                        minmax, ctx->d_err, vec16(x) & vec16(out), (const int32_t *)nullptr);
@@ -775,79 +781,39 @@ __device__ void pr_reduce_sums(const PSum *sum, int64_t nsum, PSum *s)
     __syncthreads();
 }
 
-// Summaries of the values whose mask is unset (sum[2b]) and set (sum[2b + 1])
-// over block b's values.  Wave w of block b takes the contiguous run of
-// wave chunks [(8b + w) * cpw, (8b + w + 1) * cpw), each as four slices of
-// 128 values, two per lane.  Each half's run is followed in sequence order
-// (WaveRun, wave_run_slice) until its first break (a value not below the
-// one before it); after the break only the minimum and maximum of that
-// half's later values can change the summary (a later value that is a new
-// running minimum is below the maximum already taken), so they are kept
-// per lane and reduced once at the end.  A chunk in which no unbroken half
-// has a value takes the minimum/maximum path alone: waves whose run lies
-// inside one region see a single half for all of it, and every wave must
-// stream at the same rate.  The eight waves join in order.
-// CHAIN: x holds the noise heights; each value is the standard rescale
-// (util.py:139) with min/max joined from the nrec block records rec (closing
-// atomics of 2,048 noise blocks on two keys took about 28 us) and left in
-// head->keys0 by block 0; the rescaled min/max and the
-// ocean level are derived from the same keys (the map is monotone, so its
-// extremes are the images of x's), and mask = t <= level (terrain.py:61-72);
-// WRITE: t and the mask are written back.  vec: x is 16-byte and mask
-// 2-byte aligned (vector accesses).
-template <bool CHAIN, bool WRITE>
-__global__ __launch_bounds__(kPrThreads) void k_pr_summary(double *x, uint8_t *mask, int64_t n,
-                                                           int64_t nunits, int64_t cpw, int vec,
-                                                           PSum *__restrict__ sum,
-                                                           PrHead *__restrict__ head, ChainArgs ca,
-                                                           int *__restrict__ err,
-                                                           const unsigned long long *__restrict__ rec,
-                                                           int nrec)
-{
-    __shared__ PSum lds[2][kPrThreads / 64];
-    double x_min = 0.0, xr = 1.0, nr = 0.0, level = 0.0;
-    if (CHAIN) {
-        __shared__ unsigned long long keys[2];
-        unsigned long long lo = ~0ull, hi = 0ull;
-        for (int i = threadIdx.x; i < nrec; i += kPrThreads) {
-            const unsigned long long a = rec[2 * i], b = rec[2 * i + 1];
-            lo = a < lo ? a : lo;
-            hi = b > hi ? b : hi;
-        }
-        block_minmax(lo, hi);
-        if (threadIdx.x == 0) {
-            keys[0] = lo;
-            keys[1] = hi;
-            if (blockIdx.x == 0) {
-                head->keys0[0] = lo;
-                head->keys0[1] = hi;
-                head->keys1[0] = head->keys2[0] = ~0ull;   // for the later passes' reductions
-                head->keys1[1] = head->keys2[1] = 0ull;
-            }
-        }
-        __syncthreads();
-        x_min = dunkey(keys[0]);
-        const double x_max = dunkey(keys[1]);
-        xr = x_max - x_min;
-        nr = ca.upper - ca.lower;
-        const double fa = ((x_min - x_min) / xr) * nr + ca.lower;
-        const double fb = ((x_max - x_min) / xr) * nr + ca.lower;
-        const double tmin = fa < fb ? fa : fb, tmax = fa < fb ? fb : fa;
-        level = tmin + ((tmax - tmin) * ca.percent / 100.0);  // util.py:556-566
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            head->xmin = tmin;
-            head->xmax = tmax;
-            head->level = level;
-            *ca.level_out = level;
-            if (xr == 0.0)
-                __hip_atomic_fetch_or(err, NX_ERR_DIV0_BIT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
+// The chain's first rescale (util.py:139) and its ocean level (util.py:556-566)
+// from the min/max of the noise heights; tmin, tmax: the rescaled heights'
+// (the map is monotone, so its extremes are the images of x's).
+struct ChainMap {
+    double x_min, xr, nr, lower, level;
+    __device__ __forceinline__ double rescale(double v) const
+    {
+        return ((v - x_min) / xr) * nr + lower;
     }
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+};
+
+__device__ __forceinline__ ChainMap chain_map(double x_min, double x_max, const ChainArgs &ca,
+                                              double &tmin, double &tmax)
+{
+    ChainMap c{x_min, x_max - x_min, ca.upper - ca.lower, ca.lower, 0.0};
+    const double fa = c.rescale(x_min), fb = c.rescale(x_max);
+    tmin = fa < fb ? fa : fb;
+    tmax = fa < fb ? fb : fa;
+    c.level = tmin + ((tmax - tmin) * ca.percent / 100.0);
+    return c;
+}
+
+// Summaries w0, w1 (valid in every lane) of the values whose mask is unset
+// and set in wave chunks u_begin..u_end-1, in order; the comment at
+// k_pr_summary describes them.
+template <bool CHAIN, bool WRITE>
+__device__ __forceinline__ void pr_wave_summary(double *x, uint8_t *mask, int64_t n, int64_t u_begin,
+                                                int64_t u_end, int vec, const ChainMap &c, PSum &w0,
+                                                PSum &w1)
+{
+    const int lane = threadIdx.x & 63;
     WaveRun R0 = {0.0, 0.0, 0, 0}, R1 = {0.0, 0.0, 0, 0};  // land, ocean
     double mn0 = INFINITY, mx0 = -INFINITY, mn1 = INFINITY, mx1 = -INFINITY;  // after the break
-    const int64_t u_begin = ((int64_t)blockIdx.x * (kPrThreads / 64) + wave) * cpw;
-    const int64_t u_end = u_begin + cpw < nunits ? u_begin + cpw : nunits;
     // Wave chunk u is kPrSlices slices of 128 values; lane l holds values
     // 2l and 2l + 1 of each slice (v[2k], v[2k + 1] of slice k), so every
     // access instruction covers one contiguous range.  Value j of the lane is
@@ -894,8 +860,8 @@ __global__ __launch_bounds__(kPrThreads) void k_pr_summary(double *x, uint8_t *m
             mb = 0;
 #pragma unroll
             for (int k = 0; k < kPrPer; ++k) {
-                v[k] = ((v[k] - x_min) / xr) * nr + ca.lower;
-                mb |= (v[k] <= level ? 1u : 0u) << k;
+                v[k] = c.rescale(v[k]);
+                mb |= (v[k] <= c.level ? 1u : 0u) << k;
             }
         }
         if (CHAIN && WRITE) {
@@ -964,7 +930,77 @@ __global__ __launch_bounds__(kPrThreads) void k_pr_summary(double *x, uint8_t *m
             }
         }
     }
-    const PSum w0 = wave_run_summary(R0, mn0, mx0), w1 = wave_run_summary(R1, mn1, mx1);
+    w0 = wave_run_summary(R0, mn0, mx0);
+    w1 = wave_run_summary(R1, mn1, mx1);
+}
+
+// Summaries of the values whose mask is unset (sum[2b]) and set (sum[2b + 1])
+// over block b's values.  Wave w of block b takes the contiguous run of
+// wave chunks [(8b + w) * cpw, (8b + w + 1) * cpw), each as four slices of
+// 128 values, two per lane.  Each half's run is followed in sequence order
+// (WaveRun, wave_run_slice) until its first break (a value not below the
+// one before it); after the break only the minimum and maximum of that
+// half's later values can change the summary (a later value that is a new
+// running minimum is below the maximum already taken), so they are kept
+// per lane and reduced once at the end.  A chunk in which no unbroken half
+// has a value takes the minimum/maximum path alone: waves whose run lies
+// inside one region see a single half for all of it, and every wave must
+// stream at the same rate.  The eight waves join in order.
+// CHAIN: x holds the noise heights; each value is the standard rescale
+// (util.py:139) with min/max joined from the nrec block records rec (closing
+// atomics of 2,048 noise blocks on two keys took about 28 us) and left in
+// head->keys0 by block 0; the rescaled min/max and the
+// ocean level are derived from the same keys (the map is monotone, so its
+// extremes are the images of x's), and mask = t <= level (terrain.py:61-72);
+// WRITE: t and the mask are written back.  vec: x is 16-byte and mask
+// 2-byte aligned (vector accesses).
+template <bool CHAIN, bool WRITE>
+__global__ __launch_bounds__(kPrThreads) void k_pr_summary(double *x, uint8_t *mask, int64_t n,
+                                                           int64_t nunits, int64_t cpw, int vec,
+                                                           PSum *__restrict__ sum,
+                                                           PrHead *__restrict__ head, ChainArgs ca,
+                                                           int *__restrict__ err,
+                                                           const unsigned long long *__restrict__ rec,
+                                                           int nrec)
+{
+    __shared__ PSum lds[2][kPrThreads / 64];
+    ChainMap c{0.0, 1.0, 0.0, 0.0, 0.0};
+    if (CHAIN) {
+        __shared__ unsigned long long keys[2];
+        unsigned long long lo = ~0ull, hi = 0ull;
+        for (int i = threadIdx.x; i < nrec; i += kPrThreads) {
+            const unsigned long long a = rec[2 * i], b = rec[2 * i + 1];
+            lo = a < lo ? a : lo;
+            hi = b > hi ? b : hi;
+        }
+        block_minmax(lo, hi);
+        if (threadIdx.x == 0) {
+            keys[0] = lo;
+            keys[1] = hi;
+            if (blockIdx.x == 0) {
+                head->keys0[0] = lo;
+                head->keys0[1] = hi;
+                head->keys1[0] = head->keys2[0] = ~0ull;   // for the later passes' reductions
+                head->keys1[1] = head->keys2[1] = 0ull;
+            }
+        }
+        __syncthreads();
+        double tmin, tmax;
+        c = chain_map(dunkey(keys[0]), dunkey(keys[1]), ca, tmin, tmax);
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            head->xmin = tmin;
+            head->xmax = tmax;
+            head->level = c.level;
+            *ca.level_out = c.level;
+            if (c.xr == 0.0)
+                __hip_atomic_fetch_or(err, NX_ERR_DIV0_BIT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int64_t u_begin = ((int64_t)blockIdx.x * (kPrThreads / 64) + wave) * cpw;
+    PSum w0, w1;
+    pr_wave_summary<CHAIN, WRITE>(x, mask, n, u_begin, u_begin + cpw < nunits ? u_begin + cpw : nunits,
+                                  vec, c, w0, w1);
     if (lane == 0) {
         lds[0][wave] = w0;
         lds[1][wave] = w1;
@@ -1184,6 +1220,128 @@ __global__ __launch_bounds__(kFinalThreads) void k_chain_final(double *h, uint8_
     }
 }
 
+// The whole chain of few heights (n <= kSmallChain) in one launch: a launch
+// costs the host about 5 us, so four of them outlast the work (with the noise,
+// 642 heights: 29.3 us a call, 21.5 in this form; 10,242: 29.6 and 21.6;
+// 16,002: 29.5 and 23.0).  The
+// heights come from x, a copy in the workspace, so that every block can
+// summarise all of them for itself while others already write their results;
+// each then maps a run of its own (one block alone took 24 us, bound by its
+// CU's divisions).  The limit is what the workspace holds beside the records.
+// The same steps, values and head as the other launches': the block records'
+// join, the wave summaries in order, the derivation, the writing pass.  Where
+// the derivation does not hold, block 0 alone takes the five-pass kernels'
+// ocean and land maps with the shift and the split rescale, with the min/max
+// between them.
+constexpr int64_t kSmallChain = 16384;
+__global__ __launch_bounds__(1024) void k_chain_small(double *x, double *h, uint8_t *mask,
+                                                      int64_t n, PrHead *__restrict__ head, ChainArgs ca,
+                                                      int *__restrict__ err,
+                                                      const unsigned long long *__restrict__ rec,
+                                                      int nrec)
+{
+    __shared__ unsigned long long keys[3][2];
+    __shared__ PSum part[2][16], s[2];
+    __shared__ ChainConsts own;
+    const int t = threadIdx.x, wave = t >> 6;
+    auto minmax = [&](unsigned long long lo, unsigned long long hi, unsigned long long (&k)[2]) {
+        block_minmax(lo, hi);
+        if (t == 0) {
+            k[0] = lo;
+            k[1] = hi;
+        }
+        __syncthreads();
+    };
+    unsigned long long lo = ~0ull, hi = 0ull;
+    for (int i = t; i < nrec; i += 1024) {
+        const unsigned long long a = rec[2 * i], b = rec[2 * i + 1];
+        lo = a < lo ? a : lo;
+        hi = b > hi ? b : hi;
+    }
+    minmax(lo, hi, keys[0]);
+    double tmin, tmax;
+    const ChainMap c = chain_map(dunkey(keys[0][0]), dunkey(keys[0][1]), ca, tmin, tmax);
+    bool zero = c.xr == 0.0;
+    const int64_t nunits = (n + kPrUnit - 1) / kPrUnit, cpw = (nunits + 15) / 16;
+    const int64_t u0 = wave * cpw;
+    PSum w0, w1;
+    pr_wave_summary<true, false>(x, mask, n, u0, u0 + cpw < nunits ? u0 + cpw : nunits, 1, c, w0, w1);
+    if ((t & 63) == 0) {
+        part[0][wave] = w0;
+        part[1][wave] = w1;
+    }
+    __syncthreads();
+    if ((t & 63) == 0 && wave < 2) {   // a half each
+        PSum r = part[wave][0];
+        for (int w = 1; w < 16; ++w) r = psum_join(r, part[wave][w]);
+        s[wave] = r;
+    }
+    __syncthreads();
+    if (t == 0) {
+        own = chain_derive(s[1], s[0], tmin, tmax, c.level);
+    }
+    if (t == 0 && blockIdx.x == 0) {
+        head->keys0[0] = keys[0][0];
+        head->keys0[1] = keys[0][1];
+        head->xmin = tmin;
+        head->xmax = tmax;
+        head->level = c.level;
+        *ca.level_out = c.level;
+        chain_publish(head, s, own);
+    }
+    __syncthreads();
+    if (own.fast) {
+        const int64_t i = (int64_t)blockIdx.x * 1024 + t;
+        if (i < n) {
+            const double v = c.rescale(x[i]);
+            const bool ocean = v <= c.level;
+            const double r = ocean ? pr_power_map(v, own.lo1, own.r1, 0.5)
+                                   : pr_power_map(v, own.lo0, own.r0, 2.0);
+            h[i] = split_rescale(r - c.level, own.h4min, own.h4max, ca.lower, ca.upper, zero);
+            mask[i] = ocean ? 1 : 0;
+        }
+    } else if (blockIdx.x == 0) {
+        // a thread's values stay its own from pass to pass
+        auto pass = [&](const double *from, unsigned long long (&k)[2], auto &&f) {
+            unsigned long long a = ~0ull, b = 0ull;
+            for (int64_t i = t; i < n; i += 1024) {
+                const double r = f(i, from[i]);
+                h[i] = r;
+                const unsigned long long q = dkey(r);
+                a = q < a ? q : a;
+                b = q > b ? q : b;
+            }
+            minmax(a, b, k);
+        };
+        double lower = tmax, upper = tmin;
+        psum_bounds(s[1], tmin, tmax, lower, upper);
+        pass(x, keys[1], [&](int64_t i, double v) {
+            v = c.rescale(v);
+            mask[i] = v <= c.level ? 1 : 0;
+            if (!mask[i]) return v;
+            zero = zero | (upper - lower == 0.0);
+            return pr_power_map(v, lower, upper - lower, 0.5);
+        });
+        const double m1 = dunkey(keys[1][0]), x1 = dunkey(keys[1][1]);
+        lower = x1;
+        upper = m1;
+        psum_bounds(s[0], m1, x1, lower, upper);
+        pass(h, keys[2], [&](int64_t i, double v) {
+            if (!mask[i]) {
+                zero = zero | (upper - lower == 0.0);
+                v = pr_power_map(v, lower, upper - lower, 2.0);
+            }
+            return v - c.level;
+        });
+        double m2 = dunkey(keys[2][0]), x2 = dunkey(keys[2][1]);
+        if (isnan(m2) || isnan(x2)) m2 = x2 = isnan(m2) ? m2 : x2;   // as k_rescale_ex
+        for (int64_t i = t; i < n; i += 1024)
+            h[i] = split_rescale(h[i], m2, x2, ca.lower, ca.upper, zero);
+    }
+    if (__any(zero) && (t & 63) == 0)
+        __hip_atomic_fetch_or(err, NX_ERR_DIV0_BIT, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 static size_t a256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 // Summary blocks: at most kPrMaxBlocks; each wave takes a contiguous run of
@@ -1196,6 +1354,13 @@ constexpr int64_t kChainBlocks = 1664;
 constexpr int64_t kJoinMax = 32;
 static_assert(sizeof(PSum) * 2 * kChainBlocks + 16 * kMaxRec <= sizeof(PSum) * 2 * kPrMaxBlocks,
               "records beside the summaries");
+// The heights of a small chain stand where the summaries of a larger one do.
+static_assert(sizeof(double) * kSmallChain + 16 * kMaxRec <= sizeof(PSum) * 2 * kPrMaxBlocks,
+              "records beside the heights");
+static double *small_heights(nx_ctx *ctx, int64_t n, void *ws)
+{
+    return ctx->chain_passes == 2 && n <= kSmallChain ? (double *)((char *)ws + 256) : nullptr;
+}
 static unsigned long long *chain_records(void *ws)
 {
     return (unsigned long long *)((char *)ws + 256 + sizeof(PSum) * 2 * kPrMaxBlocks) - 2 * kMaxRec;
@@ -1259,8 +1424,8 @@ int power_rescale(nx_ctx *ctx, const double *x, const uint8_t *mask, int64_t n, 
     const PrGrid g = pr_grid(ctx, n, pr_blocks_per_cu<false, false>());
     const unsigned grid = red_grid(ctx, n);
     hipLaunchKernelGGL(k_minmax_init, dim3(1), dim3(64), 0, stream, head->keys0);
-    hipLaunchKernelGGL(k_minmax, dim3(mm_grid(ctx, n)), dim3(kMinmaxThreads), 0, stream, x, n, head->keys0,
-                       vec16(x), (unsigned long long *)nullptr);
+    hipLaunchKernelGGL(k_minmax<>, dim3(mm_grid(ctx, n)), dim3(kMinmaxThreads), 0, stream, x, n, head->keys0,
+                       vec16(x), (unsigned long long *)nullptr, (double *)nullptr);
     hipLaunchKernelGGL((k_pr_summary<false, false>), dim3((unsigned)g.blocks), dim3(kPrThreads), 0,
                        stream, const_cast<double *>(x), const_cast<uint8_t *>(mask), n, g.nunits,
                        g.cpw, pr_vec(x, mask), sum, head, ChainArgs{0.0, 0.0, 0.0, nullptr},
@@ -1293,7 +1458,8 @@ int power_rescale(nx_ctx *ctx, const double *x, const uint8_t *mask, int64_t n, 
 
 size_t height_chain_workspace_bytes(int64_t n) { return power_rescale_workspace_bytes(n); }
 
-// The chain after the nrec block records of the min/max of h.
+// The chain after the nrec block records of the min/max of h (of
+// small_heights where it gives a place for them).
 static int chain_after_keys(nx_ctx *ctx, int nrec, double *h, int64_t n, double min_alt, double max_alt,
                             double ocean_percent, uint8_t *mask, double *level, void *ws,
                             hipStream_t stream)
@@ -1308,7 +1474,13 @@ static int chain_after_keys(nx_ctx *ctx, int nrec, double *h, int64_t n, double 
     const unsigned grid = red_grid(ctx, n);
     const ChainArgs ca{min_alt, max_alt, ocean_percent, level};
     const int vsum = pr_vec(h, mask), vmap = vec16(h) & vec2(mask);
-    if (ctx->chain_passes == 2) {
+    if (double *x = small_heights(ctx, n, ws)) {
+        hipLaunchKernelGGL(k_chain_small, dim3((unsigned)((n + 1023) / 1024)), dim3(1024), 0, stream, x,
+                           h, mask, n, head, ca, ctx->d_err, rec, nrec);
+        NX_HIP(hipGetLastError());
+        return NX_OK;
+    }
+    if (two) {
         // The summary pass, the join and derivation, then the writing pass;
         // the last two of the five-pass kernels after it return at once when
         // head->fast, else continue from the heights after the ocean's map
@@ -1362,8 +1534,9 @@ int height_chain(nx_ctx *ctx, double *h, int64_t n, double min_alt, double max_a
     NX_HIP(hipSetDevice(ctx->device));
     const unsigned blocks = mm_grid(ctx, n);
     if (blocks > (unsigned)kMaxRec) return set_error(NX_EINVAL, "%u min/max blocks", blocks);
-    hipLaunchKernelGGL(k_minmax, dim3(blocks), dim3(kMinmaxThreads), 0, stream, h, n,
-                       (unsigned long long *)nullptr, vec16(h), chain_records(ws));
+    double *copy = small_heights(ctx, n, ws);
+    hipLaunchKernelGGL((copy ? k_minmax<true> : k_minmax<>), dim3(blocks), dim3(kMinmaxThreads), 0, stream,
+                       (const double *)h, n, (unsigned long long *)nullptr, vec16(h), chain_records(ws), copy);
     return chain_after_keys(ctx, (int)blocks, h, n, min_alt, max_alt, ocean_percent, mask, level, ws, stream);
 }
 
@@ -1378,7 +1551,8 @@ int terrain_heights(nx_ctx *ctx, const double *verts, int64_t V, const int32_t *
     if (rc) return rc;
     NX_HIP(hipSetDevice(ctx->device));
     int nrec = kMaxRec;
-    rc = sample_octaves_keys(ctx, verts, V, perm, pgi, n_oct, rough, strength, radius, h, 0,
+    double *x = small_heights(ctx, V, ws);
+    rc = sample_octaves_keys(ctx, verts, V, perm, pgi, n_oct, rough, strength, radius, x ? x : h, 0,
                              nullptr, nullptr, chain_records(ws), &nrec, stream);
     if (rc) return rc;
     return chain_after_keys(ctx, nrec, h, V, min_alt, max_alt, ocean_percent, mask, level, ws, stream);

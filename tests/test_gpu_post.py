@@ -350,3 +350,21 @@ def test_terrain_heights_fused_equals_two_calls(oracle):
     assert lv.item() == ref_level
     assert np.array_equal(m.cpu().numpy().astype(bool), ref_mask)
     assert np.abs(h.cpu().numpy() - ref_h).max() <= 64 * EPS * (8850.0 + 4000.0)
+
+
+@pytest.mark.parametrize("n", [1, 2, 1024, 10_242, 16_384, 16_385])
+@pytest.mark.parametrize("case", ["normal", "two_values", "one_nan"])
+def test_small_chain_in_one_block(n, case):
+    """Up to 16,384 heights take the whole chain in one block, with the
+    five-pass steps inside it where the derivation does not hold: bit for bit
+    the five-pass form's results on both sides of the limit, NaN included,
+    and the same errors."""
+    x = np.random.default_rng(n).standard_normal(n)
+    if case == "two_values":
+        x = (np.arange(n) % 2).astype(np.float64)
+    elif case == "one_nan":
+        x[n // 2] = np.nan
+    print("small chain", n, case, flush=True)
+    (h2, m2, l2, e2, _), (h5, m5, l5, e5, _) = _chain_both_forms(x)
+    assert np.array_equal(h2, h5, equal_nan=True) and np.array_equal(m2, m5) and e2 is e5
+    assert np.array_equal([l2], [l5], equal_nan=True)
