@@ -310,13 +310,13 @@ __device__ __forceinline__ void batch_tile(double2 *A, double2 *B, double2 *hw0,
     if constexpr (K == 2)
         erode_tile_pair<1024, true>(A, B, hw0, hw1, s0, s1, p, plan, tile, rain_mid, rain_next);
     else
-        erode_tile_quad<3, NS>(A, B, hw0, hw1, s0, s1, p, plan, tile, rain_mid, rain_next);
+        erode_tile_quad<3, NS>(A, B, hw0, hw1, s0, s1, p, plan, quad_tile(plan, tile), rain_mid, rain_next);
 }
 
 template <int K>
 struct TileLds {
     static constexpr int kA = K == 2 ? kLoadMax : kQuadLoadMax;
-    static constexpr int kB = K == 2 ? kStepOneMax : kQuadStepOne;
+    static constexpr int kAll = K == 2 ? kLoadMax + kStepOneMax : kQuadLds;
 };
 
 // A launch that covers one planet takes the single-planet kernel's
@@ -332,8 +332,8 @@ __global__ __launch_bounds__(1024) void k_erode_batch_tile_one(const ErosionMeta
                                                                TilePlanDev plan, int tail, int64_t k,
                                                                int64_t total_iters, double rain)
 {
-    __shared__ double2 A[TileLds<K>::kA];
-    __shared__ double2 B[TileLds<K>::kB];
+    __shared__ double2 A[TileLds<K>::kAll];
+    double2 *const B = A + TileLds<K>::kA;
     const int64_t tile = xcd_tile(blockIdx.x, plan.ntiles);
     if (tile >= plan.ntiles) return;
     const ErosionMeta m = *meta;
@@ -367,8 +367,8 @@ template <int K, int NS>
 __global__ __launch_bounds__(1024) void k_erode_batch_tile_args(const TileLaunchArgs a,
                                                                 int32_t nt_total, int64_t k)
 {
-    __shared__ double2 A[TileLds<K>::kA];
-    __shared__ double2 B[TileLds<K>::kB];
+    __shared__ double2 A[TileLds<K>::kAll];
+    double2 *const B = A + TileLds<K>::kA;
     const int b = (int)xcd_tile(blockIdx.x, nt_total);
     if (b >= nt_total) return;
     // b and the prefix entries lie in [0, 2^31): b - prefix[q] is negative,
@@ -394,8 +394,8 @@ __global__ __launch_bounds__(1024) void k_erode_batch_tile(const BatchPlanetDev 
                                                            int active, int64_t nt_total,
                                                            int64_t k)
 {
-    __shared__ double2 A[TileLds<K>::kA];
-    __shared__ double2 B[TileLds<K>::kB];
+    __shared__ double2 A[TileLds<K>::kAll];
+    double2 *const B = A + TileLds<K>::kA;
     const int64_t b = xcd_tile(blockIdx.x, nt_total);
     if (b >= nt_total) return;
     // The planet is the same for the whole block: keep its descriptor in

@@ -159,12 +159,13 @@ __global__ __launch_bounds__(1024) void k_erode_quad(ErosionMeta *__restrict__ m
                                                        int64_t done, double rain_first,
                                                        double rain_mid, double rain_next)
 {
-    __shared__ double2 A[kQuadLoadMax];
-    __shared__ double2 B[kQuadStepOne];
-    const int p = launch_buffer(meta, j, done);
-    const int64_t tile = xcd_tile(blockIdx.x, P.ntiles);
+    __shared__ double2 A[kQuadLds];
+    double2 *const B = A + kQuadLoadMax;
+    const int64_t tile = xcd_tile(blockIdx.x, P.ntiles);   // block 0's is 0
     if (tile >= P.ntiles) return;
-    erode_tile_quad<RULE, NS, FIRST>(A, B, hw0, hw1, s0, s1, p, P, tile, rain_mid,
+    const QuadTile q = quad_tile(P, tile);
+    const int p = launch_buffer(meta, j, done);
+    erode_tile_quad<RULE, NS, FIRST>(A, B, hw0, hw1, s0, s1, p, P, q, rain_mid,
                               rain_next, rain_first);
 }
 

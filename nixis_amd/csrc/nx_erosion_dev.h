@@ -74,19 +74,32 @@ NX_EHD void erode_accumulate(double h, double hn, double wn, double d, double &S
 // slope has the difference's sign and comparing the heights gives it.
 constexpr double kCompare = 0x1p-940;
 
+// x with its sign turned over where diff's is set.
+NX_EHD double turn_sign(double x, double diff)
+{
+    const uint64_t u = __builtin_bit_cast(uint64_t, x), v = __builtin_bit_cast(uint64_t, diff);
+#if defined(__HIP_DEVICE_COMPILE__)
+    // one instruction, hi ^ (diff's hi & the sign bit): 1% of a d=1000 launch
+    const uint32_t hi = __builtin_amdgcn_bitop3_b32((uint32_t)(u >> 32), (uint32_t)(v >> 32), 0x80000000u, 0x78);
+    return __builtin_bit_cast(double, (uint64_t)hi << 32 | (uint32_t)u);
+#else
+    return __builtin_bit_cast(double, u ^ (v & 0x8000000000000000ull));
+#endif
+}
+
 // erode_accumulate for |h| >= kCompare: the products take the difference's
 // sign (S - t is S + -t, and -w k is -(w k)), so one comparison and two sums
 // serve both directions.
 template <int RULE = 3>
 NX_EHD void erode_compare(double h, double hn, double wn, double d, double &S, double &W)
 {
-    const uint64_t down = __builtin_bit_cast(uint64_t, hn - h) & 0x8000000000000000ull;
+    const double down = hn - h;
     double ts, tw;
     if (RULE == 4) {
-        ts = __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, max0(kSol * wn)) ^ down);
-        tw = __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, max0(wn * d)) ^ down);
+        ts = turn_sign(max0(kSol * wn), down);
+        tw = turn_sign(max0(wn * d), down);
     } else {
-        const double w = __builtin_bit_cast(double, __builtin_bit_cast(uint64_t, wn) ^ down);
+        const double w = turn_sign(wn, down);
         ts = kSol * w;
         tw = w * d;
     }

@@ -35,6 +35,7 @@ constexpr int kLoadMaxMulti = 3072; // tile + its kMultiSteps rings
 constexpr int kQuadStepOne = 2048;
 static_assert(16 * 2688 <= 65536, "a staged vertex's byte offset fits 16 bits");
 constexpr int kQuadLoadMax = 2688;
+constexpr int kQuadLds = kQuadLoadMax + kQuadStepOne;   // the block's LDS, both buffers
 constexpr int kQuadChunk = 1152;
 // Default chunk of a four-step plan over V vertices.  A launch takes as long
 // as its fullest CU: up to about two tiles per CU of kCus, the tiles are made
@@ -347,13 +348,44 @@ __device__ __forceinline__ void erode_tile_multi(double2 *A, double2 *hw0, doubl
     }
 }
 
-// Four steps of tile `tile` (a four-step plan within kQuadStepOne and
+// What a block reads of a four-step plan's tables for its tile, loaded
+// together before anything else waits for memory.
+struct QuadTile {
+    int64_t rbase, cbase, ebase;
+    int a, T, c3, c2, c1, L, nl;   // pref: tile + ring 1, .. + ring 4; nl lengths
+};
+__device__ __forceinline__ QuadTile quad_tile(const TilePlanDev &P, int64_t tile)
+{
+    QuadTile q;
+    const auto start = gmem(P.start) + tile, pref = gmem(P.pref) + tile * (kMultiSteps + 1);
+    const auto ebase = gmem(P.ebase) + tile;
+    q.a = start[0];
+    const int end = start[1];
+    q.c3 = pref[1];
+    q.c2 = pref[2];
+    q.c1 = pref[3];
+    q.L = pref[4];
+    q.rbase = gmem(P.rbase)[tile];
+    q.cbase = gmem(P.cbase)[tile];
+    q.ebase = ebase[0];
+    const int64_t eend = ebase[1];
+    asm volatile("" ::: "memory");
+    q.T = end - q.a;
+    q.nl = (int)(eend - q.ebase);
+    return q;
+}
+
+// Four steps of a tile q of plan P (a four-step plan within kQuadStepOne and
 // kQuadLoadMax) by a 1024-thread block, reading buffer p and writing p ^ 1.
 // Each thread keeps up to two first-step vertices (li and li + 1024): their
-// sediment, neighbours (LDS byte offsets, two to a word) and edge lengths are loaded
-// before the first barrier, while the field gathers are in flight, and stay
-// in registers for all four steps.  h and w of the tile and its four rings
-// are staged in A; step 1 (tile + rings 1..3) writes B, step 2 (tile + rings
+// sediment, neighbours (LDS byte offsets, two to a word) and edge lengths
+// stay in registers for all four steps.  The lengths come through the LDS
+// that the fields take afterwards, in 16-byte lines: gathered from memory by
+// slot code, 12 loads a thread over scattered lines, they kept the CU's
+// return path busy for 84% of the launch (10,000,002 vertices: 308 us, 276 in
+// this form; 1,024,002: 39 and 34).  What bounds it now is memory: 1.15 GB a
+// launch, 235 us at the rate of a large copy.  h and w of the tile and its four
+// rings are staged in A; step 1 (tile + rings 1..3) writes B, step 2 (tile + rings
 // 1..2) A, step 3 (tile + ring 1) B, and step 4 writes the tile: one barrier
 // between steps.  Every vertex is computed from the same inputs with the
 // same arithmetic as by one-step launches, so the results are bit for bit
@@ -365,7 +397,7 @@ __device__ __forceinline__ void erode_tile_multi(double2 *A, double2 *hw0, doubl
 template <int RULE = 3, int NS = 4, bool FIRST = false>
 __device__ __forceinline__ void erode_tile_quad(double2 *A, double2 *B, double2 *hw0, double2 *hw1,
                                                 double *s0, double *s1, int p,
-                                                const TilePlanDev &P, int64_t tile,
+                                                const TilePlanDev &P, const QuadTile &Q,
                                                 double rain_mid, double rain_next,
                                                 double rain_first = 0.0)
 {
@@ -375,52 +407,95 @@ __device__ __forceinline__ void erode_tile_quad(double2 *A, double2 *B, double2 
     const auto s_src = gmem(p ? s1 : s0);
     const auto hw_dst = gmem(p ? hw0 : hw1);
     const auto s_dst = gmem(p ? s0 : s1);
-    const int64_t a = gmem(P.start)[tile];
-    const int T = (int)(gmem(P.start)[tile + 1] - a);
-    const auto pref = gmem(P.pref) + tile * (kMultiSteps + 1);
+    const int a = Q.a, T = Q.T;
     static_assert(NS >= 2 && NS <= kMultiSteps, "2..4 steps");
-    const int c3 = pref[1], c2 = pref[2], c1 = pref[3], L = pref[4];
+    const int c3 = Q.c3, c2 = Q.c2, c1 = Q.c1, L = Q.L, nl = Q.nl;
     // first-step set and staged set of this launch; slot codes and lengths
     // keep the plan's layout over the c1 first-step vertices
     const int cf = NS == 4 ? c1 : NS == 3 ? c2 : c3;
     const int cl = NS == 4 ? L : NS == 3 ? c1 : c2;
-    const auto ring = gmem(P.ring) + gmem(P.rbase)[tile];
-    const int64_t cb = gmem(P.cbase)[tile];
-    const auto lcol = gmem(P.lcol) + 6 * cb;
-    const auto lel = gmem(P.lel) + gmem(P.ebase)[tile];
+    const auto ring = gmem(P.ring) + Q.rbase;
+    const auto lcol = gmem(P.lcol) + 6 * Q.cbase;
+    const auto lel = gmem(P.lel) + Q.ebase;
 
-    for (int li = threadIdx.x; li < cl; li += TH) {
-        double2 v = hw_src[li < T ? a + li : ring[li - T]];
-        if (FIRST) v.y = v.y + rain_first;
-        A[li] = v;
+    // The lengths come through LDS, read from memory in whole 16-byte lines
+    // (from the line the block begins in), while the field gathers are in flight;
+    // a block that does not fit is gathered from memory.
+    using Line = uint32_t __attribute__((ext_vector_type(4)));
+    constexpr int kLoadPer = (kQuadLoadMax + TH - 1) / TH, kLenPer = 3;
+    const int lsh = (int)(Q.ebase & 1), ln = (nl + lsh + 1) / 2;
+    const bool staged = ln <= kQuadLds;
+    const auto lsrc = (decltype(gmem((const Line *)nullptr)))(lel - lsh);
+    Line *const lines = (Line *)A;
+    const double *const ls = (const double *)A + lsh;
+
+    int at[kLoadPer], code[kPer][6];
+#pragma unroll
+    for (int m = 0; m < kLoadPer; ++m) {
+        const int li = threadIdx.x + m * TH;
+        at[m] = li >= T && li < cl ? ring[li - T] : a + li;
     }
-    double sed[kPer];
-    int code[kPer][6];
 #pragma unroll
     for (int m = 0; m < kPer; ++m) {
         const int li = threadIdx.x + m * TH;
-        sed[m] = 0.0;
         if (li < cf) {
-            sed[m] = s_src[li < T ? a + li : ring[li - T]];
 #pragma unroll
             for (int q = 0; q < 6; ++q) code[m][q] = lcol[q * c1 + li];
         }
     }
-    // the code loads go out together, before any length's address depends on one
+    Line lv[kLenPer];
+    if (staged) {
+#pragma unroll
+        for (int m = 0; m < kLenPer; ++m) {
+            const int i = threadIdx.x + m * TH;
+            lv[m] = i < ln ? (Line)lsrc[i] : (Line)0;
+        }
+    }
     asm volatile("" ::: "memory");
+    double h[kLoadPer], w[kLoadPer], sed[kPer];
+#pragma unroll
+    for (int m = 0; m < kLoadPer; ++m) {
+        const int li = threadIdx.x + m * TH;
+        const double2 v = li < cl ? (double2)hw_src[at[m]] : make_double2(0.0, 0.0);
+        h[m] = v.x;
+        w[m] = v.y;
+        if (m < kPer) sed[m < kPer ? m : 0] = li < cf ? s_src[at[m]] : 0.0;
+    }
+    asm volatile("" ::: "memory");
+    if (staged) {
+#pragma unroll
+        for (int m = 0; m < kLenPer; ++m) {
+            const int i = threadIdx.x + m * TH;
+            if (i < ln) lines[i] = lv[m];
+        }
+        for (int i = threadIdx.x + kLenPer * TH; i < ln; i += TH) lines[i] = lsrc[i];
+        __syncthreads();
+    }
     uint32_t nbp[kPer][3];
     double len[kPer][6];
 #pragma unroll
     for (int m = 0; m < kPer; ++m) {
         const int li = threadIdx.x + m * TH;
         if (li < cf) {
+            if (staged) {
 #pragma unroll
-            for (int q = 0; q < 6; ++q) len[m][q] = slot_len(code[m][q], li, c1, T, lel);
+                for (int q = 0; q < 6; ++q) len[m][q] = slot_len(code[m][q], li, c1, T, ls);
+            } else {
+#pragma unroll
+                for (int q = 0; q < 6; ++q) len[m][q] = slot_len(code[m][q], li, c1, T, lel);
+            }
 #pragma unroll
             for (int q = 0; q < 3; ++q)
                 nbp[m][q] = (uint32_t)slot_nbr(code[m][2 * q]) << 4 |
                             (uint32_t)slot_nbr(code[m][2 * q + 1]) << 20;
         }
+    }
+    if (staged) __syncthreads();
+#pragma unroll
+    for (int m = 0; m < kLoadPer; ++m) {
+        const int li = threadIdx.x + m * TH;
+        if (FIRST) w[m] = w[m] + rain_first;
+        if (li < cl) A[li] = make_double2(h[m], w[m]);
     }
     __syncthreads();
 

@@ -158,3 +158,46 @@ def test_slot_update_at_the_comparison_edges(oracle, rule, kind, radius):
             nan = np.isnan(r)
             assert np.array_equal(nan, np.isnan(a))
             assert np.array_equal(a[~nan].view(np.int64), r[~nan].view(np.int64))
+
+
+@pytest.mark.parametrize("rule", [3, 4])
+def test_length_blocks_of_every_size(rule):
+    """Four-step launches stage a tile's length block in LDS line by line, from
+    either half of a 16-byte line, in rounds of 6,144 lengths, up to 9,472; a
+    larger one is gathered.  Blocks padded to those edges give the steps of
+    the plan as it was built bit for bit, tails included."""
+    pts, nb, h = _planet(26)
+    rng = np.random.default_rng(3)
+    w, s = rng.uniform(0, 1, h.size), rng.uniform(0, 0.02, h.size)
+    g, padded = erosion.ErosionGraph(pts, nb), erosion.ErosionGraph(pts, nb)
+    assert g.plan.steps == 4
+    plan, img = padded.plan, padded._plan_blob.cpu().numpy()
+    nt = int(plan.ntiles)
+    eb = img[plan.off_ebase:plan.off_ebase + 8 * (nt + 1)].view(np.int64)
+    sizes = [0, 6143, 6144, 6145, 9471, 9472, 9473, 12001]
+    out = [np.maximum(n, sizes[t % len(sizes)]) for t, n in enumerate(np.diff(eb))]
+    neb = np.concatenate([[0], np.cumsum(out)]).astype(np.int64)
+    assert neb[-1] > 9473 * 2 and (neb[:-1] & 1).any()
+    lel = np.zeros(neb[-1] + 32)
+    old = img[plan.off_lel:plan.off_lel + 8 * eb[-1]].view(np.float64)
+    for t in range(nt):
+        lel[neb[t]:neb[t] + eb[t + 1] - eb[t]] = old[eb[t]:eb[t + 1]]
+    at = [int(plan.bytes), int(plan.bytes) + -(-lel.nbytes // 256) * 256]
+    new = np.zeros(at[1] + neb.nbytes, np.uint8)
+    new[:img.size] = img
+    new[at[0]:at[0] + lel.nbytes] = lel.view(np.uint8)
+    new[at[1]:] = neb.view(np.uint8)
+    plan.off_lel, plan.off_ebase, plan.bytes = at[0], at[1], new.size
+    padded._set_plan(plan, torch.from_numpy(new).cuda())
+    for n in (2, 3, 4, 9):
+        got = []
+        for q in (g, padded):
+            st = erosion.ErosionState(q.V)
+            st.load(*[torch.from_numpy(q.permute(a)).cuda() for a in (h, w, s)])
+            st.run(q, n, 0.3 / 320, rule=rule)
+            res = [torch.empty(q.V, dtype=torch.float64, device="cuda") for _ in range(3)]
+            st.store(*res)
+            st.ctx.sync_check()
+            got.append(res)
+        for a, b in zip(*got):
+            assert torch.equal(a, b)
