@@ -300,7 +300,8 @@ def stream_ptr(stream=None):
     """hipStream_t of a torch stream (default: the current stream)."""
     import torch
     if stream is None:
-        stream = torch.cuda.current_stream()
+        # the handle without a Stream object: 0.5 us of host time instead of 3
+        return _c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
     return _c_void_p(stream.cuda_stream)
 
 

@@ -41,10 +41,10 @@ constexpr int kQuadChunk = 1152;
 // as its fullest CU: up to about two tiles per CU of kCus, the tiles are made
 // equal in size and just enough to go round the CUs once, or twice (2% over,
 // for the shorter last one), which measured faster than fewer, full tiles at
-// 64 to 200 divisions (us per step: 41k vertices 2.0 against 3.4, 100k 2.5
-// against 3.4, 225k 3.4 against 3.5, 400k 5.0 against 5.5); beyond two rounds
-// of two tiles per CU full tiles win (1000 divisions: 79.8, 81.6 at 1024, 101
-// at 512).  Below kQuadSmall the rings outgrow the tiles.
+// 64 to 300 divisions (us per step: 41k vertices 1.6 against 2.6, 225k 2.6
+// against 2.8, 400k 4.3 against 4.6, 900k 7.4 against 7.7); beyond two rounds
+// of two tiles per CU full tiles win (1000 divisions: 64.7, 66.1 at 1024, 67.7
+// at 1280).  Below kQuadSmall the rings outgrow the tiles.
 constexpr int kCus = 256;
 constexpr int kQuadSmall = 256;
 inline int quad_chunk(int64_t V)
