@@ -164,7 +164,9 @@ class MeshCache:
             if tuning is None:
                 from . import autotune
                 tuning = autotune.lookup_erosion(10 * d * d + 2)
-            kw = tuning.graph_kwargs() if tuning is not None else {"chunk": BATCH_CHUNK}
+            kw = tuning.graph_kwargs() if tuning is not None else {"chunk": 0}
+            if kw.get("steps", 4) == 4:
+                kw["chunk"] = kw["chunk"] or BATCH_CHUNK
             g = self._build_graph(d, **kw)
             self._graphs[d] = g
         return g

@@ -413,8 +413,14 @@ __global__ __launch_bounds__(1024) void k_erode_batch_tile(const BatchPlanetDev 
     const TilePlanDev plan = D.plan;
     double2 *hw0 = D.hw0, *hw1 = D.hw1;
     double *s0 = D.s0, *s1 = D.s1;
-    batch_tile<K, NS>(A, B, hw0, hw1, s0, s1, D.meta->it, D.meta->buf, plan, D.tail_steps,
-                      D.total_iters, D.rain, b - prefix[r], k);
+    // the step counter in scalar registers too: in vector ones the four-step
+    // kernels need more than 64 and a CU holds one block instead of two
+    const int64_t it = gmem(D.meta)->it;
+    const int64_t t = (int64_t)((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(it >> 32)) << 32 |
+                                (uint32_t)__builtin_amdgcn_readfirstlane((int)it));
+    const int buf = __builtin_amdgcn_readfirstlane(gmem(D.meta)->buf);
+    batch_tile<K, NS>(A, B, hw0, hw1, s0, s1, t, buf, plan, D.tail_steps, D.total_iters, D.rain,
+                      b - prefix[r], k);
 }
 
 // The three launch forms of one tile phase.

@@ -53,7 +53,7 @@ struct nx_ctx {
     unsigned long long *d_keys = nullptr;  // kKeySlots x 2 reduction keys
     std::atomic<unsigned> key_slot{0};
     hipStream_t capture_stream = nullptr;  // default priority, graph capture only
-    int graph_chunk = 32;                  // erosion steps per captured graph; 0 = eager
+    int graph_chunk = 32;                  // erosion steps per captured graph without a plan; 0 = eager
     int pair_variant = 0;                  // two-step kernel variant (0 = default)
     int multi_variant = 0;                 // four-step kernel variant (0 = default)
     int chain_passes = 2;                  // height chain: 2 (default) or the five-pass form

@@ -31,7 +31,7 @@ constexpr int kLoadMaxMulti = 3072; // tile + its kMultiSteps rings
 // Four-step plans keep the first step's vertices (tile + rings 1..3) within
 // kQuadStepOne, two per thread of a 1024-thread block, and tile + rings
 // 1..4 within kQuadLoadMax, so that both LDS buffers of erode_tile_quad fit
-// two blocks per CU; they start from tiles of kQuadChunk vertices.
+// two blocks per CU; they start from tiles of quad_chunk vertices.
 constexpr int kQuadStepOne = 2048;
 static_assert(16 * 2688 <= 65536, "a staged vertex's byte offset fits 16 bits");
 constexpr int kQuadLoadMax = 2688;

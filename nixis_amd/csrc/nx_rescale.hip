@@ -3,13 +3,13 @@
 // (terrain.py:61-72), power_rescale (util.py:178-254) and the chain of
 // nixis.py:330-364.
 //
-// Min/max reductions run per block and end in one atomic per block on an
-// order-preserving integer encoding of the doubles; the maps then use the
+// Min/max reductions run per block on an order-preserving integer encoding of
+// the doubles and end in one atomic per block, or in the chain in a record per
+// block that the next kernel joins; the maps then use the
 // reference's FP64 operation order (IEEE division, no contraction), so
 // rescale and the mask are bit-identical to the reference.  power_rescale's
-// bounds follow the reference's sequential if/elif loop exactly, through an
-// exclusive min-scan of the selected values (the running minimum each
-// element was compared with).
+// bounds follow the reference's sequential if/elif loop exactly, from
+// in-order summaries of the selected values.
 #include <hip/hip_runtime.h>
 
 #include <atomic>
