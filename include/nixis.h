@@ -206,9 +206,10 @@ int nx_terrain_heights_noalloc(nx_ctx *ctx, const double *verts, int64_t V,
  * KDTree returns them: dists = sqrt of the squared differences summed in
  * x, y, z order (f64), nbrs = point indices (int64); equal distances are
  * ordered by index.  Where fewer than k points exist the rest is +inf / V.
- * The structure is a uniform grid of cells in a device workspace of
- * nx_knn_grid_bytes(V) bytes (256-byte aligned): points sorted by cell and
- * a hash table of occupied cells.  1 <= k <= 8, V < 2^31 - 1. */
+ * The structure is a set of bins in a device workspace of
+ * nx_knn_grid_bytes(V) bytes (256-byte aligned): bands of latitude cut into
+ * cells for points around a sphere, hashed cubes for any others.
+ * 1 <= k <= 8, V < 2^31 - 1. */
 size_t nx_knn_grid_bytes(int64_t V);
 int nx_knn_grid_build(nx_ctx *ctx, const double *points, int64_t V,
                       void *grid, void *stream);
@@ -247,8 +248,11 @@ int nx_make_gray_array(nx_ctx *ctx, int64_t npix, int k, const double *dists,
  * coordinates are device f64 [V][3]; results are device float32, summed as
  * numba adds a double to a float32 element (double sum, rounded to float).
  * The rotation, tilt and seasonal sines and cosines come from the host C
- * library; per-vertex asin / atan2 / cos run on the device, so values agree
- * with the reference's to a few float32 ulp per summed step.
+ * library; the reference's per-vertex asin, atan2 and cosines are taken as
+ * products of the rotated vector's components (FP64) where its length is the
+ * radius, so values agree with the reference's to a few float32 ulp per
+ * summed step.  A year is the sum of the days' tables in FP64, interpolated
+ * once per vertex.
  * ws: nx_climate_workspace_bytes() of 256-byte aligned device memory. */
 size_t nx_climate_workspace_bytes(void);
 /* climate.py:416-446 (sample_insolation) for nsteps (<= 360) rotations from

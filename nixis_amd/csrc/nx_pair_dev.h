@@ -383,8 +383,8 @@ __device__ __forceinline__ QuadTile quad_tile(const TilePlanDev &P, int64_t tile
 // that the fields take afterwards, in 16-byte lines: gathered from memory by
 // slot code, 12 loads a thread over scattered lines, they kept the CU's
 // return path busy for 84% of the launch (10,000,002 vertices: 308 us, 276 in
-// this form; 1,024,002: 39 and 34).  What bounds it now is memory: 1.15 GB a
-// launch, 235 us at the rate of a large copy.  h and w of the tile and its four
+// this form; 1,024,002: 39 and 34).  What bounds it now is memory: 1.18 GB a
+// launch, 239 us at the rate of a large copy.  h and w of the tile and its four
 // rings are staged in A; step 1 (tile + rings 1..3) writes B, step 2 (tile + rings
 // 1..2) A, step 3 (tile + ring 1) B, and step 4 writes the tile: one barrier
 // between steps.  Every vertex is computed from the same inputs with the
