@@ -1223,7 +1223,7 @@ __global__ __launch_bounds__(kFinalThreads) void k_chain_final(double *h, uint8_
 // The whole chain of few heights (n <= kSmallChain) in one launch: a launch
 // costs the host about 5 us, so four of them outlast the work (with the noise,
 // 642 heights: 29.3 us a call, 21.5 in this form; 10,242: 29.6 and 21.6;
-// 16,002: 29.5 and 23.0).  The
+// 16,002: 29.5 and 21.2).  The
 // heights come from x, a copy in the workspace, so that every block can
 // summarise all of them for itself while others already write their results;
 // each then maps a run of its own (one block alone took 24 us, bound by its
@@ -1234,14 +1234,15 @@ __global__ __launch_bounds__(kFinalThreads) void k_chain_final(double *h, uint8_
 // ocean and land maps with the shift and the split rescale, with the min/max
 // between them.
 constexpr int64_t kSmallChain = 16384;
-__global__ __launch_bounds__(1024) void k_chain_small(double *x, double *h, uint8_t *mask,
+constexpr int kSmallThreads = 512;   // 14.6 us a launch at 10,242 heights; 15.9 at 1024, 15.3 at 256
+__global__ __launch_bounds__(kSmallThreads) void k_chain_small(double *x, double *h, uint8_t *mask,
                                                       int64_t n, PrHead *__restrict__ head, ChainArgs ca,
                                                       int *__restrict__ err,
                                                       const unsigned long long *__restrict__ rec,
                                                       int nrec)
 {
     __shared__ unsigned long long keys[3][2];
-    __shared__ PSum part[2][16], s[2];
+    __shared__ PSum part[2][kSmallThreads / 64], s[2];
     __shared__ ChainConsts own;
     const int t = threadIdx.x, wave = t >> 6;
     auto minmax = [&](unsigned long long lo, unsigned long long hi, unsigned long long (&k)[2]) {
@@ -1253,7 +1254,7 @@ __global__ __launch_bounds__(1024) void k_chain_small(double *x, double *h, uint
         __syncthreads();
     };
     unsigned long long lo = ~0ull, hi = 0ull;
-    for (int i = t; i < nrec; i += 1024) {
+    for (int i = t; i < nrec; i += kSmallThreads) {
         const unsigned long long a = rec[2 * i], b = rec[2 * i + 1];
         lo = a < lo ? a : lo;
         hi = b > hi ? b : hi;
@@ -1262,7 +1263,7 @@ __global__ __launch_bounds__(1024) void k_chain_small(double *x, double *h, uint
     double tmin, tmax;
     const ChainMap c = chain_map(dunkey(keys[0][0]), dunkey(keys[0][1]), ca, tmin, tmax);
     bool zero = c.xr == 0.0;
-    const int64_t nunits = (n + kPrUnit - 1) / kPrUnit, cpw = (nunits + 15) / 16;
+    const int64_t nunits = (n + kPrUnit - 1) / kPrUnit, cpw = (nunits + kSmallThreads / 64 - 1) / (kSmallThreads / 64);
     const int64_t u0 = wave * cpw;
     PSum w0, w1;
     pr_wave_summary<true, false>(x, mask, n, u0, u0 + cpw < nunits ? u0 + cpw : nunits, 1, c, w0, w1);
@@ -1273,7 +1274,7 @@ __global__ __launch_bounds__(1024) void k_chain_small(double *x, double *h, uint
     __syncthreads();
     if ((t & 63) == 0 && wave < 2) {   // a half each
         PSum r = part[wave][0];
-        for (int w = 1; w < 16; ++w) r = psum_join(r, part[wave][w]);
+        for (int w = 1; w < kSmallThreads / 64; ++w) r = psum_join(r, part[wave][w]);
         s[wave] = r;
     }
     __syncthreads();
@@ -1291,7 +1292,7 @@ __global__ __launch_bounds__(1024) void k_chain_small(double *x, double *h, uint
     }
     __syncthreads();
     if (own.fast) {
-        const int64_t i = (int64_t)blockIdx.x * 1024 + t;
+        const int64_t i = (int64_t)blockIdx.x * kSmallThreads + t;
         if (i < n) {
             const double v = c.rescale(x[i]);
             const bool ocean = v <= c.level;
@@ -1304,7 +1305,7 @@ __global__ __launch_bounds__(1024) void k_chain_small(double *x, double *h, uint
         // a thread's values stay its own from pass to pass
         auto pass = [&](const double *from, unsigned long long (&k)[2], auto &&f) {
             unsigned long long a = ~0ull, b = 0ull;
-            for (int64_t i = t; i < n; i += 1024) {
+            for (int64_t i = t; i < n; i += kSmallThreads) {
                 const double r = f(i, from[i]);
                 h[i] = r;
                 const unsigned long long q = dkey(r);
@@ -1335,7 +1336,7 @@ __global__ __launch_bounds__(1024) void k_chain_small(double *x, double *h, uint
         });
         double m2 = dunkey(keys[2][0]), x2 = dunkey(keys[2][1]);
         if (isnan(m2) || isnan(x2)) m2 = x2 = isnan(m2) ? m2 : x2;   // as k_rescale_ex
-        for (int64_t i = t; i < n; i += 1024)
+        for (int64_t i = t; i < n; i += kSmallThreads)
             h[i] = split_rescale(h[i], m2, x2, ca.lower, ca.upper, zero);
     }
     if (__any(zero) && (t & 63) == 0)
@@ -1475,7 +1476,7 @@ static int chain_after_keys(nx_ctx *ctx, int nrec, double *h, int64_t n, double 
     const ChainArgs ca{min_alt, max_alt, ocean_percent, level};
     const int vsum = pr_vec(h, mask), vmap = vec16(h) & vec2(mask);
     if (double *x = small_heights(ctx, n, ws)) {
-        hipLaunchKernelGGL(k_chain_small, dim3((unsigned)((n + 1023) / 1024)), dim3(1024), 0, stream, x,
+        hipLaunchKernelGGL(k_chain_small, dim3((unsigned)((n + kSmallThreads - 1) / kSmallThreads)), dim3(kSmallThreads), 0, stream, x,
                            h, mask, n, head, ca, ctx->d_err, rec, nrec);
         NX_HIP(hipGetLastError());
         return NX_OK;
