@@ -152,7 +152,8 @@ class ErosionGraph:
         return self
 
     def _build_plan_device(self, stream):
-        """The four-step plan from the device tables; False when refused."""
+        """The four-step plan from the device tables, written before this
+        returns; False when refused."""
         import torch
         L = _lib.lib()
         plan = _lib.NxTilePlan()
@@ -171,8 +172,8 @@ class ErosionGraph:
             _lib.check(rc)
             blob = torch.zeros(plan.bytes, dtype=torch.uint8, device=self.device)
             _lib.check(build(blob, plan.bytes))
-        if stream is not None:
-            ctx.sync_check(stream)
+        # complete on return, as the tables are: a run may be on any stream
+        ctx.sync_check(stream)
         self._set_plan(plan, blob)
         return True
 
