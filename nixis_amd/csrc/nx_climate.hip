@@ -99,15 +99,16 @@ __device__ __forceinline__ double insol_vector(double x, double y, double z, dou
 }
 
 // nsteps rotations of one vertex added to acc, each step as numba adds a
-// double to a float32 element.  Day of 360 steps at d=320 (1,024,002
+// double to a float32 element.  finite: every angle's cosine and sine are (the
+// maximum below takes a NaN for 0).  Day of 360 steps at d=320 (1,024,002
 // vertices): 3215 us a call with the angles, 97 us this way, every float equal.
 __device__ __forceinline__ float insol_sum(double x, double y, double z, double r,
                                            const double *__restrict__ rot, int nsteps, double ct,
-                                           double st, float acc)
+                                           double st, bool finite, float acc)
 {
     const double r2 = r * r, v2 = x * x + y * y + z * z;
     const bool r_ok = r2 >= 0x1p-900 && r2 <= 0x1p900;
-    if (r_ok && fabs(v2 - r2) <= kOnSphere * r2) {
+    if (finite && r_ok && fabs(v2 - r2) <= kOnSphere * r2) {
         const double xs = x * ct / r, ys = -y * ct / r, zs = z * st / r;
 #pragma unroll 4
         for (int s = 0; s < nsteps; ++s) {
@@ -146,13 +147,13 @@ __global__ __launch_bounds__(256) void k_surface_temp(const double *__restrict__
 // nsteps rotations of each vertex, accumulated into arr (float32).
 __global__ __launch_bounds__(256) void k_insolation(const double *__restrict__ verts, int64_t V,
                                                     double radius, const double *__restrict__ rot,
-                                                    int nsteps, double ct, double st,
+                                                    int nsteps, double ct, double st, int finite,
                                                     float *__restrict__ arr)
 {
     const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (v >= V) return;
     arr[v] = insol_sum(verts[3 * v], verts[3 * v + 1], verts[3 * v + 2], radius, rot, nsteps, ct,
-                       st, arr[v]);
+                       st, finite != 0, arr[v]);
 }
 
 // climate.py:503-533 for one tilt: table[k] over the 181 slice vertices, 360
@@ -164,7 +165,7 @@ __global__ __launch_bounds__(64) void k_slice(const double *__restrict__ sverts,
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= kSlice) return;
     table[k] = insol_sum(sverts[3 * k], sverts[3 * k + 1], sverts[3 * k + 2], radius, rot, nsteps,
-                         ct, st, 0.0f);
+                         ct, st, ct == ct, 0.0f);
 }
 
 // The year's table: a block per slice vertex, a thread per day (the daily
@@ -182,7 +183,7 @@ __global__ __launch_bounds__(kYearThreads) void k_year_slice(const double *__res
     double sum = 0.0;
     if (d < kDays)
         sum = (double)insol_sum(sverts[3 * k], sverts[3 * k + 1], sverts[3 * k + 2], radius, rot,
-                                nsteps, tilt[2 * d], tilt[2 * d + 1], 0.0f);
+                                nsteps, tilt[2 * d], tilt[2 * d + 1], tilt[2 * d] == tilt[2 * d], 0.0f);
     __shared__ double part[kYearThreads / 64];
     for (int off = 32; off > 0; off >>= 1) sum += __shfl_down(sum, off, 64);
     if ((d & 63) == 0) part[d >> 6] = sum;
@@ -222,15 +223,19 @@ __global__ __launch_bounds__(256) void k_interpolate(const double *__restrict__ 
 
 size_t climate_workspace_bytes() { return climate_layout().total; }
 
-// rot[2s], rot[2s+1] = cos, sin of (rotation * pi) / 180 for s = 0..nsteps-1.
-static void fill_rot(double *t, double rot0, double rot_step, int nsteps)
+// rot[2s], rot[2s+1] = cos, sin of (rotation * pi) / 180 for s = 0..nsteps-1;
+// whether all are finite (not for an infinite angle or a NaN).
+static bool fill_rot(double *t, double rot0, double rot_step, int nsteps)
 {
     const double pi = 3.141592653589793;
     double rotation = rot0;
+    bool finite = true;
     for (int s = 0; s < nsteps; ++s) {
         sincos(rotation * pi / 180, &t[2 * s + 1], &t[2 * s]);
+        finite = finite && std::isfinite(t[2 * s]);
         rotation += rot_step;
     }
+    return finite;
 }
 
 static int climate_check(nx_ctx *ctx, const void *ws)
@@ -255,12 +260,13 @@ int sample_insolation(nx_ctx *ctx, const double *verts, int64_t V, double radius
     int slot = 0;
     double *t = (double *)stage_begin(ctx, 16 * (size_t)nsteps, &slot);
     if (!t) return set_error(NX_ENOMEM, "pinned staging buffer allocation failed");
-    fill_rot(t, rot0, rot_step, nsteps);
+    const bool finite = fill_rot(t, rot0, rot_step, nsteps);
     if ((rc = stage_commit(ctx, slot, (char *)ws + L.rot, 16 * (size_t)nsteps, stream))) return rc;
     double st, ct;
     sincos(tilt * 3.141592653589793 / 180, &st, &ct);
     hipLaunchKernelGGL(k_insolation, dim3((unsigned)((V + 255) / 256)), dim3(256), 0, stream, verts,
-                       V, radius, (const double *)((char *)ws + L.rot), nsteps, ct, st, arr);
+                       V, radius, (const double *)((char *)ws + L.rot), nsteps, ct, st,
+                       finite && std::isfinite(ct) ? 1 : 0, arr);
     NX_HIP(hipGetLastError());
     return NX_OK;
 }

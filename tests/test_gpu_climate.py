@@ -173,3 +173,32 @@ def test_year_of_each_latitude_band(oracle, radius):
     day_ulp = float(np.spacing(np.float32(ref.max() / 360)))
     tol = 360 * 361 * day_ulp + 360 * float(np.spacing(np.float32(ref.max())))
     assert got.dtype == np.float32 and np.abs(got.astype(np.float64) - ref).max() <= tol
+
+
+@pytest.mark.parametrize("nsteps", [1, 3])
+@pytest.mark.parametrize("rot,step,tilt", [(np.nan, 1.0, 23.0), (np.inf, 1.0, 23.0), (10.0, np.inf, 23.0),
+                                           (10.0, 1.0, np.nan), (10.0, 1.0, -np.inf),
+                                           (1e308, -1e308, 23.0)])
+def test_insolation_at_angles_that_are_not_finite(oracle, rot, step, tilt, nsteps):
+    """A NaN or infinite tilt or rotation (or one whose radians overflow) gives
+    NaN wherever the oracle has it, for vertices on the sphere as for others."""
+    pts, _ = util.create_mesh(6)
+    verts = np.concatenate([pts, pts * 1.01])
+    arr = torch.zeros(verts.shape[0], dtype=torch.float32, device="cuda")
+    climate.sample_insolation_device(arr, torch.from_numpy(verts).cuda(), 1.0, rot, tilt, nsteps, step)
+    got = arr.cpu().numpy()
+    ref = oracle.sample_insolation(np.zeros(verts.shape[0], np.float32), verts, 1.0, rot, tilt, nsteps,
+                                   step)
+    fine = np.isfinite(ref)
+    assert np.array_equal(np.isnan(got), np.isnan(ref))
+    assert not fine.any() or np.abs(got[fine] - ref[fine]).max() <= nsteps * np.spacing(np.float32(1))
+
+
+@pytest.mark.parametrize("tilt", [np.nan, np.inf])
+def test_tables_at_a_tilt_that_is_not_finite(oracle, tilt):
+    pts, _ = util.create_mesh(4)
+    assert np.isnan(oracle.insolation_slice(1.0, tilt)).all()
+    assert np.isnan(climate.calc_insolation_slice(1.0, tilt)).all()
+    assert np.isnan(climate.calc_daily_insolation(pts, None, 1.0, tilt)).all()
+    assert np.isnan(oracle.yearly_insolation(pts, 1.0, tilt)).all()
+    assert np.isnan(climate.calc_yearly_insolation(pts, None, 1.0, tilt)).all()
