@@ -12,7 +12,7 @@
 //
 // cos(latitude) * cos(longitude) of a rotated vertex t is, without the
 // angles, sqrt(1 - (t.z / r)^2) * t.x / sqrt(t.x^2 + t.y^2); on the sphere of
-// radius r the two roots cancel and it is t.x / r, the sun's direction
+// radius r the two roots cancel and it is t.x / |r|, the sun's direction
 // component.  k_insolation and k_slices use the second form for vertices on
 // the sphere to within rounding, the first elsewhere, and the angles
 // themselves (insol_value) only where the first form's quotients could
@@ -109,7 +109,8 @@ __device__ __forceinline__ float insol_sum(double x, double y, double z, double 
     const double r2 = r * r, v2 = x * x + y * y + z * z;
     const bool r_ok = r2 >= 0x1p-900 && r2 <= 0x1p900;
     if (finite && r_ok && fabs(v2 - r2) <= kOnSphere * r2) {
-        const double xs = x * ct / r, ys = -y * ct / r, zs = z * st / r;
+        const double d = fabs(r);   // the longitude does not depend on the radius's sign
+        const double xs = x * ct / d, ys = -y * ct / d, zs = z * st / d;
 #pragma unroll 4
         for (int s = 0; s < nsteps; ++s) {
             const double t = fma(xs, rot[2 * s], fma(ys, rot[2 * s + 1], zs));

@@ -202,3 +202,21 @@ def test_tables_at_a_tilt_that_is_not_finite(oracle, tilt):
     assert np.isnan(climate.calc_daily_insolation(pts, None, 1.0, tilt)).all()
     assert np.isnan(oracle.yearly_insolation(pts, 1.0, tilt)).all()
     assert np.isnan(climate.calc_yearly_insolation(pts, None, 1.0, tilt)).all()
+
+
+@pytest.mark.parametrize("radius", [-1.0, -6378100.0])
+def test_insolation_of_a_negative_radius(oracle, radius):
+    """The angles do not depend on the radius's sign but for the latitude's:
+    on the sphere of |radius|, off it and in the tables, against the oracle,
+    one float32 ulp per summed step."""
+    pts, _ = util.create_mesh(17)
+    verts = np.concatenate([pts, pts * 1.01]) * abs(radius)
+    for nsteps in (1, 360):
+        arr = torch.zeros(verts.shape[0], dtype=torch.float32, device="cuda")
+        climate.sample_insolation_device(arr, torch.from_numpy(verts).cuda(), radius, -180.0, 23.44,
+                                         nsteps, 360.0 / nsteps)
+        ref = oracle.sample_insolation(np.zeros(verts.shape[0], np.float32), verts, radius, -180.0,
+                                       23.44, nsteps, 360.0 / nsteps)
+        _report(f"radius {radius} steps {nsteps}", arr.cpu().numpy(), ref, nsteps)
+    _report(f"slice radius {radius}", climate.calc_insolation_slice(radius, 12.5),
+            oracle.insolation_slice(radius, 12.5), 360)
