@@ -816,6 +816,12 @@ __device__ __forceinline__ bool knn_near(const GridView &v, const ShellQuery &q,
     return bd[K - 1] <= beyond(g, q.norm, g.cosa[R - 1], g.sin2a[R - 1]);
 }
 
+// From this far rounding leaves every point of a shell (norms up to 2^300) at
+// one distance, infinite where its square overflows: a coordinate of 2^353 or
+// more takes no change from a point's, and the square of a smaller one none
+// of the sum.  The nearest are then the first by index.
+constexpr double kFar = 0x1p500;
+
 // Rounds of doubling reach in FP64, for queries knn_near does not settle.
 // The angles' terms double with the reach (sin 2a = 2 sin a cos a).
 template <int K, int R>
@@ -827,7 +833,17 @@ __device__ __forceinline__ void knn_rounds(const GridView &v, const ShellQuery &
     float sina = g.sina[R - 1];
     double ca = g.cosa[R - 1], s2 = g.sin2a[R - 1];
     none_yet<K>(bd, bi);
-    if (!(q.norm < INFINITY)) return;   // no distance to compare
+    if (q.norm != q.norm) return;   // a NaN: no distance to compare
+    if (q.norm >= kFar) {
+        const int32_t n = v.start[g.nbins];   // the number of points
+#pragma unroll
+        for (int m = 0; m < K; ++m)
+            if (m < n) {
+                bd[m] = dist2(v.pts + 3 * m, q.x, q.y, q.z);
+                bi[m] = m;
+            }
+        return;
+    }
     for (int r = R;; r *= 2) {
         none_yet<K>(bd, bi);
         bool circle;

@@ -219,3 +219,24 @@ def test_query_pixels_rows_share_their_points(oracle, d, wh):
     d_, n_ = util.KnnGrid(pts).query_pixels_device(wh[0], wh[1], 1.0, 3)
     rd, rn = oracle.knn(pts, oracle.make_ll_arr(wh[0], wh[1], 1.0), 3)
     assert np.array_equal(d_.cpu().numpy(), rd) and np.array_equal(n_.cpu().numpy(), rn)
+
+
+@pytest.mark.parametrize("k", [1, 3, 8])
+def test_query_from_where_squared_distances_overflow(oracle, k):
+    """Every point is then equally far, at an infinite distance where the square
+    overflows: the first points by index, not none."""
+    for pts in (util.create_mesh(9)[0], util.create_mesh(9)[0] * 6378100.0, np.concatenate([np.eye(3), -np.eye(3)])):
+        q = np.array([[1e200, 0, 0], [0, -1e200, 0], [1e200, 1e200, -1e200], [np.inf, 0, 0],
+                      [-np.inf, np.inf, 1.0], [1e160, 1, 1], [1e-3, 2.0, -1.35e154], [1.34e154, 3.0, 0],
+                      [0, 0, 1e152], [1e120, 1e153, 1e100]])
+        grid = util.KnnGrid(pts)
+        d, n = grid.query(q, k=k)
+        rd, rn = oracle.knn(pts, q, k)
+        if k == 1:
+            rd, rn = rd[..., 0], rn[..., 0]
+        assert np.array_equal(d, rd) and np.array_equal(n, rn)
+        for radius in (1e200, -1e200, 1e160, 1e153):
+            for w, h in ((8, 5), (300, 3)):
+                d, n = grid.query_pixels_device(w, h, radius, k)
+                rd, rn = oracle.knn(pts, oracle.make_ll_arr(w, h, radius), k)
+                assert np.array_equal(d.cpu().numpy(), rd) and np.array_equal(n.cpu().numpy(), rn)
