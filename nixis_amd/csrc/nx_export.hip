@@ -492,24 +492,48 @@ __device__ __forceinline__ void none_yet(double (&bd)[K], int32_t (&bi)[K])
     }
 }
 
+// How many points a query reads together from a dense run (scan).  More cover
+// more latency but take registers, which the pixels' kernels need for waves
+// (8192 x 4096 on d=1000, K = 3: 939 us at 2 and seven waves, 1,055 at 4 and six;
+// points in the caller's order are faster with fewer waves anyway: 3,333,334
+// queries on d=1000, 497 us at 4 and four waves, 643 at 2 and seven).
+constexpr int kPointScan = 4;
+constexpr int pixel_scan(int k) { return k <= 3 ? 2 : 4; }
+
 // The points of entries j..e-1 among the K best, T at a time, so that a long
-// run's loads go out together.  Points may come that were met before.  Two at a
-// time and bins in blocks (cell_bin): 499,281 queries of 998,562 vertices off the
-// origin 300 us, 670 where each candidate's entry was read and compared first
-// and cells were hashed one by one.
-constexpr int kScan = 2;
-template <int K, int T>
+// run's loads go out together.  SHELL: an entry lies within 0.87 of its unit of
+// its point, so its own distance tells whether the point can be among the K
+// (most: squared, in units, the largest that can, with slack for FP32); where
+// none of T can, no point is read.  AGAIN: points may come that were met before.
+// 499,281 queries of 998,562 vertices off the origin (cells): 263 us, 670 where
+// each candidate's entry was read and compared before its point and cells were
+// hashed one by one.
+template <int K, int T, bool SHELL, bool AGAIN>
 __device__ __forceinline__ void scan(const GridView &v, int j, int e, double qx, double qy,
-                                     double qz, double (&bd)[K], int32_t (&bi)[K])
+                                     double qz, double f, float &most, double (&bd)[K],
+                                     int32_t (&bi)[K])
 {
     for (; j < e; j += T) {
-        double s[T], least = INFINITY;
+        double s[T];
         int32_t id[T];
+        if (SHELL) {
+            bool near = false;
+#pragma unroll
+            for (int u = 0; u < T; ++u) {
+                const GridEntry p = v.entry[min(j + u, e - 1)];
+                const float dx = (float)fma(qx, f, -(double)p.x), dy = (float)fma(qy, f, -(double)p.y),
+                            dz = (float)fma(qz, f, -(double)p.z);
+                near = near || !(fmaf(dz, dz, fmaf(dy, dy, dx * dx)) > most);
+                id[u] = p.idx;
+            }
+            if (!near) continue;
+        }
+        double least = INFINITY;
 #pragma unroll
         for (int u = 0; u < T; ++u) {
             const int at = min(j + u, e - 1);
-            id[u] = v.entry[at].idx;
-            s[u] = dist2(v.pts + 3 * (int64_t)at, qx, qy, qz);
+            if (!SHELL) id[u] = v.entry[at].idx;
+            s[u] = dist2(v.pts + 3 * (int64_t)(SHELL ? id[u] : at), qx, qy, qz);
             least = fmin(least, s[u]);
         }
         if (!(least <= bd[K - 1])) continue;
@@ -526,14 +550,19 @@ __device__ __forceinline__ void scan(const GridView &v, int j, int e, double qx,
 #pragma unroll 1
         for (int u = 0; u < T; ++u) {
             bool held = false;
+            if (AGAIN)
 #pragma unroll
-            for (int h = 0; h < K; ++h) held = held || bi[h] == id[0];
+                for (int h = 0; h < K; ++h) held = held || bi[h] == id[0];
             if (!held && before(s[0], id[0], bd[K - 1], bi[K - 1])) insert<K>(s[0], id[0], bd, bi);
 #pragma unroll
             for (int w = 1; w < T; ++w) {
                 s[w - 1] = s[w];
                 id[w - 1] = id[w];
             }
+        }
+        if (SHELL) {
+            const float far = (float)(sqrt(bd[K - 1]) * f) + 2.0f;
+            most = far * far * (1.0f + 2e-6f);
         }
     }
 }
@@ -542,7 +571,7 @@ __device__ __forceinline__ void scan(const GridView &v, int j, int e, double qx,
 // cell until the K-th squared distance is within the block's guaranteed
 // radius (the distance from q to the nearest face of the block that does not
 // lie on the grid's border, less a margin for rounding of the cell bounds).
-template <int K>
+template <int K, int T>
 __device__ __forceinline__ void knn_cells(const GridView &v, double qx, double qy, double qz,
                                        double (&bd)[K], int32_t (&bi)[K])
 {
@@ -556,6 +585,7 @@ __device__ __forceinline__ void knn_cells(const GridView &v, double qx, double q
     const int cz = cell_of(qz, oz, cell, dz);
     const int rmax = max(dx, max(dy, dz));
     const double margin = 1e-9 * cell;
+    float most = 0.0f;   // (shells only)
     for (int r = 0; r <= rmax; ++r) {
         for (int z = cz - r; z <= cz + r; ++z) {
             if (z < 0 || z >= dz) continue;
@@ -567,7 +597,7 @@ __device__ __forceinline__ void knn_cells(const GridView &v, double qx, double q
                     if (x < 0 || x >= dx) continue;
                     const int32_t *s = v.start + cell_bin(x, y, z, mask);
                     // other cells' points in the bin are no worse candidates
-                    scan<K, kScan>(v, s[0], s[1], qx, qy, qz, bd, bi);
+                    scan<K, T, false, true>(v, s[0], s[1], qx, qy, qz, 0.0, most, bd, bi);
                 }
             }
         }
@@ -584,13 +614,14 @@ __device__ __forceinline__ void knn_cells(const GridView &v, double qx, double q
     }
 }
 
-// Latitude bands.  A round of reach r visits the bands within r of q's and,
-// in each, the cells within longitude D of q, sin D = sin(r h) / cos(latitude
-// of q) for a band height h (all cells where that passes 1, near the poles).
-// Every point not visited then lies at an angle of at least r h from q (its
-// latitude differs by that, or its meridian passes q no nearer), and at an
-// angle a and norms in [rmin, rmax] its squared distance is at least
-// (|q| - t)^2 + 4 |q| t sin^2(a / 2), t = |q| cos a clamped to those norms.
+// Latitude bands.  A round of reach a visits the bands within a of q's latitude
+// (or r bands on either side, a = r h for a band height h) and, in each, the
+// cells within longitude D of q, sin D = sin a / cos(latitude of q) (all cells
+// where that passes 1, near the poles).  Every point not visited then lies at
+// an angle of at least a from q (its latitude differs by that, or its meridian
+// passes q no nearer), and with a norm in [rmin, rmax] its squared distance is
+// at least (|q| - t)^2 + 4 |q| t sin^2(a / 2), t = |q| cos a clamped to those
+// norms.
 struct ShellQuery {
     double x, y, z, norm;
     float lat, lon, clat;
@@ -644,6 +675,9 @@ __device__ __forceinline__ double beyond(const GridHead &g, double qn, double ca
     return ((qn - t) * (qn - t) + 4.0 * qn * t * s2) * (1.0 - kGuardSlack);
 }
 
+// Candidates whose number fits the words of knn_near where they are not staged.
+constexpr int kMost = 64;
+
 // The first round, of reach R: the candidates' squared distances in FP32 from
 // exact integer differences, the K + 1 least kept as one word each (the
 // number of the candidate in the low bits), then FP64 for the K.  False where
@@ -661,9 +695,9 @@ __device__ __forceinline__ double beyond(const GridHead &g, double qn, double ca
 // in FP64); 2048 x 1024 on d=320: 76 (86, 137).
 template <int K, int R, bool STAGED>
 __device__ __forceinline__ bool knn_near(const GridView &v, const ShellQuery &q, float4 *lds,
-                                         double (&bd)[K], int32_t (&bi)[K])
+                                         double (&bd)[K], int32_t (&bi)[K], int &total)
 {
-    constexpr int kBands = 2 * R + 1, kMost = 64;
+    constexpr int kBands = 2 * R + 1;
     const GridHead &g = *v.g;
     if (!(q.norm <= 2.0 * g.rmax)) return false;   // the differences stay within 31 bits
     const double f = g.fixed;
@@ -672,7 +706,6 @@ __device__ __forceinline__ bool knn_near(const GridView &v, const ShellQuery &q,
     const float D = window(g.sina[R - 1], q.clat, circle);
     const int own = STAGED ? __builtin_amdgcn_readfirstlane(q.own) : q.own;
     Run run[kBands];
-    int total = 0;
     // Most waves' windows are parts of their bands, with no end in between:
     // then each band's runs are one, from the first query's start to the last's end.
     bool simple = STAGED && !__any(circle);
@@ -858,16 +891,13 @@ __device__ __forceinline__ bool knn_near(const GridView &v, const ShellQuery &q,
 // of the sum.  The nearest are then the first by index.
 constexpr double kFar = 0x1p500;
 
-// Rounds of doubling reach in FP64, for queries knn_near does not settle.
-// The angles' terms double with the reach (sin 2a = 2 sin a cos a).
-template <int K, int R>
-__device__ __forceinline__ void knn_rounds(const GridView &v, const ShellQuery &q, double (&bd)[K],
-                                           int32_t (&bi)[K])
+// Rounds in FP64 for queries knn_near does not settle: of reach a0, then of a1
+// and its doubles.  sin a is bounded by a from above and by a - a^3 / 6 from below.
+template <int K, int T>
+__device__ __forceinline__ void knn_rounds(const GridView &v, const ShellQuery &q, float a0,
+                                           float a1, double (&bd)[K], int32_t (&bi)[K])
 {
     const GridHead &g = *v.g;
-    const float h = 3.14159265f / (float)v.bands;
-    float sina = g.sina[R - 1];
-    double ca = g.cosa[R - 1], s2 = g.sin2a[R - 1];
     none_yet<K>(bd, bi);
     if (q.norm != q.norm) return;   // a NaN: no distance to compare
     if (q.norm >= kFar) {
@@ -880,33 +910,46 @@ __device__ __forceinline__ void knn_rounds(const GridView &v, const ShellQuery &
             }
         return;
     }
-    for (int r = R;; r *= 2) {
+    const double f = g.fixed;
+    for (float a = a0;; a = fmaxf(2.0f * a, a1)) {
         none_yet<K>(bd, bi);
+        float most = INFINITY;
+        const bool whole = a >= 3.2f;
         bool circle;
-        const float D = window((float)r * h < 1.5f ? sina : 2.0f, q.clat, circle);
-        for (int k = 0; k <= 2 * r; ++k) {   // q's band, then outwards
-            const Run run = band_run(v, q, q.own + ((k & 1) ? -((k + 1) >> 1) : (k >> 1)), D, circle);
-            for (int i = 0; i < run.n; ++i) {
-                const int32_t id = v.entry[run.at(i)].idx;
-                const double s = dist2(v.pts + 3 * (int64_t)id, q.x, q.y, q.z);
-                if (before(s, id, bd[K - 1], bi[K - 1])) insert<K>(s, id, bd, bi);
+        const float D = window(a < 1.5f ? a : 2.0f, q.clat, circle), up = a + 2.0f * kAngleSlack;
+        const int lo = whole ? 0 : band_of(q.lat - up, v.bands, g.perband);
+        const int hi = whole ? v.bands - 1 : band_of(q.lat + up, v.bands, g.perband);
+        const int reach = max(q.own - lo, hi - q.own);
+        for (int k = 0; k <= 2 * reach; ++k) {   // q's band, then outwards
+            const int b = q.own + ((k & 1) ? -((k + 1) >> 1) : (k >> 1));
+            if (b < lo || b > hi) continue;
+            const Run run = band_run(v, q, b, D, circle);
+#pragma unroll 1
+            for (int part = 0; part < 2; ++part) {
+                const int j = part ? run.jb : run.ja, n = part ? run.n - run.na : run.na;
+                scan<K, T, true, false>(v, j, j + n, q.x, q.y, q.z, f, most, bd, bi);
             }
         }
-        if (circle && q.own - r <= 0 && q.own + r >= v.bands - 1) return;   // all points visited
-        // a reach of pi or more passes every band: the next round covers all
-        if ((float)r * h < 3.14f && bd[K - 1] <= beyond(g, q.norm, ca, s2)) return;
-        sina = 2.0f * sina * sqrtf(fmaxf(1.0f - sina * sina, 0.0f));
-        s2 = 4.0 * s2 * (1.0 - s2);
-        ca = 1.0 - 2.0 * s2;
+        if (whole || (circle && lo == 0 && hi == v.bands - 1)) return;   // all points visited
+        const float x = 0.5f * (a - 2.0f * kAngleSlack), s = fmaxf(x * (1.0f - x * x / 6.0f), 0.0f);
+        const double s2 = (double)s * s * (1.0 - kGuardSlack);
+        if (bd[K - 1] <= beyond(g, q.norm, 1.0 - 2.0 * s2, s2)) return;
     }
 }
 
-template <int K, bool STAGED>
+template <int K, int T, bool STAGED>
 __device__ __forceinline__ void knn_shell(const GridView &v, const ShellQuery &q, float4 *lds,
                                           double (&bd)[K], int32_t (&bi)[K])
 {
     constexpr int R = K <= 3 ? 1 : 2;
-    if (!knn_near<K, R, STAGED>(v, q, lds, bd, bi)) knn_rounds<K, R>(v, q, bd, bi);
+    int total = 0;
+    if (knn_near<K, R, STAGED>(v, q, lds, bd, bi, total)) return;
+    // where the window holds more than kMost points, the first round's takes about
+    // that many at their density (400,000 points, half of them in a cap of 1 degree,
+    // 2,000 queries: 6.1 ms, 92 where every round took the whole window)
+    const float a1 = (float)R * (3.14159265f / (float)v.bands);
+    const float a0 = a1 * __builtin_amdgcn_sqrtf((float)kMost / (float)max(total, kMost));
+    knn_rounds<K, T>(v, q, fmaxf(a0, 16.0f * kAngleSlack), a1, bd, bi);
 }
 
 __device__ __forceinline__ ShellQuery shell_query(const GridView &v, double x, double y, double z)
@@ -971,9 +1014,9 @@ __global__ __launch_bounds__(256) void k_knn_points(GridView v, int64_t V,
     int32_t bi[K];
     const double x = q[3 * p], y = q[3 * p + 1], z = q[3 * p + 2];
     if (v.g->shell)
-        knn_shell<K, false>(v, shell_query(v, x, y, z), nullptr, bd, bi);
+        knn_shell<K, kPointScan, false>(v, shell_query(v, x, y, z), nullptr, bd, bi);
     else
-        knn_cells<K>(v, x, y, z, bd, bi);
+        knn_cells<K, kPointScan>(v, x, y, z, bd, bi);
     knn_store<K>(lds, p0, (int)min((int64_t)256, nq - p0), bd, bi, V, dists, nbrs);
 }
 
@@ -986,11 +1029,10 @@ __global__ __launch_bounds__(256) void k_knn_points(GridView v, int64_t V,
 // so that an XCD's L2 reads the points of its stripes once: 8192 x 4096 on
 // d=1000 STRIPES.  Otherwise blocks take 256 pixels across rows.
 template <int K, bool ROWS>
-__global__ __launch_bounds__(256) void k_knn_pixels(GridView v, int64_t V, int64_t width,
-                                                    int64_t height, double radius, int stripe,
-                                                    float dlat, float dlon, const double *__restrict__ trig,
-                                                    double *__restrict__ dists,
-                                                    int64_t *__restrict__ nbrs)
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(K <= 3 ? 7 : 4))) void
+k_knn_pixels(GridView v, int64_t V, int64_t width, int64_t height, double radius, int stripe,
+             float dlat, float dlon, const double *__restrict__ trig, double *__restrict__ dists,
+             int64_t *__restrict__ nbrs)
 {
     int64_t p0, h, w;
     int count;
@@ -1017,16 +1059,16 @@ __global__ __launch_bounds__(256) void k_knn_pixels(GridView v, int64_t V, int64
     double bd[K];
     int32_t bi[K];
     if (!v.g->shell) {
-        knn_cells<K>(v, x, y, z, bd, bi);
+        knn_cells<K, pixel_scan(K)>(v, x, y, z, bd, bi);
     } else if (radius > 0.0) {
         // the angles are the pixel's own
         ShellQuery q{x, y, z, radius, 0.0f, 0.0f, (float)clat, 0};
         q.lat = 3.14159265f - (float)(int)h * dlat;
         q.lon = (float)(int)w * dlon;
         q.own = band_of(q.lat, v.bands, v.g->perband);
-        knn_shell<K, ROWS>(v, q, lds.entry[threadIdx.x >> 6], bd, bi);
+        knn_shell<K, pixel_scan(K), ROWS>(v, q, lds.entry[threadIdx.x >> 6], bd, bi);
     } else {
-        knn_shell<K, false>(v, shell_query(v, x, y, z), nullptr, bd, bi);
+        knn_shell<K, pixel_scan(K), false>(v, shell_query(v, x, y, z), nullptr, bd, bi);
     }
     knn_store<K>(lds, p0, count, bd, bi, V, dists, nbrs);
 }
