@@ -139,78 +139,95 @@ bool cut(const int32_t *col, int64_t V, int64_t a, int64_t len, int K, int limit
 int tile_edges(const int32_t *lc, const double *len, const int32_t *dev, int c, int T,
                uint16_t *codes, double *lens)
 {
-    // bit k of own[j]: j holds the edge of its slot k; of movable[j]: the
-    // other end could hold it (the neighbour is in the set and the two slots
-    // name each other first)
-    std::vector<uint8_t> own((size_t)c, 0), movable((size_t)c, 0), back((size_t)6 * c, 0);
+    // a vertex's six neighbours beside each other
+    std::vector<int32_t> nb((size_t)6 * c);
+    for (int k = 0; k < 6; ++k)
+        for (int32_t j = 0; j < c; ++j) nb[(size_t)6 * j + k] = lc[(size_t)k * c + j];
+    // bit k of own[j]: j holds the edge of its slot k (held[j] of them); of
+    // movable[j]: the other end could hold it (the neighbour is in the set and
+    // the two slots name each other first)
+    std::vector<uint8_t> own((size_t)c, 0), movable((size_t)c, 0), held((size_t)c, 0), back((size_t)6 * c, 0);
     auto first = [&](int32_t n, int32_t j) {
         for (int q = 0; q < 6; ++q)
-            if (lc[(size_t)q * c + n] == j) return q;
+            if (nb[(size_t)6 * n + q] == j) return q;
         return -1;
     };
     for (int32_t j = 0; j < c; ++j)
         for (int k = 0; k < 6; ++k) {
-            const int32_t n = lc[(size_t)k * c + j];
+            const int32_t n = nb[(size_t)6 * j + k];
             if (n == j) continue;
             const int q = n < c ? first(n, j) : -1;
             bool mine = true;
             if (q >= 0 && first(j, n) == k) {
-                back[(size_t)k * c + j] = (uint8_t)q;
+                back[(size_t)6 * j + k] = (uint8_t)q;
                 movable[(size_t)j] |= (uint8_t)(1 << k);
                 mine = (j >= T) != (n >= T) ? j >= T : dev[j] < dev[n];
             }
-            if (mine) own[(size_t)j] |= (uint8_t)(1 << k);
+            if (mine) {
+                own[(size_t)j] |= (uint8_t)(1 << k);
+                ++held[(size_t)j];
+            }
         }
-    auto held = [&](int32_t j) { return __builtin_popcount(own[(size_t)j]); };
     int kr = kOwnRing;
     auto cap = [&](int32_t j) { return j < T ? kLenFull : kr; };
     std::vector<uint8_t> dist((size_t)c);
-    std::vector<int32_t> over, moves;   // vertices over their cap; slots that pass an edge
+    // vertices over their cap; the last label's and the next one's; those that
+    // may pass an edge; slots that do
+    std::vector<int32_t> over, at, next, pass, moves;
     for (int round = 0;; ++round) {
         over.clear();
-        for (int32_t j = 0; j < c; ++j)
-            if (held(j) > cap(j)) over.push_back(j);
+        at.clear();
+        for (int32_t j = 0; j < c; ++j) {
+            dist[(size_t)j] = kOwnFar;
+            if (held[(size_t)j] > cap(j)) over.push_back(j);
+            if (held[(size_t)j] < cap(j)) {
+                dist[(size_t)j] = 0;
+                at.push_back(j);
+            }
+        }
         if (over.empty()) break;
         if (round == kOwnRounds) return -1;
-        for (int32_t j = 0; j < c; ++j) dist[(size_t)j] = held(j) < cap(j) ? 0 : kOwnFar;
-        for (int s = 1; s < kOwnFar; ++s) {
-            bool changed = false;
-            for (int32_t j = 0; j < c; ++j) {
-                if (dist[(size_t)j] != kOwnFar) continue;
-                const int m = own[(size_t)j] & movable[(size_t)j];
-                for (int k = 0; k < 6; ++k)
-                    if ((m >> k & 1) && dist[(size_t)lc[(size_t)k * c + j]] == s - 1) {
-                        dist[(size_t)j] = (uint8_t)s;
-                        changed = true;
-                        break;
-                    }
-            }
-            if (!changed) break;
+        for (int s = 1; s < kOwnFar && !at.empty(); ++s) {
+            next.clear();
+            for (int32_t x : at)   // the ends that hold an edge to x
+                for (int m = movable[(size_t)x] & ~own[(size_t)x]; m; m &= m - 1) {
+                    const int32_t n = nb[(size_t)6 * x + __builtin_ctz(m)];
+                    if (dist[(size_t)n] != kOwnFar) continue;
+                    dist[(size_t)n] = (uint8_t)s;
+                    next.push_back(n);
+                }
+            at.swap(next);
             if (std::none_of(over.begin(), over.end(),
                              [&](int32_t j) { return dist[(size_t)j] == kOwnFar; }))
                 break;
         }
         // edges pass down the labels until no vertex over its cap has one to pass
         bool moved = false;
-        for (;;) {
+        for (pass = over;; moved = true) {
             moves.clear();
-            for (int32_t j = 0; j < c; ++j) {
-                const int at = dist[(size_t)j];
-                if (at == 0 || at == kOwnFar || held(j) <= cap(j)) continue;
-                const int m = own[(size_t)j] & movable[(size_t)j];
-                for (int k = 0; k < 6; ++k)
-                    if ((m >> k & 1) && dist[(size_t)lc[(size_t)k * c + j]] == at - 1) {
-                        moves.push_back(6 * j + k);
-                        break;
-                    }
+            for (int32_t j : pass) {
+                const int d = dist[(size_t)j];
+                if (d == 0 || d == kOwnFar || held[(size_t)j] <= cap(j)) continue;
+                for (int m = own[(size_t)j] & movable[(size_t)j]; m; m &= m - 1) {
+                    const int k = __builtin_ctz(m);
+                    if (dist[(size_t)nb[(size_t)6 * j + k]] != d - 1) continue;
+                    moves.push_back(6 * j + k);
+                    break;
+                }
             }
             if (moves.empty()) break;
-            moved = true;
+            pass.clear();
             for (int32_t e : moves) {
-                const int32_t j = e / 6, k = e % 6;
+                const int32_t j = e / 6, k = e % 6, n = nb[(size_t)e];
                 own[(size_t)j] &= (uint8_t)~(1 << k);
-                own[(size_t)lc[(size_t)k * c + j]] |= (uint8_t)(1 << back[(size_t)k * c + j]);
+                --held[(size_t)j];
+                own[(size_t)n] |= (uint8_t)(1 << back[(size_t)e]);
+                ++held[(size_t)n];
+                pass.push_back(j);
+                pass.push_back(n);
             }
+            std::sort(pass.begin(), pass.end());
+            pass.erase(std::unique(pass.begin(), pass.end()), pass.end());
         }
         if (!moved) {
             if (kr >= 6) return -1;
@@ -218,7 +235,7 @@ int tile_edges(const int32_t *lc, const double *len, const int32_t *dev, int c, 
         }
     }
     int kt = 1;
-    for (int32_t j = 0; j < c; ++j) kt = std::max(kt, held(j));
+    for (int32_t j = 0; j < c; ++j) kt = std::max<int>(kt, held[(size_t)j]);
     if (!codes) return kt;
     // columns in slot order of each owner
     auto column = [&](int32_t j, int k) { return __builtin_popcount(own[(size_t)j] & ((1 << k) - 1)); };
@@ -234,7 +251,7 @@ int tile_edges(const int32_t *lc, const double *len, const int32_t *dev, int c, 
                 code = (uint32_t)n | (uint32_t)column(j, k) << 12 | 0x8000u;
                 lens[len_index(column(j, k), j, c, T)] = len[sl];
             } else {   // n owns the edge, in its slot back to j
-                code = (uint32_t)n | (uint32_t)column(n, back[sl]) << 12;
+                code = (uint32_t)n | (uint32_t)column(n, back[(size_t)6 * j + k]) << 12;
             }
             codes[sl] = (uint16_t)code;
         }
