@@ -364,8 +364,9 @@ int nx_tile_plan_build_steps(const int32_t *col, const double *elen, int64_t V,
 /* nx_tile_plan_build_steps with the starting tile size `chunk` (kTileMin =
  * 32 .. 1024 vertices for 2 steps, .. 2048 for 4; 0 for the default: 768 for
  * 2 steps; for 4 steps 1152, or less for planets of up to 1.2 million vertices,
- * so that a launch fills the GPU; batches of planets, which fill it together,
- * are faster with 1152).
+ * so that a launch fills the GPU, and 1152 again where the rings of a graph with
+ * longer edges outgrow the smaller tiles; batches of planets, which fill it
+ * together, are faster with 1152).
  * Tiles are halved from there until their rings fit, so the chunk trades
  * ring overhead against the number of blocks per launch; the erosion
  * autotuner picks it per mesh size.  The results of erosion do not depend on
@@ -379,8 +380,9 @@ int nx_tile_plan_build_chunk(const int32_t *col, const double *elen, int64_t V,
  * memory of nx_tile_plan_device_workspace_bytes(V, chunk) bytes.  With out ==
  * NULL it cuts the tiles, waits for the stream and fills `plan`; called again
  * with the same workspace and plan and a zeroed device buffer of plan->bytes
- * it writes the image there, on the stream.  NX_ERANGE also for a neighbour
- * table that is not symmetric, which only the host planner takes. */
+ * it writes the image there, on the stream.  NX_ERANGE also for what only the
+ * host planner takes: a neighbour table that is not symmetric, and with chunk 0
+ * a graph whose rings outgrow the smaller default tiles. */
 size_t nx_tile_plan_device_workspace_bytes(int64_t V, int chunk);
 int nx_tile_plan_build_device(nx_ctx *ctx, const int32_t *col,
                               const double *elen, int64_t V, int chunk,

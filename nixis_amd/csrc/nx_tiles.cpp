@@ -280,8 +280,9 @@ void plan_layout(nx_tile_plan &q, int64_t nt, int64_t nring, int64_t ncs, int64_
     q.bytes = o;
 }
 
-int tile_plan_build(const int32_t *col, const double *elen, int64_t V, int K, void *out,
-                    int64_t cap, nx_tile_plan *plan, int chunk_in)
+// The plan of tiles that start at chunk_in vertices (0: the default size).
+static int plan_of_chunk(const int32_t *col, const double *elen, int64_t V, int K, void *out,
+                         int64_t cap, nx_tile_plan *plan, int chunk_in)
 {
     if (!col || !elen || !plan || V <= 0 || V > INT32_MAX)
         return set_error(NX_EINVAL, "tile plan needs col, elen, plan and 0 < V < 2^31");
@@ -448,6 +449,16 @@ int tile_plan_build(const int32_t *col, const double *elen, int64_t V, int K, vo
     }, 64);
     if (bad.load()) return set_error(NX_EINVAL, "tile plan: a neighbour fell outside its tile's rings");
     return NX_OK;
+}
+
+int tile_plan_build(const int32_t *col, const double *elen, int64_t V, int K, void *out,
+                    int64_t cap, nx_tile_plan *plan, int chunk_in)
+{
+    const int rc = plan_of_chunk(col, elen, V, K, out, cap, plan, chunk_in);
+    // a graph with longer edges whose rings outgrow the small default tiles
+    if (rc == NX_ERANGE && chunk_in == 0 && K == kMultiSteps && quad_chunk(V) < kQuadChunk)
+        return plan_of_chunk(col, elen, V, K, out, cap, plan, kQuadChunk);
+    return rc;
 }
 
 }  // namespace nx

@@ -356,3 +356,23 @@ def test_two_step_plan_is_no_slower_to_make():
                                                            None, 0, ctypes.byref(q)))
             best[K] = min(best.get(K, np.inf), time.perf_counter() - t)
     assert best[2] <= 1.2 * best[4], best
+
+
+@pytest.mark.parametrize("seed", range(6))
+def test_default_chunk_takes_what_full_tiles_take(seed):
+    """A small mesh with a few edges across it: its default tiles are smaller than
+    full ones, and where their rings hold too many vertices the plan is made of
+    full tiles, not refused."""
+    _, _, _, col, elen = _ell(17)
+    V = col.shape[1]
+    rng = np.random.default_rng(seed)
+    for _ in range(30):
+        col[rng.integers(6), rng.integers(V)] = rng.integers(V)
+    plans = {}
+    for chunk in (0, 256, 1152):
+        q = _lib.NxTilePlan()
+        rc = _lib.lib().nx_tile_plan_build_chunk(_lib.ptr(col), _lib.ptr(elen), V, 4, chunk, None, 0,
+                                                 ctypes.byref(q))
+        plans[chunk] = (rc, q.bytes, q.ntiles)
+    assert plans[1152][0] == _lib.NX_OK
+    assert plans[0] == (plans[256] if plans[256][0] == _lib.NX_OK else plans[1152])
