@@ -153,14 +153,17 @@ class ErosionGraph:
 
     def _build_plan_device(self, stream):
         """The four-step plan from the device tables, written before this
-        returns; False when refused."""
+        returns; False when refused, or without memory for its workspace."""
         import torch
         L = _lib.lib()
         plan = _lib.NxTilePlan()
         ctx = _lib.Context.get(self.device)
         with torch.cuda.stream(stream):      # the buffers belong to the planner's stream
-            ws = torch.empty(int(L.nx_tile_plan_device_workspace_bytes(self.V, self.chunk)),
-                             dtype=torch.uint8, device=self.device)
+            try:
+                ws = torch.empty(int(L.nx_tile_plan_device_workspace_bytes(self.V, self.chunk)),
+                                 dtype=torch.uint8, device=self.device)
+            except torch.OutOfMemoryError:
+                return False    # about 47 bytes a vertex; the host planner needs none here
 
             def build(out, cap):
                 return L.nx_tile_plan_build_device(

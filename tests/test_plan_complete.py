@@ -46,6 +46,22 @@ def test_planner_waits_for_the_image(monkeypatch, given):
     assert calls == [("size", stream), ("write", stream), ("wait", stream), ("use", None)]
 
 
+def test_no_memory_for_the_planner(monkeypatch):
+    """Without device memory for the planner's workspace the plan is left to the
+    host planner, which needs none."""
+    def empty(*args, **kw):
+        raise torch.OutOfMemoryError("full")
+
+    monkeypatch.setattr(_lib, "lib", lambda: SimpleNamespace(
+        nx_tile_plan_device_workspace_bytes=lambda V, chunk: 256))
+    monkeypatch.setattr(_lib.Context, "get", lambda device=None: SimpleNamespace(handle=None))
+    monkeypatch.setattr(torch.cuda, "stream", lambda s: contextlib.nullcontext())
+    monkeypatch.setattr(torch, "empty", empty)
+    g = erosion.ErosionGraph.__new__(erosion.ErosionGraph)
+    g.V, g.chunk, g.device = 12, 0, torch.device("cpu")
+    assert g._build_plan_device(None) is False
+
+
 @pytest.mark.gpu
 def test_run_on_another_stream_after_the_build(oracle):
     """The state is loaded and run on a second stream, which waits for nothing
