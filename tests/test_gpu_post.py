@@ -368,3 +368,30 @@ def test_small_chain_in_one_block(n, case):
     (h2, m2, l2, e2, _), (h5, m5, l5, e5, _) = _chain_both_forms(x)
     assert np.array_equal(h2, h5, equal_nan=True) and np.array_equal(m2, m5) and e2 is e5
     assert np.array_equal([l2], [l5], equal_nan=True)
+
+
+@pytest.mark.parametrize("n,low,high,small", [(5120, 0.0, 8850.0, True), (5121, 0.0, 8850.0, False),
+                                              (5121, -4000.0, 0.0, False), (16_384, 0.0, 8850.0, False),
+                                              (16_384, -4000.0, 8850.0, True)])
+def test_small_chain_at_an_altitude_of_zero(n, low, high, small):
+    """With an altitude of 0 the derivation does not hold, and the one launch,
+    whose first block alone then does the work, is for fewer heights (it copies
+    them into the workspace, behind the head).  The five-pass form's results
+    bit for bit on both sides of the limit."""
+    x = np.random.default_rng(n).standard_normal(n)
+    ctx = _lib.Context.get(0)
+    out = []
+    try:
+        for passes in (2, 5):
+            ctx.set_chain_passes(passes)
+            ws = torch.full((_lib.lib().nx_height_chain_workspace_bytes(n),), 0xa5, dtype=torch.uint8,
+                            device="cuda")
+            h, m, lv = util.height_chain_device(_dev(x), low, high, 55.0, workspace=ws)
+            ctx.sync_check()
+            copied = not bool((ws[256 + 8 * (n - 8):256 + 8 * n] == 0xa5).all())
+            out.append((h.cpu().numpy(), m.cpu().numpy(), lv.item(), copied))
+    finally:
+        ctx.set_chain_passes(2)
+    (h2, m2, l2, copied), (h5, m5, l5, _) = out
+    assert _same_bits(h2, h5) and np.array_equal(m2, m5) and l2 == l5
+    assert copied is small
