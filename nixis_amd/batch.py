@@ -59,9 +59,10 @@ def _L():
     return L
 
 
-# Starting tile size of a batch's plans: planets that share launches fill the
-# GPU together, so their tiles are full ones (the library's default makes a
-# small planet's tiles smaller to spread them over an otherwise idle GPU).
+# Starting tile size of a batch's plans without a tuning: planets that share
+# launches fill the GPU together, so their tiles are full ones (the library's
+# default makes a small planet's tiles smaller to spread them over an otherwise
+# idle GPU; a tuning's chunk of 0 is that default, which its search timed).
 BATCH_CHUNK = 1152
 
 
@@ -164,9 +165,7 @@ class MeshCache:
             if tuning is None:
                 from . import autotune
                 tuning = autotune.lookup_erosion(10 * d * d + 2)
-            kw = tuning.graph_kwargs() if tuning is not None else {"chunk": 0}
-            if kw.get("steps", 4) == 4:
-                kw["chunk"] = kw["chunk"] or BATCH_CHUNK
+            kw = tuning.graph_kwargs() if tuning is not None else {"chunk": BATCH_CHUNK}
             g = self._build_graph(d, **kw)
             self._graphs[d] = g
         return g

@@ -49,3 +49,22 @@ def test_merge_keeps_faster_unsearched_step_count():
     slow = dict(four, us_per_step=130.0)
     assert autotune.merge_erosion_entry(slow, two, {2: None}) == two
     assert autotune.merge_erosion_entry(None, two, {2: None}) == two
+
+
+def test_mesh_cache_cuts_plans_as_tuned(monkeypatch):
+    """MeshCache.graph takes a tuning's chunk as it was timed, 0 (the library's
+    default) too, as MeshCache.tune_erosion does; without a tuning plans start
+    from full tiles."""
+    from nixis_amd import batch
+    made = []
+    meshes = batch.MeshCache(device="cpu")
+    monkeypatch.setattr(meshes, "_build_graph", lambda d, **kw: made.append((d, kw.get("chunk"))))
+    monkeypatch.setattr(autotune, "tune_erosion", lambda make, **kw: (autotune.ErosionTuning(0, 0, 32, 4), []))
+    monkeypatch.setattr(autotune, "lookup_erosion", lambda V: None)
+    meshes.graph(32)
+    meshes.graph(64, tuning=autotune.ErosionTuning(0, 0, 32, 4))
+    meshes.graph(66, tuning=autotune.ErosionTuning(640, 0, 32, 2))
+    meshes.tune_erosion(68)
+    monkeypatch.setattr(autotune, "lookup_erosion", lambda V: autotune.ErosionTuning(0, 0, 32, 4))
+    meshes.graph(70)
+    assert made == [(32, batch.BATCH_CHUNK), (64, 0), (66, 640), (68, 0), (70, 0)]
