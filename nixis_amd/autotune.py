@@ -5,11 +5,12 @@ keyed by the batch's shape class (log2 of the total vertex count and the
 mean octave count).
 
 Erosion: the tile plan's steps per launch (four or two), its starting
-chunk (tile size before halving), the kernel variant and the steps per
-captured hipGraph, keyed by the mesh's size class (log2 of its vertex
-count).  For each step count a coordinate search times the variants on the
-default plan, then the chunks with the best variant; the graph chunks are
-timed for the best of all.  None of the choices changes the results.
+chunk (tile size before halving) and the kernel variant, keyed by the mesh's
+size class (log2 of its vertex count).  For each step count a coordinate
+search times the variants on the default plan, then the chunks with the best
+variant.  For a mesh without a plan, whose runs replay captured hipGraphs,
+the steps per graph are timed instead.  None of the choices changes the
+results.
 
 Candidates are timed with HIP events on the launch stream; the best one is
 stored in a JSON file, so later work of the same class reuses it without
@@ -99,7 +100,7 @@ GRAPH_CHUNKS = (8, 16, 32, 64)
 class ErosionTuning:
     chunk: int = 0          # tile plan starting chunk (0: the library default)
     variant: int = 0        # kernel variant for the plan's steps per launch
-    graph_chunk: int = 32   # erosion steps per captured graph
+    graph_chunk: int = 32   # erosion steps per captured graph (runs without a plan)
     steps: int = 4          # steps per launch of the tile plan (4 or 2)
 
     def graph_kwargs(self):
@@ -137,7 +138,8 @@ def tune_erosion(make_graph, heights=None, steps=20, reps=3, path=CACHE_PATH, pe
     field) start every timed run.  For each step count in step_options, the
     kernel variants (variants[steps], default VARIANTS) are timed on the
     default plan, then the chunks (chunks[steps], default CHUNKS) with the
-    best variant; the graph chunks are timed for the best of all.  Returns
+    best variant; the graph chunks are timed for a mesh without a plan (over a
+    plan they change nothing: their rows repeat the best's time).  Returns
     the best ErosionTuning and the table of (us per step, steps, chunk,
     variant, graph chunk) timings; the cache keeps the best and, when it is
     not two-step, the best two-step tuning beside it."""
@@ -198,9 +200,11 @@ def tune_erosion(make_graph, heights=None, steps=20, reps=3, path=CACHE_PATH, pe
         per_steps[K] = (t_best, ErosionTuning(c_best, v_best, gchunk0, K), g_best)
     if not per_steps:
         raise ValueError(f"no tile plan of {step_options} steps per launch for this mesh")
-    _, best, g_best = min(per_steps.values(), key=lambda r: r[0])
-    if graph_chunks:
+    us, best, g_best = min(per_steps.values(), key=lambda r: r[0])
+    if g_best.plan is None and graph_chunks:
         best.graph_chunk = min(graph_chunks, key=lambda k: time_it(g_best, best.variant, k))
+    else:       # runs over a plan launch eagerly: the same launches for every graph chunk
+        table += [(round(us, 3), best.steps, g_best.chunk, best.variant, k) for k in graph_chunks]
     if persist:
         entry = {"chunk": best.chunk, "variant": best.variant, "graph_chunk": best.graph_chunk,
                  "steps": best.steps, "us_per_step": min(t for t, *_ in table)}

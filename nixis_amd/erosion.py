@@ -65,8 +65,8 @@ class ErosionGraph:
     `chunk` is the plan's starting tile size (0: the library's default),
     `variant` the kernel variant for the plan's step count (the context's
     NX_OPT_MULTI_KERNEL or NX_OPT_PAIR_KERNEL) and `graph_chunk` the steps
-    per captured graph that runs on this graph use (None: the context's
-    setting); autotune.tune_erosion picks the four per mesh size.  None of
+    per captured graph of runs without a plan (None: the context's setting);
+    autotune.tune_erosion picks the four per mesh size.  None of
     them changes the results.
     """
 
@@ -293,7 +293,7 @@ class ErosionState:
         plan = ctypes.byref(graph.plan) if graph.plan is not None else None
         variant = getattr(graph, "variant", None)
         four = graph.plan is not None and graph.plan.steps == 4
-        with self.ctx.options(graph_chunk=getattr(graph, "graph_chunk", None),
+        with self.ctx.options(graph_chunk=None if graph.plan is not None else getattr(graph, "graph_chunk", None),
                               pair_kernel=None if four else variant,
                               multi_kernel=variant if four else None):
             _lib.check(_lib.lib().nx_erosion_run_rule(

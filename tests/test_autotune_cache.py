@@ -68,3 +68,51 @@ def test_mesh_cache_cuts_plans_as_tuned(monkeypatch):
     monkeypatch.setattr(autotune, "lookup_erosion", lambda V: autotune.ErosionTuning(0, 0, 32, 4))
     meshes.graph(70)
     assert made == [(32, batch.BATCH_CHUNK), (64, 0), (66, 640), (68, 0), (70, 0)]
+
+
+def test_tuner_times_graph_chunks_without_a_plan_only(monkeypatch, tmp_path):
+    """Runs over a plan replay no graphs: the tuner runs nothing for the graph
+    chunks and keeps the default, where every one would have measured noise.
+    Without a plan it times each."""
+    from types import SimpleNamespace
+
+    import torch
+    from nixis_amd import erosion
+    runs = []
+
+    class State:
+        def __init__(self, V, device=None):
+            pass
+
+        def load(self, heights):
+            pass
+
+        def run(self, graph, iters, rain):
+            runs.append(graph.graph_chunk)
+
+    class Event:
+        def __init__(self, enable_timing=False):
+            pass
+
+        def record(self, stream):
+            self.at = len(runs)
+
+        def synchronize(self):
+            pass
+
+        def elapsed_time(self, other):      # a later run looks a little faster
+            return 1.0 / other.at
+
+    monkeypatch.setattr(erosion, "ErosionState", State)
+    monkeypatch.setattr(torch.cuda, "Event", Event)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: None)
+    for plan in (object(), None):
+        del runs[:]
+        best, table = autotune.tune_erosion(
+            lambda c, k: SimpleNamespace(V=12, device="cpu", plan=plan, steps=k, chunk=c),
+            heights=torch.zeros(12), path=str(tmp_path / "t.json"), graph_chunks=(8, 16, 32, 64))
+        assert {k for *_, k in table} == {8, 16, 32, 64}
+        if plan is None:
+            assert set(runs) == {8, 16, 32, 64} and best.graph_chunk == 64
+        else:
+            assert set(runs) == {32} and best.graph_chunk == 32
