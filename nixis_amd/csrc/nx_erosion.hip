@@ -101,8 +101,8 @@ __global__ __launch_bounds__(THREADS) void k_erode_pair(ErosionMeta *__restrict_
                                                        double2 *__restrict__ hw1,
                                                        double *__restrict__ s0,
                                                        double *__restrict__ s1, TilePlanDev P, int j,
-                                                       int64_t done, double rain_first,
-                                                       double rain_mid, double rain_next)
+                                                       int64_t done, double rain_mid,
+                                                       double rain_next)
 {
     __shared__ double2 A[kLoadMax];
     __shared__ double2 B[THREADS == 1024 ? kStepOneMax : 1];
@@ -116,7 +116,7 @@ __global__ __launch_bounds__(THREADS) void k_erode_pair(ErosionMeta *__restrict_
 // Kernel variants (NX_OPT_PAIR_KERNEL): block size and register use.
 struct PairVariant {
     void (*fn)(ErosionMeta *, double2 *, double2 *, double *, double *, TilePlanDev, int, int64_t,
-               double, double, double);
+               double, double);
     int threads;
 };
 static const PairVariant kPairVariants[] = {
@@ -135,8 +135,8 @@ __global__ __launch_bounds__(THREADS) void k_erode_multi(ErosionMeta *__restrict
                                                         double2 *__restrict__ hw1,
                                                         double *__restrict__ s0,
                                                         double *__restrict__ s1, TilePlanDev P, int j,
-                                                       int64_t done, double rain_first,
-                                                       double rain_mid, double rain_next)
+                                                       int64_t done, double rain_mid,
+                                                       double rain_next)
 {
     __shared__ double2 A[kLoadMaxMulti];
     const int p = launch_buffer(meta, j, done);
@@ -156,8 +156,8 @@ __global__ __launch_bounds__(1024) void k_erode_quad(ErosionMeta *__restrict__ m
                                                     double2 *__restrict__ hw1,
                                                     double *__restrict__ s0,
                                                     double *__restrict__ s1, TilePlanDev P, int j,
-                                                       int64_t done, double rain_first,
-                                                       double rain_mid, double rain_next)
+                                                       int64_t done, double rain_mid,
+                                                       double rain_next)
 {
     __shared__ double2 A[kQuadLds];
     double2 *const B = A + kQuadLoadMax;
@@ -165,8 +165,7 @@ __global__ __launch_bounds__(1024) void k_erode_quad(ErosionMeta *__restrict__ m
     if (tile >= P.ntiles) return;
     const QuadTile q = quad_tile(P, tile);
     const int p = launch_buffer(meta, j, done);
-    erode_tile_quad<RULE, NS, FIRST>(A, B, hw0, hw1, s0, s1, p, P, q, rain_mid,
-                              rain_next, rain_first);
+    erode_tile_quad<RULE, NS, FIRST>(A, B, hw0, hw1, s0, s1, p, P, q, rain_mid, rain_next);
 }
 
 // NX_OPT_MULTI_KERNEL variants: 0 keeps each thread's first-step data in
@@ -184,7 +183,7 @@ static const PairVariant kQuadTails[2][2] = {   // [rule 4][steps 3]
     {{k_erode_quad<3, 2>, 1024}, {k_erode_quad<3, 3>, 1024}},
     {{k_erode_quad<4, 2>, 1024}, {k_erode_quad<4, 3>, 1024}},
 };
-// The first launch of a run with rain, by its steps 2..4.
+// The first launch of a run with rain, by its steps 2..4 (rain_mid is added first, too).
 static const PairVariant kQuadFirst[2][3] = {
     {{k_erode_quad<3, 2, true>, 1024}, {k_erode_quad<3, 3, true>, 1024}, {k_erode_quad<3, 4, true>, 1024}},
     {{k_erode_quad<4, 2, true>, 1024}, {k_erode_quad<4, 3, true>, 1024}, {k_erode_quad<4, 4, true>, 1024}},
@@ -381,7 +380,7 @@ static void launch_steps(const ErosionBufs &b, int64_t V, const int32_t *col, co
                                    : per == 2    ? (rule == 4 ? kPairRule4 : kPairVariants[variant])
                                                  : (rule == 4 ? kMultiRule4 : kMultiVariants[mvariant]);
             hipLaunchKernelGGL(v.fn, dim3(tgrid), dim3(v.threads), 0, stream, b.meta, b.hw[0],
-                               b.hw[1], b.s[0], b.s[1], P, j, done, rain, rain, rain_next);
+                               b.hw[1], b.s[0], b.s[1], P, j, done, rain, rain_next);
         }
         k += steps;
     }

@@ -392,14 +392,13 @@ __device__ __forceinline__ QuadTile quad_tile(const TilePlanDev &P, int64_t tile
 // theirs.  NS = 3 or 2 runs the last three or two of those steps (a run's
 // tail of steps that does not fill a four-step launch): the first step then
 // covers tile + rings 1..2 or tile + ring 1, and only the vertices it reads
-// are staged.  FIRST adds rain_first to the water as it is staged (the first
+// are staged.  FIRST adds rain_mid to the water as it is staged (the first
 // rain of a run, erosion.py:182).
 template <int RULE = 3, int NS = 4, bool FIRST = false>
 __device__ __forceinline__ void erode_tile_quad(double2 *A, double2 *B, double2 *hw0, double2 *hw1,
                                                 double *s0, double *s1, int p,
                                                 const TilePlanDev &P, const QuadTile &Q,
-                                                double rain_mid, double rain_next,
-                                                double rain_first = 0.0)
+                                                double rain_mid, double rain_next)
 {
     constexpr int TH = 1024;
     constexpr int kPer = kQuadStepOne / TH;
@@ -494,7 +493,7 @@ __device__ __forceinline__ void erode_tile_quad(double2 *A, double2 *B, double2 
 #pragma unroll
     for (int m = 0; m < kLoadPer; ++m) {
         const int li = threadIdx.x + m * TH;
-        if (FIRST) w[m] = w[m] + rain_first;
+        if (FIRST) w[m] = w[m] + rain_mid;
         if (li < cl) A[li] = make_double2(h[m], w[m]);
     }
     __syncthreads();
