@@ -13,10 +13,10 @@
 // cos(latitude) * cos(longitude) of a rotated vertex t is, without the
 // angles, sqrt(1 - (t.z / r)^2) * t.x / sqrt(t.x^2 + t.y^2); on the sphere of
 // radius r the two roots cancel and it is t.x / |r|, the sun's direction
-// component.  k_insolation and k_slices use the second form for vertices on
-// the sphere to within rounding, the first elsewhere, and the angles
-// themselves (insol_value) only where the first form's quotients could
-// overflow or a value is not finite.  The kernels are bound by FP64 issue:
+// component.  k_insolation, k_slice and k_year_slice use the second form for
+// vertices on the sphere to within rounding, the first (insol_vector) elsewhere
+// and at angles that are not finite, and the angles themselves (insol_value)
+// only where the first form's quotients could overflow or a value is not finite.  The kernels are bound by FP64 issue:
 // six FP64 instructions per vertex and step on the sphere.
 #include <hip/hip_runtime.h>
 

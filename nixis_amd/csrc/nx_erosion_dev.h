@@ -89,7 +89,8 @@ NX_EHD double turn_sign(double x, double diff)
 
 // erode_accumulate for |h| >= kCompare: the products take the difference's
 // sign (S - t is S + -t, and -w k is -(w k)), so one comparison and two sums
-// serve both directions.
+// serve both directions.  A sum that is not a number may carry the other sign
+// (fields that have overflowed); every other value is the same bit for bit.
 template <int RULE = 3>
 NX_EHD void erode_compare(double h, double hn, double wn, double d, double &S, double &W)
 {

@@ -1027,7 +1027,8 @@ __global__ __launch_bounds__(256) void k_knn_points(GridView v, int64_t V,
 // ROWS: a block's pixels lie in one row, and stripes of 1 << stripe rows go to
 // the XCDs in turn (blockIdx.x is the XCD: consecutive blocks go round them),
 // so that an XCD's L2 reads the points of its stripes once: 8192 x 4096 on
-// d=1000 STRIPES.  Otherwise blocks take 256 pixels across rows.
+// d=1000 947 us in stripes of 16, 982 row by row.  Otherwise blocks take 256
+// pixels across rows.
 template <int K, bool ROWS>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(K <= 3 ? 7 : 4))) void
 k_knn_pixels(GridView v, int64_t V, int64_t width, int64_t height, double radius, int stripe,

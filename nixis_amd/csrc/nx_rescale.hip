@@ -1567,15 +1567,16 @@ int terrain_heights(nx_ctx *ctx, const double *verts, int64_t V, const int32_t *
 
 // ---- terrain_heights without a caller workspace ---------------------------
 //
-// The chain's workspace (the 256-byte head and at most kPrMaxBlocks pairs of
-// block summaries) as a file-scope device array: one copy per GPU, held
+// The chain's workspace (the 256-byte head, then at most kChainBlocks pairs of
+// block summaries or the heights of a small chain, and the records of the
+// min/max) as a file-scope device array: one copy per GPU, held
 // until the process ends.  Its device address is taken once per context,
 // with the context's device current (chain_scratch_init, called when the
 // context is created), and passed to the kernels exactly as terrain_heights
-// passes a caller's workspace.  Every reduction key in the head is reset by a
-// fill kernel at the start of its pass and every summary is written before
-// it is read, so nothing carries over from the previous call; calls that
-// overlap on one GPU share the array and race.
+// passes a caller's workspace.  The summary pass joins the min/max from this
+// call's records and resets the keys of the later passes, and every summary,
+// record and height is written before it is read, so nothing carries over from
+// the previous call; calls that overlap on one GPU share the array and race.
 constexpr size_t kChainScratchBytes = 256 + ((sizeof(PSum) * 2 * (size_t)kPrMaxBlocks + 255) & ~(size_t)255);
 static_assert(kChainScratchBytes == 196864, "include/nixis.h states the scratch size");
 static __device__ __align__(256) unsigned char scratch[kChainScratchBytes];

@@ -138,22 +138,26 @@ class ErosionGraph:
             ctx.handle, _lib.ptr(neighbors.contiguous()), V, _lib.ptr(verts.contiguous()),
             _lib.ptr(order), _lib.ptr(col), _lib.ptr(elen), _lib.ptr(ws),
             _lib.stream_ptr(stream)))
-        ctx.sync_check(stream)
         self.col, self.elen = col, elen
         self._odev = order
-        self.order = order.cpu().numpy() if order is not None else None
         self.plan = None
         self._stream_bytes = None
         self._plan_blob = None
         self.steps = int(steps)
         self._tuning(chunk, variant, graph_chunk)
-        if tiled and not (self.steps == 4 and self._build_plan_device(stream)):
+        # tables and plan are complete on return: a run may be on any stream
+        planned = tiled and self.steps == 4 and self._build_plan_device(stream)
+        if not planned:
+            ctx.sync_check(stream)
+        self.order = order.cpu().numpy() if order is not None else None
+        if tiled and not planned:
             self._build_plan(col.cpu().numpy(), elen.cpu().numpy())
         return self
 
     def _build_plan_device(self, stream):
-        """The four-step plan from the device tables, written before this
-        returns; False when refused, or without memory for its workspace."""
+        """The four-step plan from the device tables, written and the stream
+        checked before this returns; False when refused, or without memory for
+        its workspace."""
         import torch
         L = _lib.lib()
         plan = _lib.NxTilePlan()
@@ -172,10 +176,11 @@ class ErosionGraph:
             rc = build(None, 0)
             if rc == _lib.NX_ERANGE:
                 return False
+            if rc != _lib.NX_OK:
+                ctx.sync_check(stream)      # an error of the tables comes first
             _lib.check(rc)
             blob = torch.zeros(plan.bytes, dtype=torch.uint8, device=self.device)
             _lib.check(build(blob, plan.bytes))
-        # complete on return, as the tables are: a run may be on any stream
         ctx.sync_check(stream)
         self._set_plan(plan, blob)
         return True
