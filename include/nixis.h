@@ -249,9 +249,9 @@ int nx_make_gray_array(nx_ctx *ctx, int64_t npix, int k, const double *dists,
  * numba adds a double to a float32 element (double sum, rounded to float).
  * The rotation, tilt and seasonal sines and cosines come from the host C
  * library; the reference's per-vertex asin, atan2 and cosines are taken as
- * products of the rotated vector's components (FP64) where its length is the
- * radius, so values agree with the reference's to a few float32 ulp per
- * summed step.  A year is the sum of the days' tables in FP64, interpolated
+ * products of the rotated vector's components (FP64), or computed where those
+ * could overflow or a value is not finite, so values agree with the
+ * reference's to a few float32 ulp per summed step.  A year is the sum of the days' tables in FP64, interpolated
  * once per vertex.
  * ws: nx_climate_workspace_bytes() of 256-byte aligned device memory. */
 size_t nx_climate_workspace_bytes(void);

@@ -258,7 +258,8 @@ class Context:
         check(lib().nx_ctx_sync_check(self.handle, stream_ptr(stream)))
 
     def set_graph_chunk(self, steps):
-        """Erosion steps per captured hipGraph (0: eager launches)."""
+        """Erosion steps per captured hipGraph of a run without a tile plan
+        (0: eager launches)."""
         check(lib().nx_ctx_set_option(self.handle, NX_OPT_GRAPH_CHUNK, int(steps)))
         self.graph_chunk = int(steps)
 

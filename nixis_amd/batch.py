@@ -109,8 +109,9 @@ class MeshCache:
     a planet's fields are per vertex in that order, ``order(d)[k]`` being
     the generator's index of vertex k (``PlanetRun.heights`` maps back).
     With ``on_device`` (default) the icosphere, its neighbour tables, the
-    order and the device neighbour layout are generated on the GPU (the same
-    arrays as the host generator); the tile plan is cut on the host."""
+    order, the device neighbour layout and four-step tile plans are made on the
+    GPU (the same arrays and images as on the host); two-step plans are cut on
+    the host."""
 
     def __init__(self, device=None, on_device=True):
         import torch
